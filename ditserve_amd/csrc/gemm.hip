@@ -382,32 +382,41 @@ __global__ __launch_bounds__(Tile<T>::WM * Tile<T>::WN * 64, Tile<T>::WAVES_PER_
   }
 }
 
-// Large tiles on one wave per SIMD (every epilogue but fp32, K % 64 == 0): the
-// 256 x 256 workgroup tile as four 128 x 128 wave tiles, 256 accumulators per
-// wave in the AGPRs.  The k loop and the bf16 staging are generated assembly
-// (gen_gemm.py -> gemm_l4_body.inc: 64-k stages through two 64 KiB LDS buffers
-// filled by direct DMA, the next chunk's fragments read under the current
-// MFMAs); this C++ part computes the per-lane addresses and runs the
+// One wave per SIMD (every epilogue but fp32, K % 64 == 0): a workgroup tile as
+// four wave tiles, their accumulators in the AGPRs (all 256 of them for the
+// 256 x 256 tile's 128 x 128 wave tiles).  The k loop and the bf16 staging are
+// generated assembly (gen_gemm.py -> gemm_l4_*_body.inc: 64-k stages through
+// NBUF LDS buffers filled by direct DMA, the next chunk's fragments read under
+// the current MFMAs); this C++ part computes the per-lane addresses and runs the
 // same epilogue arithmetic as gemm_kernel on the staged rows.  Same MFMA
 // (16x16x32, W rows as the A operand), same k order, same bias add and rounding:
 // bitwise equal to gemm_kernel.
-// FI feature fragments of 16 per wave tile: 8 (128 x 128 wave tiles, 256 x 256
-// workgroup tiles, gemm_l4_body.inc) or 6 (128 x 96, 256 x 192,
-// gemm_l4w96_body.inc: for shapes whose 256-wide tiles would leave CUs idle in
-// the last round).
-template <int FI>
+// A wave tile is FI feature and FJ token fragments of 16; the six tiles generated
+// are listed with their times at kL4 below.  What bounds them: a 256 x 256 tile's
+// stage is 2048 MFMA cycles for 64 KiB of operand DMA (MFMA-bound); at 128 x 128 it
+// is 512 cycles for 32 KiB, and the CU's ~60 B/clk from L2 takes about as long
+// (1560 x 1536 x 8960 on 64 x 128 tiles of gemm_kernel 81 us, 128 x 96 here 54 us;
+// 2048 x 6144 x 1536 on 256 x 192 as before).
+template <int FI, int FJ>
 struct L4 {
-  static constexpr int WTM = 128, WTN = 16 * FI, GBM = 256, GBN = 2 * WTN;
+  static constexpr int WTM = 16 * FJ, WTN = 16 * FI, GBM = 2 * WTM, GBN = 2 * WTN;
+  static constexpr int NBUF = FJ == 8 ? 2 : FI >= 6 ? 3 : FI == 3 ? 5 : 4;  // stage buffers, as generated
   static constexpr int BUF = (GBM + GBN) * 128;            // one 64-k stage: A rows, then W rows
   static constexpr int STG_ROW = 2 * WTN + 16;             // staging row bytes
-  static constexpr int LDS_BYTES = 2 * BUF > 4 * WTM * STG_ROW ? 2 * BUF : 4 * WTM * STG_ROW;
+  // the stage buffers and the prefetch's spare line, or the staging rows
+  static constexpr int LDS_BYTES = NBUF * BUF + 1024 > 4 * WTM * STG_ROW ? NBUF * BUF + 1024 : 4 * WTM * STG_ROW;
 };
 #define DITK_L4_OPERANDS                                                                                        \
   [a_lo] "s"(su((uint32_t)abase)), [a_hi] "s"(su((uint32_t)(abase >> 32))), [w_lo] "s"(su((uint32_t)wbase)),   \
       [w_hi] "s"(su((uint32_t)(wbase >> 32))), [nk] "s"(su(K / 64)), [lds] "s"(su(lds0)),                       \
-      [wave1k] "s"(su(wave_u * 1024u)), [rdx00] "v"(rdx[0][0]), [rdx01] "v"(rdx[0][1]), [rdx10] "v"(rdx[1][0]), \
-      [rdx11] "v"(rdx[1][1]), [rdw00] "v"(rdw[0][0]), [rdw01] "v"(rdw[0][1]), [rdw10] "v"(rdw[1][0]),           \
-      [rdw11] "v"(rdw[1][1]), [aoff0] "v"(aoff[0]), [aoff1] "v"(aoff[1]), [aoff2] "v"(aoff[2]),                 \
+      [wave1k] "s"(su(wave_u * 1024u)), [pf_lo] "s"(su((uint32_t)(uint64_t)(uintptr_t)W)),                       \
+      [pf_hi] "s"(su((uint32_t)((uint64_t)(uintptr_t)W >> 32))), [pfn] "s"(su(pf.n)), [pfn0] "s"(su(pf.n0)),     \
+      [pflpr] "s"(su(pf.lines)), [pfstep] "s"(su(pf.lines * 128u)), [pfmax] "v"(pf_max), [pfoff] "v"(pf_off), [rdx00] "v"(rdx[0][0]), [rdx01] "v"(rdx[0][1]), [rdx10] "v"(rdx[1][0]), \
+      [rdx11] "v"(rdx[1][1]), [rdx20] "v"(rdx[2][0]), [rdx21] "v"(rdx[2][1]), [rdx30] "v"(rdx[3][0]),           \
+      [rdx31] "v"(rdx[3][1]), [rdx40] "v"(rdx[4][0]), [rdx41] "v"(rdx[4][1]), [rdw00] "v"(rdw[0][0]),           \
+      [rdw01] "v"(rdw[0][1]), [rdw10] "v"(rdw[1][0]), [rdw11] "v"(rdw[1][1]), [rdw20] "v"(rdw[2][0]),           \
+      [rdw21] "v"(rdw[2][1]), [rdw30] "v"(rdw[3][0]), [rdw31] "v"(rdw[3][1]), [rdw40] "v"(rdw[4][0]),           \
+      [rdw41] "v"(rdw[4][1]), [aoff0] "v"(aoff[0]), [aoff1] "v"(aoff[1]), [aoff2] "v"(aoff[2]),                 \
       [aoff3] "v"(aoff[3]), [aoff4] "v"(aoff[4]), [aoff5] "v"(aoff[5]), [aoff6] "v"(aoff[6]),                   \
       [aoff7] "v"(aoff[7]), [woff0] "v"(woff[0]), [woff1] "v"(woff[1]), [woff2] "v"(woff[2]),                   \
       [woff3] "v"(woff[3]), [woff4] "v"(woff[4]), [woff5] "v"(woff[5]), [woff6] "v"(woff[6]),                   \
@@ -418,20 +427,37 @@ struct L4 {
       [b20] "v"(bv[20]), [b21] "v"(bv[21]), [b22] "v"(bv[22]), [b23] "v"(bv[23]), [b24] "v"(bv[24]),            \
       [b25] "v"(bv[25]), [b26] "v"(bv[26]), [b27] "v"(bv[27]), [b28] "v"(bv[28]), [b29] "v"(bv[29]),            \
       [b30] "v"(bv[30]), [b31] "v"(bv[31])
-template <int EPI, int FI>
+// Weight prefetch (see prefetch_start in gen_gemm.py): the launch's `count`
+// workgroups together touch every 128-byte line of W [N, K] once, in k order, a
+// batch of `lines` 64-k stages of all rows at a time and a few stages ahead of
+// their use, so that only the first reader of a line waits for HBM.
+struct L4Prefetch {
+  uint32_t n = 0, n0 = 0, lines = 1;  // batches, batches before the k loop, lines per row and batch
+  int rank = 0;
+};
+__device__ __forceinline__ L4Prefetch l4_prefetch(int rank, int count, int N, int K, bool on) {
+  L4Prefetch p;
+  p.lines = (uint32_t)(count * 256) / (uint32_t)N;
+  if (!on || p.lines == 0) return L4Prefetch{};
+  p.n = ((uint32_t)(K / 64) + p.lines - 1) / p.lines;
+  p.n0 = min(p.n, 1 + (8 + p.lines - 1) / p.lines);
+  p.rank = rank;
+  return p;
+}
+template <int EPI, int FI, int FJ>
 __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __restrict__ A, int64_t lda,
                                         const bf16_t* __restrict__ W, int64_t ldw, const float* __restrict__ bias,
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m);
-template <int EPI, int FI>
+                                        int group_m, L4Prefetch pf);
+template <int EPI, int FI, int FJ>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
     const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
     const float* __restrict__ bias, void* __restrict__ Cv, int64_t ldc, int M, int N, int K,
     const bf16_t* R, int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
-    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m) {
-  __shared__ u32x4_t lds[L4<FI>::LDS_BYTES / 16];
+    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m, bool prefetch) {
+  __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   // Persistent: XCD x (= blockIdx % 8) owns the tiles [x * per_xcd, (x + 1) *
   // per_xcd), which its workgroups take in turn (the order a one-tile-per-
   // workgroup launch would run them in), so each workgroup loads its kernel
@@ -440,9 +466,12 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
   const int nb = gridDim.x, b = blockIdx.x;
   const int ntiles = tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
   const int tlo = (b & 7) * per_xcd, thi = min(tlo + per_xcd, ntiles);
-  for (int L = tlo + (b >> 3); L < thi; L += nb >> 3)
-    l4_tile<EPI, FI>(lds, L, A, lda, W, ldw, bias, Cv, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, tiles_m,
-                     tiles_n, group_m);
+  L4Prefetch pf = l4_prefetch(b, nb, N, K, prefetch);
+  for (int L = tlo + (b >> 3); L < thi; L += nb >> 3) {
+    l4_tile<EPI, FI, FJ>(lds, L, A, lda, W, ldw, bias, Cv, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, tiles_m,
+                     tiles_n, group_m, pf);
+    pf.n = 0;  // once per workgroup
+  }
 }
 
 // One product of a paired launch (see gemm_kernel_l4_pair).
@@ -467,30 +496,38 @@ struct L4Prob {
 // first product's tiles, then the second's, taken per XCD as gemm_kernel_l4
 // takes one product's.  Each tile is computed exactly as a launch of its own
 // product would compute it.
-template <int EPI, int FI>
-__global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob p1, int N, int K, int tiles_n) {
-  __shared__ u32x4_t lds[L4<FI>::LDS_BYTES / 16];
+template <int EPI, int FI, int FJ>
+__global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob p1, int N, int K, int tiles_n,
+                                                           bool prefetch) {
+  __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   const int nb = gridDim.x, b = blockIdx.x;
   const int t0 = p0.tiles_m * tiles_n, ntiles = t0 + p1.tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
   const int tlo = (b & 7) * per_xcd, thi = min(tlo + per_xcd, ntiles);
+  // Workgroups in the order of their first tiles: the first c0 start in product 0
+  // and prefetch its weights, the others product 1's.
+  const int wpx = nb >> 3, x0 = t0 / per_xcd, rank = (b & 7) * wpx + (b >> 3);
+  const int c0 = min(nb, x0 * wpx + min(t0 - x0 * per_xcd, wpx));
+  L4Prefetch pf = rank < c0 ? l4_prefetch(rank, c0, N, K, prefetch)
+                            : l4_prefetch(rank - c0, nb - c0, N, K, prefetch);
   for (int L = tlo + (b >> 3); L < thi; L += nb >> 3) {
     const bool s = L >= t0;  // wave-uniform: the fields below are scalar selects
-    l4_tile<EPI, FI>(lds, s ? L - t0 : L, s ? p1.A : p0.A, s ? p1.lda : p0.lda, s ? p1.W : p0.W,
+    l4_tile<EPI, FI, FJ>(lds, s ? L - t0 : L, s ? p1.A : p0.A, s ? p1.lda : p0.lda, s ? p1.W : p0.W,
                      s ? p1.ldw : p0.ldw, s ? p1.bias : p0.bias, s ? p1.C : p0.C, s ? p1.ldc : p0.ldc,
                      s ? p1.M : p0.M, N, K, s ? p1.R : p0.R, s ? p1.ldr : p0.ldr, s ? p1.gate : p0.gate,
                      s ? p1.gate_stride : p0.gate_stride, s ? p1.cu : p0.cu, s ? p1.nseg : p0.nseg,
-                     s ? p1.tiles_m : p0.tiles_m, tiles_n, s ? p1.group_m : p0.group_m);
+                     s ? p1.tiles_m : p0.tiles_m, tiles_n, s ? p1.group_m : p0.group_m, pf);
+    pf.n = 0;
   }
 }
 
-template <int EPI, int FI>
+template <int EPI, int FI, int FJ>
 __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __restrict__ A, int64_t lda,
                                         const bf16_t* __restrict__ W, int64_t ldw, const float* __restrict__ bias,
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m) {
-  using G = L4<FI>;
+                                        int group_m, L4Prefetch pf) {
+  using G = L4<FI, FJ>;
   constexpr int GBM = G::GBM, GBN = G::GBN, WTM = G::WTM, WTN = G::WTN, STG_ROW = G::STG_ROW;
   const int group = L / (group_m * tiles_n);
   const int first_m = group * group_m;
@@ -511,9 +548,9 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   // fragment reads of 32-k chunk c: row ql of a 16-row fragment, 16-byte unit
   // 4 c + g of its 64 k, stored at unit (4 c + g) ^ ((row >> 1) & 7) of the
   // 128-byte LDS row (as gemm_kernel's 64-k stages)
-  uint32_t rdx[2][2], rdw[2][2];
+  uint32_t rdx[5][2] = {}, rdw[5][2] = {};
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
+  for (int s = 0; s < G::NBUF; ++s)
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const uint32_t lane_part = (uint32_t)(ql * 128 + (((c * 4 + g) ^ ((ql >> 1) & 7)) * 16));
@@ -527,9 +564,14 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   for (int d = 0; d < 8; ++d) {
     const int row = (d * 4 + wave_u) * 8 + lane / 8;
     const int usw = ((lane & 7) ^ ((row >> 1) & 7)) * 16;
-    aoff[d] = (uint32_t)((int64_t)min(row, M - 1 - m0) * lda * 2 + usw);
+    aoff[d] = d < FJ ? (uint32_t)((int64_t)min(row, M - 1 - m0) * lda * 2 + usw) : 0u;
     woff[d] = d < FI ? (uint32_t)((int64_t)min(row, N - 1 - n0) * ldw * 2 + usw) : 0u;
   }
+  // this lane's prefetch row (of lane 256 rank + tid over `lines` lanes a row) and
+  // the first and last of its lines, as byte offsets into W
+  const uint32_t pf_lane = (uint32_t)(pf.rank * 256 + tid), pf_row = min(pf_lane / pf.lines, (uint32_t)(N - 1));
+  const uint32_t pf_base = pf_row * (uint32_t)(ldw * 2), pf_off = pf_base + (pf_lane % pf.lines) * 128u;
+  const uint32_t pf_max = pf_base + (uint32_t)(K / 64 - 1) * 128u;
   const uint32_t stg = lds0 + wave_u * (WTM * STG_ROW) + ql * STG_ROW + g * 8;
   float bv[32];
 #pragma unroll
@@ -543,13 +585,30 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   auto su = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
   const uint64_t abase = (uint64_t)(uintptr_t)(A + (int64_t)m0 * lda);
   const uint64_t wbase = (uint64_t)(uintptr_t)(W + (int64_t)n0 * ldw);
-  if constexpr (FI == 8)
+  static_assert(FI == 8 || FI == 6 || (FJ == 4 && (FI == 4 || FI == 3)), "a generated wave tile");
+  if constexpr (FI == 8 && FJ == 8)
     asm volatile(
-#include "gemm_l4_body.inc"
+#include "gemm_l4_256x256_body.inc"
         : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
-  else
+  else if constexpr (FI == 6 && FJ == 8)
     asm volatile(
-#include "gemm_l4w96_body.inc"
+#include "gemm_l4_256x192_body.inc"
+        : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
+  else if constexpr (FI == 8 && FJ == 4)
+    asm volatile(
+#include "gemm_l4_128x256_body.inc"
+        : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
+  else if constexpr (FI == 6 && FJ == 4)
+    asm volatile(
+#include "gemm_l4_128x192_body.inc"
+        : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
+  else if constexpr (FI == 4 && FJ == 4)
+    asm volatile(
+#include "gemm_l4_128x128_body.inc"
+        : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
+  else if constexpr (FI == 3 && FJ == 4)
+    asm volatile(
+#include "gemm_l4_128x96_body.inc"
         : : DITK_L4_OPERANDS : DITK_GEMM_L4_CLOBBERS "scc", "memory");
 
   // epilogue on this wave's staged rows (the wave wrote them and waited for them).
@@ -666,86 +725,76 @@ int cu_count() {
   }
   return c;
 }
-template <int EPI, int FI>
+// The tile configurations of gemm_kernel_l4: workgroup tile (tokens x features)
+// and its measured time in us, start + rounds x (tile + stage x K / 64) with a round
+// one tile per CU (least squares over 14 weight shapes of the Wan and SD3.5 blocks,
+// 8 to 28000 rows, weights from HBM; 8-9% rms).  A 256 x 256 tile's stage does 2.3
+// PFLOP/s over the chip, a 128 x 96 one's 1.4: the small tiles move more operand
+// bytes per MFMA, but let 1000-row products use most of the CUs.
+struct L4Cfg {
+  int gbm, gbn;
+  float start, tile, stage;
+};
+constexpr int kL4Cfgs = 6;
+constexpr L4Cfg kL4[kL4Cfgs] = {{256, 256, -4.4f, 10.2f, 1.207f}, {256, 192, -2.3f, 6.6f, 1.054f},
+                                {128, 256, -0.1f, 5.1f, 0.744f},  {128, 192, 0.6f, 3.7f, 0.592f},
+                                {128, 128, 1.2f, 2.6f, 0.439f},   {128, 96, 1.7f, 2.5f, 0.381f}};
+
+// Tile order of gemm_kernel_l4.  Up to two rounds of tiles, all of an XCD's tiles
+// run about together, so its block of them is made about square in operand rows:
+// it then pulls the fewest operand bytes into its L2 (2048 x 1536 x 8960: 63.5 us
+// in the long-K order below, 61 us in groups of 4-6 m-tiles).  More rounds:
+// gemm_group_m's orders.
+int l4_group_m(int64_t tiles_m, int64_t tiles_n, int gbm, int gbn, int K) {
+  const int64_t tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
+  if (tiles > 2 * cu_count()) return gemm_group_m(K, (int)tiles_n);
+  int64_t g = 1;
+  while (g < tiles_m && (g + 1) * (g + 1) * gbm <= per_xcd * gbn) ++g;
+  const int64_t groups = (tiles_m + g - 1) / g;
+  return (int)((tiles_m + groups - 1) / groups);
+}
+
+// Whether a launch prefetches its weights (see L4Prefetch).  Where every tile row
+// is full, the workgroups run in step and all wait for HBM at the first touch of
+// each weight line: 2048 x 1536 x 8960 at 128 x 128 tiles 78 -> 61 us, x 6144
+// 55 -> 42 us, 6400 x 1536 x 8960 at 256 x 192 160 -> 142 us, 4608 x 1536 33.0 ->
+// 29.7 us.  A short last tile row (its missing rows re-read one row) runs ahead and
+// does the same for nothing: with up to a third of a tile left the prefetch costs
+// 0-3%, beyond that it wins by as much as with full tiles, but with 256-row tiles
+// only at long K.  Few tile rows share too little: at 512 rows 11.7 -> 12.1 us
+// (1536 x 1536) but 69 -> 55 us (1536 x 8960), at 100 rows (one) 55 -> 80 us.
+bool l4_prefetch_on(int M, int N, int K, int64_t ldw, int gbm) {
+  const int rem = M % gbm, tiles_m = (M + gbm - 1) / gbm;
+  if (tiles_m < (K >= 4096 ? 4 : 8)) return false;
+  return (int64_t)N * ldw * 2 < (1ll << 31) && (rem == 0 || (3 * rem > gbm && (gbm == 128 || K >= 4096)));
+}
+template <int EPI, int FI, int FJ>
 int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
               int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
               const int32_t* cu, int nseg, hipStream_t stream) {
-  constexpr int GBN = L4<FI>::GBN;
-  const int tiles_m = (M + 255) / 256, tiles_n = (N + GBN - 1) / GBN;
+  constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
+  const int tiles_m = (M + GBM - 1) / GBM, tiles_n = (N + GBN - 1) / GBN;
   // one persistent workgroup per CU (a multiple of 8: the same number per XCD)
   const int64_t nblocks = std::min<int64_t>(((int64_t)tiles_m * tiles_n + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
-  gemm_kernel_l4<EPI, FI><<<(unsigned)nblocks, 256, 0, stream>>>(
+  gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
-      gate_stride, cu, nseg, tiles_m, tiles_n, gemm_group_m(K, tiles_n));
+      gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM));
   return ditk_check_launch("ditk_gemm");
 }
 
-template <int EPI>
+template <int EPI, int FI, int FJ>
 int launch_l4_pair(L4Prob p0, L4Prob p1, int N, int K, hipStream_t stream) {
-  const int tiles_n = (N + 255) / 256;
-  p0.tiles_m = (p0.M + 255) / 256;
-  p1.tiles_m = (p1.M + 255) / 256;
-  p0.group_m = p1.group_m = gemm_group_m(K, tiles_n);
+  constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
+  const int tiles_n = (N + GBN - 1) / GBN;
+  p0.tiles_m = (p0.M + GBM - 1) / GBM;
+  p1.tiles_m = (p1.M + GBM - 1) / GBM;
+  p0.group_m = l4_group_m(p0.tiles_m, tiles_n, GBM, GBN, K);
+  p1.group_m = l4_group_m(p1.tiles_m, tiles_n, GBM, GBN, K);
   const int64_t tiles = (int64_t)(p0.tiles_m + p1.tiles_m) * tiles_n;
   const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
-  gemm_kernel_l4_pair<EPI, 8><<<(unsigned)nblocks, 256, 0, stream>>>(p0, p1, N, K, tiles_n);
+  gemm_kernel_l4_pair<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
+      p0, p1, N, K, tiles_n, l4_prefetch_on(p0.M, N, K, p0.ldw, GBM) && (int64_t)N * p1.ldw * 2 < (1ll << 31));
   return ditk_check_launch("ditk_gemm_pair");
-}
-
-// The one-wave-per-SIMD kernel where it measured faster than gemm_kernel's large
-// tiles (same box, Wan2.1 block shapes at M = 65520): N >= 3072 or K >= 4096
-// (qkv -3.4%, ffn-up -2.9%, ffn-down -4.7%, N = 3072 SiLU -3.3%), and, since its
-// workgroups are persistent, at N = K = 1536 too except with the gated residual
-// (bias -4%, residual -4%; gated residual +3%, also with the gate looked up
-// before the k loop).  The choice changes no result.
-bool use_l4(int N, int K, int epi) {
-  return K % 64 == 0 && (N >= 3072 || K >= 4096 || epi != EPI_GATE_RES);
-}
-
-// 256 x 192 tiles when they fill the GPU's CUs in fewer tile-rounds than
-// 256 x 256 ones, a 192-wide tile taking 0.85 of a 256-wide one's time (measured
-// 0.82-0.88 at M = 54560, K = 3072-14336: its k loop moves the same token rows
-// for 3/4 of the MFMAs): e.g. M = 8192 and N = 1536 is 256 tiles = one round
-// instead of 192 = one round with a quarter of the CUs idle (SD3.5: ffn-down
-// -12%); N = 4608 is 768 tiles = 3 rounds instead of 576 = 2.25, so 3 (SD3.5
-// qkv -16%); but M = 54560 and N = 3072 is 3424 tiles = 14 rounds instead of
-// 2568 = 11 (Wan2.2-5B: ffn-down -11%, qkv -8%, o-proj -6% with 256-wide tiles).
-bool use_w192(int M, int N) {
-  const int64_t tm = (M + 255) / 256, ncu = cu_count();
-  const int64_t r256 = (tm * ((N + 255) / 256) + ncu - 1) / ncu, r192 = (tm * ((N + 191) / 192) + ncu - 1) / ncu;
-  return r192 * 85 < r256 * 100;
-}
-
-// The rows of a short last 256-row tile, when leaving them to the small-tile
-// kernel (a second launch right after) saves the persistent kernel a round of
-// tiles: a 256-row tile costs the same however few of its rows are real, while
-// the small tiles (64 x 128) of the leftover rows take a fraction of a round.
-// E.g. M = 54560 = 213 * 256 + 32 and N = 3072: 2568 tiles = 11 rounds of 256
-// CUs, of which the last holds 8 tiles; 2556 tiles = 10 rounds plus the 32 rows
-// (Wan2.2-5B ffn-down 3.89 -> 3.56 ms, N = K = 3072 -8%, qkv -3%).  Every row is
-// computed the same way by either kernel, so the split changes no result.
-int l4_tail_rows(int M, int N, int gbn) {
-  const int64_t tm = (M + 255) / 256, rem = M % 256;
-  if (rem == 0 || tm < 2) return 0;
-  const int64_t tn = (N + gbn - 1) / gbn, ncu = std::max(8, cu_count() / 8 * 8);
-  const int64_t r_all = (tm * tn + ncu - 1) / ncu, r_main = ((tm - 1) * tn + ncu - 1) / ncu;
-  return r_main < r_all ? (int)rem : 0;
-}
-
-// A paired launch (256 x 256 tiles) when its rounds of tiles cost no more than
-// the larger product alone (its own tile width) plus 0.4 of a round for the
-// smaller one's separate launch (measured: 666 rows at N = 1536, K = 1536 and
-// 6144 take 30-50 us beside 52-134 us rounds).  SD3.5's gated-residual
-// projections, 8192 image + 666 text rows at N = 1536: 192 + 18 tiles are one
-// round, against one 192-wide round plus a text launch.  qkv (N = 4608) and the
-// feed-forward input (N = 6144) do not pair: the text tiles would add a round.
-bool pair_pays(int M0, int M1, int N) {
-  const int64_t ncu = std::max(8, cu_count() / 8 * 8), tn = (N + 255) / 256;
-  const int64_t big = std::max(M0, M1), t_all = ((int64_t)(M0 + 255) / 256 + (M1 + 255) / 256) * tn;
-  const int64_t tb = (big + 255) / 256;
-  const int64_t r_pair = (t_all + ncu - 1) / ncu, r256 = (tb * tn + ncu - 1) / ncu,
-                r192 = (tb * ((N + 191) / 192) + ncu - 1) / ncu;
-  return r_pair * 100 <= std::min(r256 * 100, r192 * 85) + 40;
 }
 
 template <int EPI, int BK, int T>
@@ -763,38 +812,103 @@ int launch_tile(const void* A, int64_t lda, const void* W, int64_t ldw, const fl
   return ditk_check_launch("ditk_gemm");
 }
 
-// Small tiles when the large ones would number fewer than kSmallBelow: the
-// choice cannot change a result, only how many CUs take part.  Measured per CU,
-// a small workgroup alone on a CU runs at about half a large one's rate and two
-// sharing one at about a quarter each, so small tiles (8 per large tile) win
-// while they fit about two per CU: 666-row text GEMMs 1.3-3x faster (54-72
-// large tiles), 8192 x 1536 1.25-1.5x slower (192 large tiles).
+// One product on the one-wave-per-SIMD kernel's tile configuration `cfg`.
+template <int EPI>
+int launch_l4_cfg(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
+                  int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
+                  int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
+  switch (cfg) {
+    case 0: return launch_l4<EPI, 8, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    case 1: return launch_l4<EPI, 6, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    case 2: return launch_l4<EPI, 8, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    case 3: return launch_l4<EPI, 6, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    case 4: return launch_l4<EPI, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    default: return launch_l4<EPI, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+  }
+}
+
+template <int EPI>
+int launch_l4_pair_cfg(int cfg, const L4Prob& p0, const L4Prob& p1, int N, int K, hipStream_t stream) {
+  switch (cfg) {
+    case 0: return launch_l4_pair<EPI, 8, 8>(p0, p1, N, K, stream);
+    case 1: return launch_l4_pair<EPI, 6, 8>(p0, p1, N, K, stream);
+    case 2: return launch_l4_pair<EPI, 8, 4>(p0, p1, N, K, stream);
+    case 3: return launch_l4_pair<EPI, 6, 4>(p0, p1, N, K, stream);
+    case 4: return launch_l4_pair<EPI, 4, 4>(p0, p1, N, K, stream);
+    default: return launch_l4_pair<EPI, 3, 4>(p0, p1, N, K, stream);
+  }
+}
+
+// Estimated time (us) of `tiles` tiles of configuration c, and of M x N on the 64 x 128
+// tiles of gemm_kernel while each has a CU to itself (two sharing one run at half
+// the rate each, where the configurations above are the faster ones).
+float l4_cost(int c, int64_t tiles, int K) {
+  const int64_t ncu = std::max(8, cu_count() / 8 * 8), rounds = (tiles + ncu - 1) / ncu;
+  return kL4[c].start + (float)rounds * (kL4[c].tile + kL4[c].stage * (float)(K / 64));
+}
+float small_cost(int M, int N, int K) {
+  const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
+  return tiles <= cu_count() ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
+}
+
+// How one product runs: configuration cfg of gemm_kernel_l4 (-1: gemm_kernel's
+// 64 x 128 tiles) for the first M - tail rows, 64 x 128 tiles for the tail.  The
+// tail is a short last tile row, left to a second launch when that saves the
+// persistent kernel more (a round of tiles) than it costs.  Every row is computed
+// the same way whichever tile holds it, so the choice changes no result.  Against
+// the fastest of all configurations at each measured size the choice loses 0.4% on
+// average.
+struct GemmPlan {
+  int cfg, tail;
+  float us;
+};
+GemmPlan gemm_plan(int M, int N, int K) {
+  GemmPlan best{-1, 0, small_cost(M, N, K)};
+  for (int c = 0; c < kL4Cfgs; ++c) {
+    const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn;
+    const int tm = (M + kL4[c].gbm - 1) / kL4[c].gbm, rem = M % kL4[c].gbm;
+    const float us = l4_cost(c, tm * tn, K);
+    if (us < best.us) best = GemmPlan{c, 0, us};
+    if (rem == 0 || tm < 2) continue;
+    const float split = l4_cost(c, (tm - 1) * tn, K) + small_cost(rem, N, K);
+    if (split < best.us) best = GemmPlan{c, rem, split};
+  }
+  return best;
+}
+
+// fp32 outputs and K % 64 != 0: gemm_kernel, on small tiles when the large ones
+// would number fewer than kSmallBelow (666 rows 1.3-3x faster at 54-72 large tiles,
+// 8192 x 1536 1.25-1.5x slower at 192).
 constexpr int64_t kSmallBelow = 128;
 template <int EPI, int BK>
 int launch(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
            int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
            int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
-  using L = Tile<TILE_LARGE>;
-  const int64_t large_tiles = (int64_t)((M + L::GBM - 1) / L::GBM) * ((N + L::GBN - 1) / L::GBN);
+  // the one-wave-per-SIMD kernel's epilogue addresses a wave tile's rows by 32-bit offsets
+  if constexpr (EPI != EPI_F32 && BK == 64) {
+    if (ldc < (1 << 22) && ldr < (1 << 22)) {
+      const GemmPlan p = gemm_plan(M, N, K);
+      // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
+      // more of the residual and gate reads (28000 x 1536 x 1536 129 -> 123 us, 9300
+      // 46.9 -> 44.6; at N = K = 3072 it is 0-3% slower)
+      if (EPI == EPI_GATE_RES && p.cfg == 0 && K < 3072)
+        return launch_tile<EPI, BK, TILE_LARGE>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+      const int Mm = p.cfg < 0 ? 0 : M - p.tail;
+      if (p.cfg >= 0)
+        if (int rc = launch_l4_cfg<EPI>(p.cfg, A, lda, W, ldw, bias, C, ldc, Mm, N, K, R, ldr, gate, gate_stride, cu,
+                                        nseg, stream))
+          return rc;
+      if (Mm == M) return 0;
+      return launch_tile<EPI, BK, TILE_SMALL>(static_cast<const bf16_t*>(A) + (int64_t)Mm * lda, lda, W, ldw, bias,
+                                              static_cast<bf16_t*>(C) + (int64_t)Mm * ldc, ldc, M - Mm, N, K,
+                                              R ? static_cast<const bf16_t*>(R) + (int64_t)Mm * ldr : nullptr, ldr,
+                                              gate, gate_stride, cu, nseg, stream, Mm);
+    }
+  }
+  const int64_t large_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
   if (large_tiles < kSmallBelow)
     return launch_tile<EPI, BK, TILE_SMALL>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-  // the large-tile kernel's epilogue addresses a wave tile's rows by 32-bit offsets
-  const bool l4_strides = ldc < (1 << 22) && ldr < (1 << 22);
-  const int fi = EPI == EPI_F32 || !l4_strides ? 0
-                 : K % 64 == 0 && use_w192(M, N) ? 6
-                 : use_l4(N, K, EPI)             ? 8
-                                                 : 0;
-  if (fi == 0)
-    return launch_tile<EPI, BK, TILE_LARGE>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-  const int tail = l4_tail_rows(M, N, fi * 32);
-  const int Mm = M - tail;
-  const int rc = fi == 6 ? launch_l4<EPI, 6>(A, lda, W, ldw, bias, C, ldc, Mm, N, K, R, ldr, gate, gate_stride, cu, nseg, stream)
-                         : launch_l4<EPI, 8>(A, lda, W, ldw, bias, C, ldc, Mm, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-  if (rc != 0 || tail == 0) return rc;
-  return launch_tile<EPI, BK, TILE_SMALL>(static_cast<const bf16_t*>(A) + (int64_t)Mm * lda, lda, W, ldw, bias,
-                                          static_cast<bf16_t*>(C) + (int64_t)Mm * ldc, ldc, tail, N, K,
-                                          R ? static_cast<const bf16_t*>(R) + (int64_t)Mm * ldr : nullptr, ldr, gate,
-                                          gate_stride, cu, nseg, stream, Mm);
+  return launch_tile<EPI, BK, TILE_LARGE>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
 }
 
 template <int EPI>
@@ -876,19 +990,32 @@ DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int
   if (int rc = gemm_validate(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N, K, epilogue, R1, ldr1, gate1,
                              gate_stride1, cu_seqlens1, nseg1))
     return rc;
-  // the large-tile kernel addresses a wave tile's output and residual rows by 32-bit offsets
+  // the one-wave-per-SIMD kernel addresses a wave tile's output and residual rows by 32-bit offsets
   const bool strides = ldc0 < (1 << 22) && ldr0 < (1 << 22) && ldc1 < (1 << 22) && ldr1 < (1 << 22);
-  if (M0 > 0 && M1 > 0 && epilogue != EPI_F32 && K % 64 == 0 && strides && pair_pays(M0, M1, N)) {
-    const L4Prob p0{(const bf16_t*)A0, lda0, (const bf16_t*)W0, ldw0, bias0, C0, ldc0, (const bf16_t*)R0, ldr0,
-                    gate0, gate_stride0, cu_seqlens0, nseg0, M0, 0, 0};
-    const L4Prob p1{(const bf16_t*)A1, lda1, (const bf16_t*)W1, ldw1, bias1, C1, ldc1, (const bf16_t*)R1, ldr1,
-                    gate1, gate_stride1, cu_seqlens1, nseg1, M1, 0, 0};
-    switch (epilogue) {
-      case EPI_BIAS: return launch_l4_pair<EPI_BIAS>(p0, p1, N, K, stream);
-      case EPI_GELU: return launch_l4_pair<EPI_GELU>(p0, p1, N, K, stream);
-      case EPI_GATE_RES: return launch_l4_pair<EPI_GATE_RES>(p0, p1, N, K, stream);
-      case EPI_RES: return launch_l4_pair<EPI_RES>(p0, p1, N, K, stream);
-      default: return launch_l4_pair<EPI_SILU>(p0, p1, N, K, stream);
+  if (M0 > 0 && M1 > 0 && epilogue != EPI_F32 && K % 64 == 0 && strides) {
+    // one launch over both tile lists where its rounds cost less than two launches
+    int cfg = -1;
+    float us = gemm_plan(M0, N, K).us + gemm_plan(M1, N, K).us;
+    for (int c = 0; c < kL4Cfgs; ++c) {
+      const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn;
+      const float t = l4_cost(c, ((M0 + kL4[c].gbm - 1) / kL4[c].gbm + (M1 + kL4[c].gbm - 1) / kL4[c].gbm) * tn, K);
+      if (t < us) {
+        us = t;
+        cfg = c;
+      }
+    }
+    if (cfg >= 0) {
+      const L4Prob p0{(const bf16_t*)A0, lda0, (const bf16_t*)W0, ldw0, bias0, C0, ldc0, (const bf16_t*)R0, ldr0,
+                      gate0, gate_stride0, cu_seqlens0, nseg0, M0, 0, 0};
+      const L4Prob p1{(const bf16_t*)A1, lda1, (const bf16_t*)W1, ldw1, bias1, C1, ldc1, (const bf16_t*)R1, ldr1,
+                      gate1, gate_stride1, cu_seqlens1, nseg1, M1, 0, 0};
+      switch (epilogue) {
+        case EPI_BIAS: return launch_l4_pair_cfg<EPI_BIAS>(cfg, p0, p1, N, K, stream);
+        case EPI_GELU: return launch_l4_pair_cfg<EPI_GELU>(cfg, p0, p1, N, K, stream);
+        case EPI_GATE_RES: return launch_l4_pair_cfg<EPI_GATE_RES>(cfg, p0, p1, N, K, stream);
+        case EPI_RES: return launch_l4_pair_cfg<EPI_RES>(cfg, p0, p1, N, K, stream);
+        default: return launch_l4_pair_cfg<EPI_SILU>(cfg, p0, p1, N, K, stream);
+      }
     }
   }
   if (int rc = gemm_run(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N, K, epilogue, R0, ldr0, gate0, gate_stride0,

@@ -1,0 +1,82 @@
+"""The GEMM tile configurations (256/128-row tiles of several widths, the small
+tiles, split tail rows, paired launches) against the fp32-output kernel."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+if torch.cuda.is_available():
+    from ditserve_amd import ops
+
+# rows at the edges of 64-, 128- and 256-row tiles and of one and several rounds of
+# 256 workgroups; features off every tile width; K from a single 64-k stage (fewer
+# stages than LDS buffers) to more stages than weight-prefetch batches
+SHAPES = [(m, n, k) for n, k in ((1536, 64), (200, 192), (1544, 320), (4616, 128)) for m in (1, 127, 129, 1024, 2305)]
+SHAPES += [(1560, 1536, 1536), (2048, 1536, 2048), (2560, 4608, 448), (1024, 8968, 256), (666, 6144, 576),
+           (3480, 1536, 4160), (16416, 3072, 256), (4096, 1536, 4096),
+           (1560, 4608, 1536), (666, 8960, 704), (5001, 3080, 64), (5001, 1544, 128), (1500, 4616, 192),
+           (2500, 1544, 64), (1500, 1544, 192)]
+
+
+
+def _operands(m, n, k, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    def r(*s):
+        return torch.randn(s, generator=g, device="cuda")
+    return r(m, k).bfloat16(), (r(n, k) * 0.05).bfloat16(), r(n), r(m, n).bfloat16(), r(2, n)
+
+
+def _want(x, w, b, res, gate, seg, epi):
+    """The epilogue in fp32 on the fp32-output kernel's products (whose sums the
+    bf16 kernels share bit for bit)."""
+    y = ops.linear(x, w, b, "f32").bfloat16()
+    f = y.float()
+    if epi == "bias":
+        return y
+    if epi == "gelu":
+        return torch.nn.functional.gelu(f, approximate="tanh")
+    if epi == "silu":
+        return torch.nn.functional.silu(f)
+    if epi == "res":
+        return res.float() + f
+    rows = torch.arange(x.shape[0], device="cuda") >= seg.cu[1]
+    return res.float() + f * gate[rows.long()]
+
+
+def _check(got, want, epi):
+    if epi == "bias":
+        assert torch.equal(got, want)
+        return
+    # one bf16 rounding of the result (2^-9 relative) and of the transcendentals' few fp32 ulps
+    err = (got.float() - want).abs()
+    assert bool((err <= want.abs() * 2.0 ** -8 + 1e-5).all()), float(err.max())
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_tiles_match_the_fp32_output_kernel(m, n, k):
+    x, w, b, res, gate = _operands(m, n, k, m + n + k)
+    seg = ops.Segments([0, m // 3, m], "cuda")
+    for epi in ("bias", "gelu", "silu", "res", "gate_res"):
+        kw = dict(residual=res) if epi in ("res", "gate_res") else {}
+        if epi == "gate_res":
+            kw.update(gate=gate, segments=seg)
+        out = torch.full((m + 1, n), 7.0, device="cuda", dtype=torch.bfloat16)
+        ops.linear(x, w, b, epi, out=out[:m], **kw)
+        _check(out[:m], _want(x, w, b, res, gate, seg, epi), epi)
+        assert bool((out[m] == 7.0).all())  # nothing past the last row
+
+
+@pytest.mark.parametrize("m0,m1,n,k", [(2048, 666, 1536, 6144), (2048, 666, 4608, 1536), (256, 100, 1536, 1536),
+                                       (64, 2048, 1544, 64), (8192, 666, 1536, 256), (129, 1, 200, 128)])
+@pytest.mark.parametrize("epi", ["bias", "gelu", "gate_res"])
+def test_paired_tiles_match_single_launches(m0, m1, n, k, epi):
+    probs = []
+    for m, seed in ((m0, 1), (m1, 2)):
+        x, w, b, res, gate = _operands(m, n, k, seed)
+        p = dict(x=x, w=w, b=b)
+        if epi == "gate_res":
+            p.update(residual=res, gate=gate, segments=ops.Segments([0, m // 2, m], "cuda"))
+        probs.append(p)
+    got = ops.linear_pair(*probs, epi)
+    for g, p in zip(got, probs):
+        assert torch.equal(g, ops.linear(epilogue=epi, **p))
