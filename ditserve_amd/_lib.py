@@ -69,6 +69,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_fns = {}  # entry point name -> bound function of the loaded library
 
 
 class DitkError(RuntimeError):
@@ -88,15 +89,17 @@ def load():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
+        _fns[name] = fn
     _lib = lib
     return lib
 
 
 def call(name, *args):
     """Call entry point `name`; raise DitkError with the library's message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    if _lib is None:
+        load()
+    rc = _fns[name](*args)
     if rc != 0:
-        msg = lib.ditk_last_error().decode(errors="replace")
+        msg = _lib.ditk_last_error().decode(errors="replace")
         raise DitkError(msg or f"{name} failed with status {rc}")
     return rc

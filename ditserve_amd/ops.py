@@ -6,6 +6,7 @@ workers/xfuser/core/attention/spec.py:244-246), allocates outputs with
 ``torch.empty`` when none is given, and launches on the caller's current
 stream without synchronising.  There is no CPU or PyTorch fallback.
 """
+import array
 import ctypes
 import math
 
@@ -18,7 +19,8 @@ _BF16 = torch.bfloat16
 
 
 def _stream():
-    return ctypes_stream(torch.cuda.current_stream())
+    """The current stream's hipStream_t (an int)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def ctypes_stream(stream):
@@ -26,13 +28,13 @@ def ctypes_stream(stream):
 
 
 def _ptr(t):
-    return _lib.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _check(t, name, dtype=None, dims=None):
     if not isinstance(t, torch.Tensor):
         raise ValueError(f"{name} must be a tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be on a cuda (HIP) device, got {t.device}")
     if dtype is not None and t.dtype != dtype:
         raise ValueError(f"{name} must be {dtype}, got {t.dtype}")
@@ -50,6 +52,20 @@ def to_device(data, dtype, device):
     return host.pin_memory().to(device, non_blocking=True)
 
 
+def to_device_tables(tables, device):
+    """Several small host tables in one upload (as to_device): flat lists of ints
+    (int32) or floats (fp32) -> 1-D device views, 16-byte aligned, of one buffer."""
+    words, spans = array.array("i"), []
+    for t in tables:
+        part = array.array("f" if t and isinstance(t[0], float) else "i", t)
+        spans.append((len(words), len(part), part.typecode))
+        words.frombytes(part.tobytes())
+        words.extend([0] * (-len(words) % 4))
+    host = torch.tensor(words, dtype=torch.int32)
+    dev = host.to(device) if torch.device(device).type != "cuda" else host.pin_memory().to(device, non_blocking=True)
+    return [dev[a:a + n] if code == "i" else dev[a:a + n].view(torch.float32) for a, n, code in spans]
+
+
 def _vec(t, name, n):
     """An fp32 per-feature vector (norm weight, bias): 1-D, n long, unit stride (the
     kernels read it as a contiguous array)."""
@@ -61,11 +77,12 @@ def _vec(t, name, n):
 
 def _rows(t, name):
     """2-D row-major view requirements: unit column stride, 16-byte aligned rows."""
-    if t.dim() != 2 or t.stride(1) != 1:
-        raise ValueError(f"{name} must be a 2-D tensor with unit column stride, got strides {t.stride()}")
-    if t.stride(0) % 8 or t.data_ptr() % 16:
+    st = t.stride()
+    if len(st) != 2 or st[1] != 1:
+        raise ValueError(f"{name} must be a 2-D tensor with unit column stride, got strides {st}")
+    if st[0] % 8 or t.data_ptr() % 16:
         raise ValueError(f"{name} rows must be 16-byte aligned (leading dim % 8 == 0)")
-    return t.stride(0)
+    return st[0]
 
 
 class Segments:
@@ -74,11 +91,12 @@ class Segments:
     ``cu`` follows build_cu_seqlens (workers/ditserve/models/sd35_batch.py:135-145):
     [0, n0, n0+n1, ...]."""
 
-    def __init__(self, cu, device):
+    def __init__(self, cu, device, dev=None):
+        """dev: the table already on the device (else it is uploaded here)."""
         self.cu = [int(x) for x in cu]
         if not self.cu or self.cu[0] != 0 or any(b < a for a, b in zip(self.cu, self.cu[1:])):
             raise ValueError(f"cu_seqlens must start at 0 and be nondecreasing, got {self.cu}")
-        self.dev = to_device(self.cu, torch.int32, device)
+        self.dev = dev if dev is not None else to_device(self.cu, torch.int32, device)
         self._nseg, self._total = len(self.cu) - 1, self.cu[-1]
 
     @classmethod
@@ -210,9 +228,9 @@ def adaln(x, shift=None, scale=None, segments=None, weight=None, bias=None, eps=
 
     x [T, D] bf16; shift/scale fp32 views [nseg, D] (row stride may exceed D);
     weight/bias fp32 [D]; kind "ln" (LayerNorm) or "rms" (RMSNorm)."""
-    out, job = _adaln_job(x, shift, scale, segments, weight, bias, eps, kind, out)
-    _lib.call("ditk_adaln", job.x, job.ldx, job.y, job.ldy, job.T, job.D, job.cu_seqlens, job.nseg, job.shift,
-              job.scale, job.mod_stride, job.weight, job.bias, job.eps, job.norm_kind, _stream())
+    out, (xp, ldx, yp, ldy, cu, sh, sc, mod_stride, wp, bp, T, D, nseg, nk, eps) = _adaln_args(
+        x, shift, scale, segments, weight, bias, eps, kind, out)
+    _lib.call("ditk_adaln", xp, ldx, yp, ldy, T, D, cu, nseg, sh, sc, mod_stride, wp, bp, eps, nk, _stream())
     return out
 
 
@@ -222,25 +240,28 @@ def adaln_multi(jobs):
     each is bitwise what adaln() returns for its job.  The jobs run concurrently:
     a job's output may be its own x (in place) but may not overlap another
     job's tensors."""
-    built = [_adaln_job(**j) for j in jobs]
+    built = [_adaln_args(**j) for j in jobs]
     _disjoint_jobs("adaln_multi", [((b[0],), tuple(j.get(k) for k in ("x", "shift", "scale", "weight", "bias")))
                                    for j, b in zip(jobs, built)])
-    arr = (_lib.AdalnJob * len(built))(*[b[1] for b in built])
+    arr = (_lib.AdalnJob * len(built))(*[b[1] for b in built])  # the tuples in field order
     _lib.call("ditk_adaln_multi", arr, len(built), _stream())
     return [b[0] for b in built]
 
 
-def _adaln_job(x, shift=None, scale=None, segments=None, weight=None, bias=None, eps=1e-6, kind="ln", out=None):
-    """Checks one adaln() call; returns (out, its ditk_adaln_job)."""
+def _adaln_args(x, shift=None, scale=None, segments=None, weight=None, bias=None, eps=1e-6, kind="ln", out=None):
+    """Checks one adaln() call; returns (out, its ditk_adaln_job as a tuple of the fields)."""
     _check(x, "x", _BF16, 2)
     T, D = x.shape
     ldx = _rows(x, "x")
     if out is None:
-        out = torch.empty((T, D), dtype=_BF16, device=x.device)
-    _check(out, "out", _BF16, 2)
-    if out.shape != (T, D):
-        raise ValueError(f"out must be [{T}, {D}], got {tuple(out.shape)}")
-    ldy = _rows(out, "out")
+        out, ldy = torch.empty((T, D), dtype=_BF16, device=x.device), D
+        if D % 8:
+            raise ValueError("out rows must be 16-byte aligned (leading dim % 8 == 0)")
+    else:
+        _check(out, "out", _BF16, 2)
+        if out.shape != (T, D):
+            raise ValueError(f"out must be [{T}, {D}], got {tuple(out.shape)}")
+        ldy = _rows(out, "out")
     mod_stride = 0
     cu = None
     nseg = 0
@@ -264,9 +285,8 @@ def _adaln_job(x, shift=None, scale=None, segments=None, weight=None, bias=None,
             _vec(t, n, D)
     if kind not in ("ln", "rms"):
         raise ValueError(f"kind must be 'ln' or 'rms', got {kind!r}")
-    job = _lib.AdalnJob(_ptr(x), ldx, _ptr(out), ldy, _ptr(cu), _ptr(shift), _ptr(scale), mod_stride, _ptr(weight),
-                        _ptr(bias), T, D, nseg, {"ln": 0, "rms": 1}[kind], float(eps))
-    return out, job
+    return out, (_ptr(x), ldx, _ptr(out), ldy, _ptr(cu), _ptr(shift), _ptr(scale), mod_stride, _ptr(weight),
+                 _ptr(bias), T, D, nseg, 0 if kind == "ln" else 1, float(eps))
 
 
 def modulation(table, proj):
@@ -289,7 +309,8 @@ class Rope:
     """3D RoPE description for a packed batch: per-axis cos/sin tables
     [max_pos, head_dim/2] fp32 (float64-built), per-segment (F', H', W') grids."""
 
-    def __init__(self, cos_tab, sin_tab, grids, segments, t_pairs, h_pairs):
+    def __init__(self, cos_tab, sin_tab, grids, segments, t_pairs, h_pairs, grids_dev=None):
+        """grids_dev: the flat grids already on the device (else they are uploaded here)."""
         for t, n in ((cos_tab, "cos table"), (sin_tab, "sin table")):
             _check(t, n, torch.float32, 2)
             if not t.is_contiguous() or t.shape != cos_tab.shape:
@@ -298,7 +319,8 @@ class Rope:
             if max(g) > cos_tab.shape[0]:
                 raise ValueError(f"grid {tuple(g)} reaches past the {cos_tab.shape[0]}-position RoPE tables")
         self.cos, self.sin = cos_tab, sin_tab
-        self.grids = to_device([list(map(int, g)) for g in grids], torch.int32, cos_tab.device).reshape(-1)
+        self.grids = (grids_dev if grids_dev is not None else
+                      to_device([list(map(int, g)) for g in grids], torch.int32, cos_tab.device).reshape(-1))
         self.segments = segments
         self.t_pairs, self.h_pairs = int(t_pairs), int(h_pairs)
         if len(grids) != segments.nseg:
@@ -416,26 +438,30 @@ def _linear_args(x, w, b, epilogue, residual, gate, segments, out):
         raise ValueError(f"unknown epilogue {epilogue!r}")
     odt = torch.float32 if epilogue == "f32" else _BF16
     if out is None:
-        out = torch.empty((M, N), dtype=odt, device=x.device)
-    _check(out, "out", odt, 2)
-    if out.shape != (M, N) or out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16:
-        raise ValueError("out must be [M, N], unit column stride, leading dim % 8 == 0, 16-byte aligned")
+        out, ldc = torch.empty((M, N), dtype=odt, device=x.device), N
+    else:
+        _check(out, "out", odt, 2)
+        ldc, unit = out.stride()
+        if out.shape != (M, N) or unit != 1 or ldc % 8 or out.data_ptr() % 16:
+            raise ValueError("out must be [M, N], unit column stride, leading dim % 8 == 0, 16-byte aligned")
     if N % 8 or K % 32:
         raise ValueError(f"linear needs N % 8 == 0 and K % 32 == 0 (got N={N}, K={K})")
     ldr, gate_stride, cu, nseg = 0, 0, None, 0
     if epilogue in ("gate_res", "res"):
         _check(residual, "residual", _BF16, 2)
-        if residual.shape != (M, N) or residual.stride(1) != 1 or residual.stride(0) % 8 or residual.data_ptr() % 16:
+        ldr, unit = residual.stride()
+        if residual.shape != (M, N) or unit != 1 or ldr % 8 or residual.data_ptr() % 16:
             raise ValueError("residual must be [M, N] row-major with 16-byte aligned rows")
-        ldr = residual.stride(0)
     if epilogue == "gate_res":
         _check(gate, "gate", torch.float32, 2)
         if segments is None or segments.total != M:
             raise ValueError("gated epilogue needs segments covering M rows")
-        if gate.shape != (segments.nseg, N) or gate.stride(1) != 1 or gate.stride(0) % 4 or gate.data_ptr() % 16:
-            raise ValueError(f"gate must be [{segments.nseg}, {N}] with unit column stride and 16-byte aligned rows")
-        gate_stride, cu, nseg = gate.stride(0), segments.dev, segments.nseg
-    return out, (_ptr(x), lda, _ptr(w), ldw, _ptr(b), _ptr(out), out.stride(0), M, _ptr(residual), ldr, _ptr(gate),
+        nseg = segments.nseg
+        gate_stride, unit = gate.stride()
+        if gate.shape != (nseg, N) or unit != 1 or gate_stride % 4 or gate.data_ptr() % 16:
+            raise ValueError(f"gate must be [{nseg}, {N}] with unit column stride and 16-byte aligned rows")
+        cu = segments.dev
+    return out, (_ptr(x), lda, _ptr(w), ldw, _ptr(b), _ptr(out), ldc, M, _ptr(residual), ldr, _ptr(gate),
                  gate_stride, _ptr(cu), nseg), N, K
 
 
@@ -456,27 +482,34 @@ def _extent(t):
     """[first, last) byte range a strided view touches (0-size views touch nothing)."""
     if t.numel() == 0:
         return 0, 0
-    span = 1 + sum((n - 1) * st for n, st in zip(t.shape, t.stride()))
-    return t.data_ptr(), t.data_ptr() + span * t.element_size()
+    span = 1
+    for n, st in zip(t.shape, t.stride()):
+        span += (n - 1) * st
+    p = t.data_ptr()
+    return p, p + span * t.element_size()
+
+
+def _meet(a, b):
+    """Whether two extents share a byte."""
+    return a[0] < b[1] and b[0] < a[1]
 
 
 def _overlap(a, b):
-    a0, a1 = _extent(a)
-    b0, b1 = _extent(b)
-    return a0 < b1 and b0 < a1
+    return _meet(_extent(a), _extent(b))
 
 
 def _disjoint_jobs(fn, jobs_io):
     """jobs_io: per job (outputs, operands).  The jobs of one launch run
     concurrently, so no job's output may overlap another job's operands or
     outputs (its own operands it may overwrite in place)."""
-    for i, (outs, _) in enumerate(jobs_io):
-        for j, (outs_j, ops_j) in enumerate(jobs_io):
+    spans = [([_extent(t) for t in outs], [_extent(t) for t in ops_ if t is not None]) for outs, ops_ in jobs_io]
+    for i, (outs, _) in enumerate(spans):
+        for j, (outs_j, ops_j) in enumerate(spans):
             if i == j:
                 continue
             for o in outs:
                 for t in (*outs_j, *ops_j):
-                    if t is not None and _overlap(o, t):
+                    if _meet(o, t):
                         raise ValueError(f"{fn}: job {i}'s output overlaps a tensor of job {j}")
 
 
@@ -496,11 +529,14 @@ def linear_pair(p0, p1, epilogue="bias"):
         raise ValueError(f"linear_pair needs one N and K (got {N0}x{K0} and {N1}x{K1})")
     # the two products' tiles run concurrently in one launch or in order in two,
     # whichever pays: one product's output may not overlap the other's operands
-    for out, other, name in ((o0, p1, "second"), (o1, p0, "first")):
-        for key in ("x", "w", "b", "residual", "gate", "out"):
-            t = other.get(key) if key != "out" else (o1 if out is o0 else o0)
-            if t is not None and _overlap(out, t):
+    e0, e1 = _extent(o0), _extent(o1)
+    for out, other, other_out, name in ((e0, p1, e1, "second"), (e1, p0, e0, "first")):
+        for key in ("x", "w", "b", "residual", "gate"):
+            t = other.get(key)
+            if t is not None and _meet(out, _extent(t)):
                 raise ValueError(f"linear_pair: an output overlaps the {name} product's {key}")
+        if _meet(out, other_out):
+            raise ValueError(f"linear_pair: an output overlaps the {name} product's out")
     _lib.call("ditk_gemm_pair", *a0, *a1, N0, K0, EPILOGUES[epilogue], _stream())
     return o0, o1
 
@@ -510,7 +546,8 @@ def linear_pair(p0, p1, epilogue="bias"):
 # ---------------------------------------------------------------------------
 
 def vt_columns(tk, nseg):
-    return int(_lib.load().ditk_vt_columns(int(tk), int(nseg)))
+    lib = _lib.load()
+    return lib.ditk_vt_columns(int(tk), int(nseg))
 
 
 def transpose_v(v, heads, head_dim, segments, out=None):
@@ -524,9 +561,10 @@ def transpose_v(v, heads, head_dim, segments, out=None):
     cols = vt_columns(v.shape[0], segments.nseg)
     if out is None:
         out = torch.empty((heads, head_dim, cols), dtype=_BF16, device=v.device)
-    _check(out, "out", _BF16, 3)
-    if out.shape != (heads, head_dim, cols) or not out.is_contiguous():
-        raise ValueError(f"out must be a contiguous [{heads}, {head_dim}, {cols}] buffer")
+    else:
+        _check(out, "out", _BF16, 3)
+        if out.shape != (heads, head_dim, cols) or not out.is_contiguous():
+            raise ValueError(f"out must be a contiguous [{heads}, {head_dim}, {cols}] buffer")
     _lib.call("ditk_transpose_v", _ptr(v), ldv, _ptr(out), cols, v.shape[0], heads, head_dim,
               _ptr(segments.dev), segments.nseg, _stream())
     return out
@@ -566,11 +604,12 @@ def flash_attn_varlen(q, k, v, seg_q, seg_k, heads, head_dim, softmax_scale=None
         vt = transpose_v(v, heads, head_dim, seg_k)
     Tq = q.shape[0]
     if out is None:
-        out = torch.empty((Tq, width), dtype=_BF16, device=q.device)
-    _check(out, "out", _BF16, 2)
-    if out.shape != (Tq, width):
-        raise ValueError(f"out must be [{Tq}, {width}], got {tuple(out.shape)}")
-    ldo = _rows(out, "out")
+        out, ldo = torch.empty((Tq, width), dtype=_BF16, device=q.device), width
+    else:
+        _check(out, "out", _BF16, 2)
+        if out.shape != (Tq, width):
+            raise ValueError(f"out must be [{Tq}, {width}], got {tuple(out.shape)}")
+        ldo = _rows(out, "out")
     lse = torch.empty((heads, Tq), dtype=torch.float32, device=q.device) if return_lse else None
     # with no keys at all no K tile is read: any valid address stands in for the empty K
     kp = _ptr(k) if k.shape[0] else _ptr(vt)
@@ -658,10 +697,9 @@ def solver_step(x, cond, coef, uncond=None, x_last=None, m_prev=None, m_prev2=No
         raise ValueError("solver_step: x must be contiguous")
     if x_next is None:
         x_next = torch.empty_like(x)
-    arr = (ctypes.c_float * 11)(*[float(c) for c in coef])
-    opt = lambda t: _ptr(t) if t is not None else None  # noqa: E731
-    _lib.call("ditk_solver_step", _ptr(x), _ptr(cond), opt(uncond), opt(x_last), opt(m_prev), opt(m_prev2),
-              _ptr(x_next), opt(x_corr), opt(m_out), n, ctypes.addressof(arr), _stream())
+    arr = (ctypes.c_float * 11)(*coef)
+    _lib.call("ditk_solver_step", _ptr(x), _ptr(cond), _ptr(uncond), _ptr(x_last), _ptr(m_prev), _ptr(m_prev2),
+              _ptr(x_next), _ptr(x_corr), _ptr(m_out), n, ctypes.addressof(arr), _stream())
     return x_next
 
 

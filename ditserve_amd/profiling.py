@@ -12,6 +12,17 @@ import contextlib
 import torch
 
 
+class _NoRegion:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NO_REGION = _NoRegion()  # stateless: shared by every untimed region
+
+
 class EventProfiler:
     """`only`: names of the regions to time (None: all).  Each timed region costs
     two event records on the stream, which matters on short steps."""
@@ -21,11 +32,14 @@ class EventProfiler:
         self.only = None if only is None else frozenset(only)
         self._events = collections.defaultdict(list)
 
-    @contextlib.contextmanager
     def region(self, name):
+        """Context manager timing the launches inside it as `name`."""
         if not self.enabled or (self.only is not None and name not in self.only):
-            yield
-            return
+            return _NO_REGION
+        return self._timed(name)
+
+    @contextlib.contextmanager
+    def _timed(self, name):
         start = torch.cuda.Event(enable_timing=True)
         end = torch.cuda.Event(enable_timing=True)
         start.record()

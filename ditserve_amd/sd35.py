@@ -19,13 +19,14 @@ Block (sd35_batch.py:647-708), per JointTransformerBlock:
   blocks); gated residuals; GELU-tanh FFNs on image and text.
 """
 import dataclasses
+import itertools
 import math
 
 import torch
 
 from . import ops
 from .ops import Segments
-from .packing import joint_layout
+from .packing import build_cu_seqlens
 from .profiling import NULL as _NULL_PROFILER
 
 _BF16 = torch.bfloat16
@@ -148,13 +149,13 @@ def pos_embed_crop(cfg, hp, wp, device):
     half = cfg.dim // 2
     omega = 1.0 / 10000 ** (torch.arange(half // 2, dtype=torch.float64) / (half / 2.0))
 
-    def enc(pos):
+    def enc(pos):  # a side's encodings, expanded over the other side on the device
         out = torch.outer(pos, omega)
-        return torch.cat([torch.sin(out), torch.cos(out)], dim=1)
+        return torch.cat([torch.sin(out), torch.cos(out)], dim=1).float().to(device)
 
     ew = enc(cols).unsqueeze(0).expand(hp, wp, half)
     eh = enc(rows).unsqueeze(1).expand(hp, wp, half)
-    return torch.cat([ew, eh], dim=-1).reshape(hp * wp, cfg.dim).float().to(device)
+    return torch.cat([ew, eh], dim=-1).reshape(hp * wp, cfg.dim)
 
 
 class SD35Transformer:
@@ -261,7 +262,7 @@ class SD35Transformer:
         """Per-head QK RMSNorm (in place on the qkv buffer) + varlen flash over seg
         (wq carries the softmax pre-scale)."""
         D, H, Dh = self.cfg.dim, self.cfg.heads, self.cfg.head_dim
-        q, k, v = qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:]
+        q, k, v = qkv.split(D, 1)
         ops.qk_norm_rope_(q, k, wq, wk, Dh, self.cfg.eps, per_head=True)
         with self.profiler.region("attn_dual_core"):
             return ops.flash_attn_varlen(q, k, v, seg, seg, H, Dh, q_prescaled=True)
@@ -272,15 +273,16 @@ class SD35Transformer:
         with prof.region("adaln"):
             # image AdaLN-Zero (and the dual branch's), text AdaLN-Zero or, in the last
             # block, AdaLN-Continuous (scale, shift): one launch
-            emb = mod[:, slice(*blk["n1_cols"])]  # [M, 6D or 9D]
-            embc = mod[:, slice(*blk["n1c_cols"])]  # [M, 2D] (last) or [M, 6D]
-            jobs = [dict(x=h, shift=emb[:, 0:D], scale=emb[:, D:2 * D], segments=seg_img, eps=eps)]
+            # mod: the [M, D] column blocks of the stacked modulations
+            emb = mod[blk["n1_cols"][0] // D:blk["n1_cols"][1] // D]  # 6 or 9 of them
+            embc = mod[blk["n1c_cols"][0] // D:blk["n1c_cols"][1] // D]  # 2 (last) or 6
+            jobs = [dict(x=h, shift=emb[0], scale=emb[1], segments=seg_img, eps=eps)]
             if blk["last"]:
-                jobs.append(dict(x=c, shift=embc[:, D:2 * D], scale=embc[:, 0:D], segments=seg_txt, eps=eps))
+                jobs.append(dict(x=c, shift=embc[1], scale=embc[0], segments=seg_txt, eps=eps))
             else:
-                jobs.append(dict(x=c, shift=embc[:, 0:D], scale=embc[:, D:2 * D], segments=seg_txt, eps=eps))
+                jobs.append(dict(x=c, shift=embc[0], scale=embc[1], segments=seg_txt, eps=eps))
             if blk["dual"]:
-                jobs.append(dict(x=h, shift=emb[:, 6 * D:7 * D], scale=emb[:, 7 * D:8 * D], segments=seg_img, eps=eps))
+                jobs.append(dict(x=h, shift=emb[6], scale=emb[7], segments=seg_img, eps=eps))
             normed = ops.adaln_multi(jobs)
             nh, nc = normed[0], normed[1]
             nh2 = normed[2] if blk["dual"] else None
@@ -290,45 +292,46 @@ class SD35Transformer:
             with prof.region("gemm_qkv_txt"):
                 qkv_t = ops.linear(nc, *blk["qkv_t"])
         with prof.region("joint_prep"):
-            D3 = 3 * D
+            q_i, k_i, v_i = qkv_i.split(D, 1)
+            q_t, k_t, v_t = qkv_t.split(D, 1)
             with prof.region("qk_norm"):  # image and text per-head QK RMSNorm, in place, one launch
                 ops.qk_norm_multi([
-                    dict(q=qkv_i[:, :D], k=qkv_i[:, D:2 * D], wq=blk["nq_pre"], wk=blk["nk"], head_dim=cfg.head_dim,
+                    dict(q=q_i, k=k_i, wq=blk["nq_pre"], wk=blk["nk"], head_dim=cfg.head_dim,
                          eps=eps, per_head=True),
-                    dict(q=qkv_t[:, :D], k=qkv_t[:, D:2 * D], wq=blk["nqt_pre"], wk=blk["nkt"],
+                    dict(q=q_t, k=k_t, wq=blk["nqt_pre"], wk=blk["nkt"],
                          head_dim=cfg.head_dim, eps=eps, per_head=True)])
             # image and text rows are read in place: no gather / scatter copies
             with prof.region("transpose_v_joint"):
-                vt = ops.transpose_v_joint(qkv_i[:, 2 * D:D3], qkv_t[:, 2 * D:D3], cfg.heads, cfg.head_dim,
+                vt = ops.transpose_v_joint(v_i, v_t, cfg.heads, cfg.head_dim,
                                            seg_img, seg_txt, seg_joint)
         with prof.region("attn_joint"):
             a_img, a_txt = ops.joint_attention_q_prescaled(
-                qkv_i[:, :D], qkv_t[:, :D], qkv_i[:, D:2 * D], qkv_t[:, D:2 * D], vt, seg_img, seg_txt,
+                q_i, q_t, k_i, k_t, vt, seg_img, seg_txt,
                 seg_joint, cfg.heads, cfg.head_dim)
         with prof.region("gemm_out"):
-            img = dict(x=a_img, w=blk["out"][0], b=blk["out"][1], residual=h, gate=emb[:, 2 * D:3 * D],
+            img = dict(x=a_img, w=blk["out"][0], b=blk["out"][1], residual=h, gate=emb[2],
                        segments=seg_img)
             if blk["last"]:
                 h = ops.linear(epilogue="gate_res", **img)
             else:  # image and text output projections, one launch where that pays
                 with prof.region("gemm_out_pair"):
                     h, c = ops.linear_pair(img, dict(x=a_txt, w=blk["out_t"][0], b=blk["out_t"][1], residual=c,
-                                                     gate=embc[:, 2 * D:3 * D], segments=seg_txt), "gate_res")
+                                                     gate=embc[2], segments=seg_txt), "gate_res")
         if blk["dual"]:
             with prof.region("attn_dual"):
                 qkv2 = ops.linear(nh2, *blk["qkv2"])
                 a2 = self._attention(qkv2, seg_img, blk["nq2_pre"], blk["nk2"])
-                ops.linear(a2, *blk["out2"], "gate_res", residual=h, gate=emb[:, 8 * D:9 * D], segments=seg_img, out=h)
+                ops.linear(a2, *blk["out2"], "gate_res", residual=h, gate=emb[8], segments=seg_img, out=h)
         with prof.region("ffn"):
-            jobs = [dict(x=h, shift=emb[:, 3 * D:4 * D], scale=emb[:, 4 * D:5 * D], segments=seg_img, eps=eps)]
+            jobs = [dict(x=h, shift=emb[3], scale=emb[4], segments=seg_img, eps=eps)]
             if not blk["last"]:
-                jobs.append(dict(x=c, shift=embc[:, 3 * D:4 * D], scale=embc[:, 4 * D:5 * D], segments=seg_txt,
+                jobs.append(dict(x=c, shift=embc[3], scale=embc[4], segments=seg_txt,
                                  eps=eps))
             normed = ops.adaln_multi(jobs)
             n2 = normed[0]
             with prof.region("gemm_ffn_up_img"):
                 fx = ops.linear(n2, *blk["ff1"], "gelu")
-            img = dict(x=fx, w=blk["ff2"][0], b=blk["ff2"][1], residual=h, gate=emb[:, 5 * D:6 * D],
+            img = dict(x=fx, w=blk["ff2"][0], b=blk["ff2"][1], residual=h, gate=emb[5],
                        segments=seg_img, out=h)
             if blk["last"]:
                 ops.linear(epilogue="gate_res", **img)
@@ -336,7 +339,7 @@ class SD35Transformer:
             fc = ops.linear(normed[1], *blk["ffc1"], "gelu")
             with prof.region("gemm_ffn_down_pair"):
                 ops.linear_pair(img, dict(x=fc, w=blk["ffc2"][0], b=blk["ffc2"][1], residual=c,
-                                          gate=embc[:, 5 * D:6 * D], segments=seg_txt, out=c), "gate_res")
+                                          gate=embc[5], segments=seg_txt, out=c), "gate_res")
         return h, c
 
     # ------------------------------------------------------------------ forward
@@ -366,27 +369,29 @@ class SD35Transformer:
                 raise ValueError(f"text contexts must be [L, {cfg.text_dim}], got {tuple(t.shape)}")
         txts = [t.reshape(-1, cfg.text_dim) for t in texts]
         txt_counts = [t.shape[0] for t in txts]
-        lay = joint_layout(img_counts, txt_counts)
-        seg_img, seg_txt = Segments(lay["cu_img"], dev), Segments(lay["cu_txt"], dev)
-        seg_joint = Segments(lay["cu_joint"], dev)
+        cu_img, cu_txt = build_cu_seqlens(img_counts), [0, *itertools.accumulate(txt_counts)]
+        cu_joint = [a + b for a, b in zip(cu_img, cu_txt)]
+        cus = (cu_img, cu_txt, cu_joint)
+        *cu_dev, t = ops.to_device_tables([*cus, [float(x) for x in timesteps]], dev)
+        seg_img, seg_txt, seg_joint = (Segments(c, dev, d) for c, d in zip(cus, cu_dev))
         # prelude: patch embed (+ cropped 2D sin-cos positions), context embedder, temb
         h = torch.empty((seg_img.total, D), dtype=_BF16, device=dev)
         for m, (l, (hp, wp)) in enumerate(zip(lats, hw)):
             patches = ops.patchify(l.reshape(cfg.in_ch, 1, *l.shape[1:]).to(_BF16), (1, P, P))
             rows = h[seg_img.cu[m]:seg_img.cu[m + 1]]
             ops.linear(patches, self.pe_w, self.pe_b, "res", residual=self._pos(hp, wp), out=rows)
-        c = ops.linear(torch.cat([t.to(device=dev, dtype=_BF16) for t in txts]), *self.ctx)
-        t = ops.to_device([float(x) for x in timesteps], torch.float32, dev)
+        c = ops.linear(torch.cat([x.to(device=dev, dtype=_BF16) for x in txts]), *self.ctx)
         te = ops.linear(ops.linear(ops.timestep_embedding(t, cfg.freq_dim), *self.te1, "silu"), *self.te2)
         pooled = torch.stack([p.reshape(-1) for p in pooleds]).to(device=dev, dtype=_BF16)
         temb = ops.linear(ops.linear(pooled, *self.pp1, "silu"), *self.pp2, "res", residual=te)
         st = ops.silu(temb)
-        mod = ops.linear(st, self.mod_w, self.mod_b, "f32")  # every block's modulation + norm_out
+        # every block's modulation + norm_out, as [M, D] column blocks
+        mod = ops.linear(st, self.mod_w, self.mod_b, "f32").split(D, 1)
         for i in range(cfg.layers):
             h, c = self._block(i, h, c, mod, seg_img, seg_txt, seg_joint)
         # epilogue: AdaLN-Continuous norm_out (scale, shift), proj_out, per-request unpatchify
-        embo = mod[:, slice(*self.norm_out_cols)]
-        x = ops.adaln(h, embo[:, D:2 * D], embo[:, 0:D], seg_img, eps=cfg.eps)
+        scale, shift = mod[self.norm_out_cols[0] // D:self.norm_out_cols[1] // D]
+        x = ops.adaln(h, shift, scale, seg_img, eps=cfg.eps)
         y = ops.linear(x, *self.proj_out)
         outs = []
         for m, (hp, wp) in enumerate(hw):
@@ -397,12 +402,12 @@ class SD35Transformer:
             "attention_backend": "ditk_flash_varlen",
             "attention_provider": "ditk",
             "packed_segments": n,
-            "cu_seqlens_img": lay["cu_img"],
-            "cu_seqlens_txt": lay["cu_txt"],
-            "cu_seqlens_joint": lay["cu_joint"],
-            "packed_image_tokens": lay["cu_img"][-1],
+            "cu_seqlens_img": cu_img,
+            "cu_seqlens_txt": cu_txt,
+            "cu_seqlens_joint": cu_joint,
+            "packed_image_tokens": cu_img[-1],
             "padded_image_tokens": n * max(img_counts),
-            "padding_saved_tokens": n * max(img_counts) - lay["cu_img"][-1],
+            "padding_saved_tokens": n * max(img_counts) - cu_img[-1],
         }
         return outs, meta
 

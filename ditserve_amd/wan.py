@@ -24,6 +24,7 @@ Block arithmetic follows workers/ditserve/models/wan/block.py:276-297:
   h  = h + W2 GELU_tanh(W1 n) * c_gate                       (GELU epilogue; gate epilogue)
 """
 import dataclasses
+import itertools
 import math
 import weakref
 
@@ -257,7 +258,11 @@ class WanTransformer:
                 raise ValueError(f"latents must be [{cfg.in_ch}, F, H, W], got {tuple(lat.shape)}")
         grids = [self._grid(l.shape) for l in latents]
         counts = [g[0] * g[1] * g[2] for g in grids]
-        seg = Segments([0] + [sum(counts[: i + 1]) for i in range(len(counts))], dev)
+        text_lens = [int(t.shape[-2]) for t in texts]
+        cu, cu_txt = [0, *itertools.accumulate(counts)], [0, *itertools.accumulate(text_lens)]
+        cu_dev, cu_txt_dev, grids_dev, t = ops.to_device_tables(
+            [cu, cu_txt, [n for g in grids for n in g], [float(x) for x in timesteps]], dev)
+        seg, seg_txt = Segments(cu, dev, cu_dev), Segments(cu_txt, dev, cu_txt_dev)
         hidden = torch.empty((seg.total, cfg.dim), dtype=_BF16, device=dev)
         cache = {}
         for i, lat in enumerate(latents):
@@ -268,12 +273,9 @@ class WanTransformer:
             patches = ops.patchify(lat.reshape(lat.shape[-4:]).to(_BF16), cfg.patch)
             ops.linear(patches, self.patch_w, self.patch_b, out=hidden[seg.cu[i]:seg.cu[i + 1]])
             cache[key] = (seg.cu[i], seg.cu[i + 1])
-        text_lens = [int(t.shape[-2]) for t in texts]
-        seg_txt = Segments([0] + [sum(text_lens[: i + 1]) for i in range(len(text_lens))], dev)
-        text = torch.cat([t.reshape(-1, cfg.text_dim).to(device=dev, dtype=_BF16) for t in texts])
-        t = ops.to_device([float(x) for x in timesteps], torch.float32, dev)
+        text = torch.cat([x.reshape(-1, cfg.text_dim).to(device=dev, dtype=_BF16) for x in texts])
         temb, projected, enc = self.condition(t, text)
-        rope = ops.Rope(self.rope_cos, self.rope_sin, grids, seg, self.rope_pairs[0], self.rope_pairs[1])
+        rope = ops.Rope(self.rope_cos, self.rope_sin, grids, seg, self.rope_pairs[0], self.rope_pairs[1], grids_dev)
         packet = dict(hidden=hidden, encoder=enc, temb=temb, projected=projected, rotary=rope,
                       shape=[(1, *g, *cfg.patch) for g in grids], pad_amount=0, local_rows=0, valid_kv_len=None,
                       thw=[list(g) for g in grids], cu_seqlens_q=seg, cu_seqlens_kv_text=seg_txt, grids=grids)
@@ -330,13 +332,14 @@ class WanTransformer:
         seg, seg_txt = packet["cu_seqlens_q"], packet["cu_seqlens_kv_text"]
         h = packet["hidden"]
         with prof.region("modulation"):
-            mod = ops.modulation(blk["sst"], packet["projected"])  # [R, 6, D] fp32
+            # [R, 6, D] fp32, one [R, D] view per modulation
+            mod = ops.modulation(blk["sst"], packet["projected"]).unbind(1)
         # self-attention (_stage1, block.py:282-285)
         with prof.region("adaln"):
-            x = ops.adaln(h, mod[:, 0], mod[:, 1], seg, eps=cfg.eps)
+            x = ops.adaln(h, mod[0], mod[1], seg, eps=cfg.eps)
         with prof.region("gemm_qkv"):
             qkv = ops.linear(x, blk["qkv_w"], blk["qkv_b"])
-        q, k, v = qkv[:, :D], qkv[:, D:2 * D], qkv[:, 2 * D:]
+        q, k, v = qkv.split(D, 1)
         with prof.region("qk_norm_rope"):
             ops.qk_norm_rope_(q, k, blk["nq1_pre"], blk["nk1"], Dh, cfg.eps, rope=packet["rotary"])
         with prof.region("transpose_v"):
@@ -344,14 +347,14 @@ class WanTransformer:
         with prof.region("attn_self"):
             a = ops.flash_attn_varlen(q, k, None, seg, seg, H, Dh, vt=vt, q_prescaled=True)
         with prof.region("gemm_o_gate"):
-            h = ops.linear(a, blk["o1_w"], blk["o1_b"], "gate_res", residual=h, gate=mod[:, 2], segments=seg)
+            h = ops.linear(a, blk["o1_w"], blk["o1_b"], "gate_res", residual=h, gate=mod[2], segments=seg)
         # cross-attention (_stage2, block.py:288-290)
         with prof.region("cross_prep"):
             x = ops.adaln(h, weight=blk["n2_w"], bias=blk["n2_b"], eps=cfg.eps)
             with prof.region("gemm_cross_q"):
                 q2 = ops.linear(x, blk["q2_w"], blk["q2_b"])
             kv2 = ops.linear(packet["encoder"], blk["kv2_w"], blk["kv2_b"])
-            k2, v2 = kv2[:, :D], kv2[:, D:]
+            k2, v2 = kv2.split(D, 1)
             # RMSNorm across heads of the image queries and the text keys, in place, one launch
             ops.adaln_multi([dict(x=q2, weight=blk["nq2_pre"], eps=cfg.eps, kind="rms", out=q2),
                              dict(x=k2, weight=blk["nk2"], eps=cfg.eps, kind="rms", out=k2)])
@@ -362,11 +365,11 @@ class WanTransformer:
             ops.linear(a, blk["o2_w"], blk["o2_b"], "res", residual=h, out=h)
         # FFN (block.py:291-293)
         with prof.region("adaln"):
-            x = ops.adaln(h, mod[:, 3], mod[:, 4], seg, eps=cfg.eps)
+            x = ops.adaln(h, mod[3], mod[4], seg, eps=cfg.eps)
         with prof.region("gemm_ffn_up_gelu"):
             f = ops.linear(x, blk["f1_w"], blk["f1_b"], "gelu")
         with prof.region("gemm_ffn_down_gate"):
-            ops.linear(f, blk["f2_w"], blk["f2_b"], "gate_res", residual=h, gate=mod[:, 5], segments=seg, out=h)
+            ops.linear(f, blk["f2_w"], blk["f2_b"], "gate_res", residual=h, gate=mod[5], segments=seg, out=h)
         packet["hidden"] = h
         return h
 
