@@ -450,13 +450,13 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m, L4Prefetch pf);
+                                        int group_m, L4Prefetch pf, bool stream_out);
 template <int EPI, int FI, int FJ>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
     const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
     const float* __restrict__ bias, void* __restrict__ Cv, int64_t ldc, int M, int N, int K,
     const bf16_t* R, int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
-    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m, bool prefetch) {
+    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m, bool prefetch, bool stream_out) {
   __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   // Persistent: XCD x (= blockIdx % 8) owns the tiles [x * per_xcd, (x + 1) *
   // per_xcd), which its workgroups take in turn (the order a one-tile-per-
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
   L4Prefetch pf = l4_prefetch(b, nb, N, K, prefetch);
   for (int L = tlo + (b >> 3); L < thi; L += nb >> 3) {
     l4_tile<EPI, FI, FJ>(lds, L, A, lda, W, ldw, bias, Cv, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, tiles_m,
-                     tiles_n, group_m, pf);
+                     tiles_n, group_m, pf, stream_out);
     pf.n = 0;  // once per workgroup
   }
 }
@@ -498,7 +498,7 @@ struct L4Prob {
 // product would compute it.
 template <int EPI, int FI, int FJ>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob p1, int N, int K, int tiles_n,
-                                                           bool prefetch) {
+                                                           bool prefetch, bool stream_out) {
   __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   const int nb = gridDim.x, b = blockIdx.x;
   const int t0 = p0.tiles_m * tiles_n, ntiles = t0 + p1.tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
@@ -515,7 +515,8 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob 
                      s ? p1.ldw : p0.ldw, s ? p1.bias : p0.bias, s ? p1.C : p0.C, s ? p1.ldc : p0.ldc,
                      s ? p1.M : p0.M, N, K, s ? p1.R : p0.R, s ? p1.ldr : p0.ldr, s ? p1.gate : p0.gate,
                      s ? p1.gate_stride : p0.gate_stride, s ? p1.cu : p0.cu, s ? p1.nseg : p0.nseg,
-                     s ? p1.tiles_m : p0.tiles_m, tiles_n, s ? p1.group_m : p0.group_m, pf);
+                     s ? p1.tiles_m : p0.tiles_m, tiles_n, s ? p1.group_m : p0.group_m, pf,
+                         stream_out);
     pf.n = 0;
   }
 }
@@ -526,7 +527,7 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m, L4Prefetch pf) {
+                                        int group_m, L4Prefetch pf, bool stream_out) {
   using G = L4<FI, FJ>;
   constexpr int GBM = G::GBM, GBN = G::GBN, WTM = G::WTM, WTN = G::WTN, STG_ROW = G::STG_ROW;
   const int group = L / (group_m * tiles_n);
@@ -706,7 +707,8 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
         }
         v[q] = pack8(x);
       }
-      __builtin_amdgcn_raw_buffer_store_b128(v[q], cdesc, off[q], 0, 2);  // non-temporal
+      if (stream_out) __builtin_amdgcn_raw_buffer_store_b128(v[q], cdesc, off[q], 0, 2);  // non-temporal
+      else __builtin_amdgcn_raw_buffer_store_b128(v[q], cdesc, off[q], 0, 0);
     }
   }
 }
@@ -768,6 +770,12 @@ bool l4_prefetch_on(int M, int N, int K, int64_t ldw, int gbm) {
   if (tiles_m < (K >= 4096 ? 4 : 8)) return false;
   return (int64_t)N * ldw * 2 < (1ll << 31) && (rem == 0 || (3 * rem > gbm && (gbm == 128 || K >= 4096)));
 }
+// Whether the output is stored past the caches.  Outputs of 64 MB and more are
+// (2.6-3.6% faster on the K = 1536 products of 65520 rows: they would not stay
+// cached until the next kernel reads them); smaller ones stay, and the next kernel
+// finds them (one-frame Wan block 300 -> 281 us, preview step of 2 x 1280 rows
+// 11.20 -> 10.90 ms, SD3.5 512 step 8.65 -> 8.37 ms).
+bool l4_stream_out(int64_t M, int N) { return M * N * 2 >= (64ll << 20); }
 template <int EPI, int FI, int FJ>
 int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
               int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
@@ -778,7 +786,8 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
   const int64_t nblocks = std::min<int64_t>(((int64_t)tiles_m * tiles_n + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
   gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
-      gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM));
+      gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM),
+      l4_stream_out(M, N));
   return ditk_check_launch("ditk_gemm");
 }
 
@@ -793,7 +802,8 @@ int launch_l4_pair(L4Prob p0, L4Prob p1, int N, int K, hipStream_t stream) {
   const int64_t tiles = (int64_t)(p0.tiles_m + p1.tiles_m) * tiles_n;
   const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
   gemm_kernel_l4_pair<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
-      p0, p1, N, K, tiles_n, l4_prefetch_on(p0.M, N, K, p0.ldw, GBM) && (int64_t)N * p1.ldw * 2 < (1ll << 31));
+      p0, p1, N, K, tiles_n, l4_prefetch_on(p0.M, N, K, p0.ldw, GBM) && (int64_t)N * p1.ldw * 2 < (1ll << 31),
+      l4_stream_out(p0.M + (int64_t)p1.M, N));
   return ditk_check_launch("ditk_gemm_pair");
 }
 
