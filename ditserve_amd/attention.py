@@ -97,20 +97,18 @@ def ditk_attention(query, key, value, call=None):
     if reason is not None:
         raise NotImplementedError(f"DITK {reason}")
     b, h, sq, d = query.shape
-    sk = key.shape[2]
-    q = _rows(query)
-    if call.varlen is not None:
+    if call.varlen is None:
+        out, lse = ops.flash_attn_bhsd(query, key, value)
+    else:
+        q = _rows(query)
         kv_k, kv_v = _rows(key), _rows(value)
         idx = call.varlen.indices_k
         k, v = kv_k.index_select(0, idx), kv_v.index_select(0, idx)
         seg_k = ops.Segments.from_device(call.varlen.cu_seqlens_k.to(torch.int32), k.shape[0])
         if seg_k.nseg != b:
             raise ValueError(f"varlen packing describes {seg_k.nseg} batches, query has {b}")
-    else:
-        k, v = _rows(key), _rows(value)
-        seg_k = ops.Segments.uniform(b, sk, query.device)
-    seg_q = ops.Segments.uniform(b, sq, query.device)
-    out, lse = ops.flash_attn_varlen(q, k, v, seg_q, seg_k, h, d, return_lse=True)
+        seg_q = ops.Segments.uniform(b, sq, query.device)
+        out, lse = ops.flash_attn_varlen(q, k, v, seg_q, seg_k, h, d, return_lse=True)
     out = out.view(b, sq, h, d).transpose(1, 2)
     lse = lse.view(h, b, sq).permute(1, 0, 2)
     return out, lse

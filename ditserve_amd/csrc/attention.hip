@@ -41,6 +41,7 @@
 // operand (text tokens) — for Q, K and O alike, so SD3.5's image and text
 // projections feed joint attention, and take its output, without a gather or
 // scatter copy.  Results are bitwise those of the gathered layout.
+#include <algorithm>
 #include <mutex>
 
 #include "ditk_common.h"
@@ -104,7 +105,7 @@ __device__ __forceinline__ int padded_key_start(const int32_t* __restrict__ cu, 
       [vdma_hi] "s"(su((uint32_t)(vdma >> 32))), [lds_k] "s"(su(lds_k)), [lds_v] "s"(su(lds_v)),                   \
       [nkt] "s"(su(nkt)), [valid_last] "s"(su(valid_last)), [ktile] "s"(su(ktile)), [wave1k] "s"(su(wave1k)),      \
       [lds_o] "s"(su(lds_o)), [npass] "s"(su(npass)), [ldqb] "s"(su(ldqb)), [sc] "s"(sc), [qend] "s"(su(q_end)), [ldob] "s"(su(ldob)), [obase_lo] "s"(su((uint32_t)obase)),             \
-      [obase_hi] "s"(su((uint32_t)(obase >> 32))), [has_lse] "s"(su(has_lse)), [lsebase] "s"(su64(lsebase)),      \
+      [obase_hi] "s"(su((uint32_t)(obase >> 32))), [has_lse] "s"(su(has_lse)), [ont] "s"(su(stream_out)), [lsebase] "s"(su64(lsebase)),      \
       [kaddr0] "v"(kaddr[0]), [kaddr1] "v"(kaddr[1]), [kaddr2] "v"(kaddr[2]), [kaddr3] "v"(kaddr[3]),             \
       [vaddr0] "v"(vaddr[0]), [vaddr1] "v"(vaddr[1]), [vaddr2] "v"(vaddr[2]), [vaddr3] "v"(vaddr[3]),             \
       [koff0] "v"(koff[0]), [koff1] "v"(koff[1]), [koff2] "v"(koff[2]), [koff3] "v"(koff[3]),                     \
@@ -119,7 +120,7 @@ __device__ __forceinline__ int padded_key_start(const int32_t* __restrict__ cu, 
       [vdma_hi] "s"(su((uint32_t)(vdma >> 32))), [lds_k] "s"(su(lds_k)), [lds_v] "s"(su(lds_v)),                   \
       [nkt] "s"(su(nkt)), [valid_last] "s"(su(valid_last)), [ktile] "s"(su(ktile)), [wave1k] "s"(su(wave1k)),      \
       [lds_o] "s"(su(lds_o)), [npass] "s"(su(npass)), [ldqb] "s"(su(ldqb)), [qend] "s"(su(q_end)), [ldob] "s"(su(ldob)), [obase_lo] "s"(su((uint32_t)obase)),                           \
-      [obase_hi] "s"(su((uint32_t)(obase >> 32))), [has_lse] "s"(su(has_lse)), [lsebase] "s"(su64(lsebase)),      \
+      [obase_hi] "s"(su((uint32_t)(obase >> 32))), [has_lse] "s"(su(has_lse)), [ont] "s"(su(stream_out)), [lsebase] "s"(su64(lsebase)),      \
       [kaddr0] "v"(kaddr[0]), [kaddr1] "v"(kaddr[1]), [kaddr2] "v"(kaddr[2]), [kaddr3] "v"(kaddr[3]),             \
       [vaddr0] "v"(vaddr[0]), [vaddr1] "v"(vaddr[1]), [vaddr2] "v"(vaddr[2]), [vaddr3] "v"(vaddr[3]),             \
       [koff0] "a"(koff[0]), [koff1] "a"(koff[1]), [koff2] "a"(koff[2]), [koff3] "a"(koff[3]),                     \
@@ -136,33 +137,40 @@ __device__ __forceinline__ int padded_key_start(const int32_t* __restrict__ cu, 
       [otxt_hi] "s"(su((uint32_t)(otxt >> 32))), [qa0lo] "a"((uint32_t)qa[0]), [qa0hi] "a"((uint32_t)(qa[0] >> 32)), \
       [qa1lo] "a"((uint32_t)qa[1]), [qa1hi] "a"((uint32_t)(qa[1] >> 32)), [krow0] "a"(krow_of[0]),                  \
       [krow1] "a"(krow_of[1]), [krow2] "a"(krow_of[2]), [krow3] "a"(krow_of[3])
-constexpr int kXcdChunk = 32;  // work items per XCD chunk (one per CU of an XCD)
-template <int HD, bool PRE, bool JOINT = false>
+// Row r, head h of segment m of an operand lies at base + h * hs + m * sa + r * ld
+// (elements).  Packed rows: hs = head_dim, sa = 0.  A [batch, heads, rows, head_dim]
+// tensor read in place: hs and ld its head and row strides, sa = batch stride -
+// rows * ld (rows count through the batch).
+struct RowLayout {
+  int64_t hs, sa;
+};
+constexpr int kXcdChunk = 32;  // most work items per XCD chunk (one per CU of an XCD)
+template <int HD, bool PRE, bool JOINT, int QB>
 __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
     const bf16_t* __restrict__ Q, int64_t ldq, const bf16_t* __restrict__ Kp, int64_t ldk,
     const bf16_t* __restrict__ Vt, int64_t vt_ld, int64_t vt_hs, bf16_t* __restrict__ O, int64_t ldo,
     float* __restrict__ lse, int64_t lse_ld, const int32_t* __restrict__ cu_q,
-    const int32_t* __restrict__ cu_k, int nseg, int heads, int np, float scale_log2,
+    const int32_t* __restrict__ cu_k, int nseg, int heads, int np, int chunk, bool stream_out, float scale_log2, RowLayout ql, RowLayout kl,
     const bf16_t* __restrict__ Qb = nullptr, const bf16_t* __restrict__ Kb = nullptr, bf16_t* __restrict__ Ob = nullptr,
     const int32_t* __restrict__ cu_a = nullptr, const int32_t* __restrict__ cu_b = nullptr) {
   static_assert(!JOINT || (PRE && HD == 64), "joint sources: pre-scaled head_dim 64");
-  constexpr int NW = 4, BM = 256;
+  constexpr int NW = 4, BM = 128 * QB;  // QB 32-query blocks per wave
   constexpr int ND = HD / 32;  // DMA instructions per wave and operand per tile
   __shared__ u32x4_t Ks[2][BN * HD / 8];
   __shared__ u32x4_t Vs[2][HD * 8];
   constexpr int OPITCH = HD * 2 + 8;  // output staging row pitch (bytes), 32 rows per wave
   __shared__ u32x4_t Os[4 * 32 * OPITCH / 16];
-  // A work item is np consecutive 256-query tiles of one (segment, head), run as
+  // A work item is np consecutive BM-query tiles of one (segment, head), run as
   // passes of the body (the next pass's loads issued under the current pass's
   // last key tile).  Items in segment-major order (segment, then head, then
   // tile), dealt to the 8 XCDs (workgroup b runs on XCD b % 8) in chunks of
-  // kXcdChunk consecutive items: every XCD gets every 8th chunk, so a ragged
-  // batch spreads evenly over the XCDs, and the items running on one XCD at a
-  // time are tiles of the same (segment, head), sharing its K and Vt in that
-  // XCD's L2.  The grid is a multiple of 8 chunks; items past the last exit.
+  // consecutive items: every XCD gets every 8th chunk, so a ragged batch spreads
+  // evenly over the XCDs, and the items running on one XCD at a time are tiles of
+  // the same (segment, head), sharing its K and Vt in that XCD's L2.  The grid is
+  // a multiple of 8 chunks; items past the last exit.
   const int b = blockIdx.x;
   const int j = b >> 3;
-  int t = ((j / kXcdChunk) * 8 + (b & 7)) * kXcdChunk + j % kXcdChunk;
+  int t = ((j / chunk) * 8 + (b & 7)) * chunk + j % chunk;
   int seg = -1, head = 0, npass = 0;
   for (int m = 0, prev = cu_q[0]; m < nseg; ++m) {
     const int next = cu_q[m + 1];
@@ -183,7 +191,7 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
   const int l32 = lane & 31, hh = lane >> 5;
   const int wave_u = __builtin_amdgcn_readfirstlane(wave);
   const int q_end = cu_q[seg + 1];
-  const int qrow0 = cu_q[seg] + t * BM + wave * 64 + l32;
+  const int qrow0 = cu_q[seg] + t * BM + wave * (32 * QB) + l32;
   const int qrow1 = qrow0 + 32;
   const int k_beg = cu_k[seg], k_len = max(cu_k[seg + 1] - k_beg, 0);
   // nkt == 0 (no keys): the body stores zero rows and lse = -inf, issuing no DMA
@@ -192,8 +200,8 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
   const int pk = padded_key_start(cu_k, seg);
   // Q rows past the segment end read its last row (their outputs are not stored);
   // the body forms each lane's 64-bit row address from qbase, its row and ldq
-  const uint64_t qbase = (uint64_t)(uintptr_t)(Q + (int64_t)head * HD);
-  uint64_t kdma = (uint64_t)(uintptr_t)(Kp + (int64_t)head * HD + (int64_t)k_beg * ldk);
+  const uint64_t qbase = (uint64_t)(uintptr_t)(Q + head * ql.hs + seg * ql.sa);
+  uint64_t kdma = (uint64_t)(uintptr_t)(Kp + head * kl.hs + seg * kl.sa + (int64_t)k_beg * ldk);
   // joint: row j of the segment is row a0 + j of the "a" (image) operands while
   // j < len_a, else row b0 + j - len_a of the "b" (text) operands
   int len_a = 0, qseg = 0;
@@ -257,28 +265,46 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
   auto su = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
   auto su64 = [&](uint64_t x) { return ((uint64_t)su((uint32_t)(x >> 32)) << 32) | su((uint32_t)x); };
   const float sc = __builtin_bit_cast(float, su(__builtin_bit_cast(uint32_t, scale_log2)));
-  if constexpr (HD == 128 && !PRE) {
+  (void)sc;
+  if constexpr (HD == 128 && !PRE && QB == 2) {
     asm volatile(
 #include "attn_d128_body.inc"
         : : DITK_ATTN_ASM_OPERANDS : DITK_D128_CLOBBERS "vcc", "scc", "memory");
-  } else if constexpr (HD == 64 && !PRE) {
+  } else if constexpr (HD == 128 && !PRE && QB == 1) {
+    asm volatile(
+#include "attn_d128q1_body.inc"
+        : : DITK_ATTN_ASM_OPERANDS : DITK_D128_CLOBBERS "vcc", "scc", "memory");
+  } else if constexpr (HD == 64 && !PRE && QB == 2) {
     asm volatile(
 #include "attn_d64_body.inc"
         : : DITK_ATTN_ASM_OPERANDS : DITK_D64_CLOBBERS "vcc", "scc", "memory");
-  } else if constexpr (JOINT) {
-    (void)sc;
+  } else if constexpr (HD == 64 && !PRE && QB == 1) {
+    asm volatile(
+#include "attn_d64q1_body.inc"
+        : : DITK_ATTN_ASM_OPERANDS : DITK_D64_CLOBBERS "vcc", "scc", "memory");
+  } else if constexpr (JOINT && QB == 2) {
     asm volatile(
 #include "attn_d64j_body.inc"
         : : DITK_ATTN_ASM_OPERANDS_JOINT : DITK_D64J_CLOBBERS "vcc", "scc", "memory");
-  } else if constexpr (HD == 128) {
-    (void)sc;
+  } else if constexpr (JOINT && QB == 1) {
+    asm volatile(
+#include "attn_d64jq1_body.inc"
+        : : DITK_ATTN_ASM_OPERANDS_JOINT : DITK_D64J_CLOBBERS "vcc", "scc", "memory");
+  } else if constexpr (HD == 128 && PRE && QB == 2) {
     asm volatile(
 #include "attn_d128p_body.inc"
         : : DITK_ATTN_ASM_OPERANDS_PRE : DITK_D128P_CLOBBERS "vcc", "scc", "memory");
-  } else {
-    (void)sc;
+  } else if constexpr (HD == 128 && PRE && QB == 1) {
+    asm volatile(
+#include "attn_d128pq1_body.inc"
+        : : DITK_ATTN_ASM_OPERANDS_PRE : DITK_D128P_CLOBBERS "vcc", "scc", "memory");
+  } else if constexpr (HD == 64 && PRE && QB == 2) {
     asm volatile(
 #include "attn_d64p_body.inc"
+        : : DITK_ATTN_ASM_OPERANDS_PRE : DITK_D64P_CLOBBERS "vcc", "scc", "memory");
+  } else if constexpr (HD == 64 && PRE && QB == 1) {
+    asm volatile(
+#include "attn_d64pq1_body.inc"
         : : DITK_ATTN_ASM_OPERANDS_PRE : DITK_D64P_CLOBBERS "vcc", "scc", "memory");
   }
 }
@@ -291,7 +317,7 @@ template <int HD>
 __global__ __launch_bounds__(256) void transpose_v_kernel(const bf16_t* __restrict__ V, int64_t ldv,
                                                           bf16_t* __restrict__ Vt, int64_t vt_ld,
                                                           int64_t vt_hs, const int32_t* __restrict__ cu,
-                                                          int nseg, const bf16_t* __restrict__ Vb,
+                                                          int nseg, RowLayout vl, const bf16_t* __restrict__ Vb,
                                                           const int32_t* __restrict__ cu_a,
                                                           const int32_t* __restrict__ cu_b) {
   // LDS tile of 32-bit words: word (d, p) holds keys 2p (low half) and 2p + 1 of
@@ -308,7 +334,7 @@ __global__ __launch_bounds__(256) void transpose_v_kernel(const bf16_t* __restri
   const int k0 = cu[seg] + t * BN;
   const int k_end = cu[seg + 1];
   const int col0 = padded_key_start(cu, seg) + t * BN;
-  const bf16_t* Vh = V + (int64_t)head * HD;
+  const bf16_t* Vh = V + head * vl.hs + seg * vl.sa;
   constexpr int CH = HD / 8;
   // row r of this tile (zero past the segment end)
   auto load_row = [&](int r, int ch) {
@@ -355,7 +381,7 @@ DITK_EXPORT int64_t ditk_vt_columns(int64_t Tk, int nseg) {
 namespace {
 int transpose_launch(const void* v, const void* vb, int64_t ldv, void* vt, int64_t vt_ld, int Tk, int heads,
                      int head_dim, const int32_t* cu_k, const int32_t* cu_a, const int32_t* cu_b, int nseg,
-                     hipStream_t stream) {
+                     RowLayout vl, hipStream_t stream) {
   DITK_REQUIRE(cu_k && (Tk == 0 || (v && vt)), "ditk_transpose_v: null tensor");
   DITK_REQUIRE(head_dim == 64 || head_dim == 128, "ditk_transpose_v: head_dim must be 64 or 128");
   DITK_REQUIRE(nseg > 0 && heads > 0 && Tk >= 0, "ditk_transpose_v: bad sizes");
@@ -369,10 +395,10 @@ int transpose_launch(const void* v, const void* vb, int64_t ldv, void* vt, int64
   const int64_t hs = (int64_t)head_dim * vt_ld;
   if (head_dim == 128)
     transpose_v_kernel<128><<<grid, 256, 0, stream>>>((const bf16_t*)v, ldv, (bf16_t*)vt, vt_ld, hs, cu_k, nseg,
-                                                       (const bf16_t*)vb, cu_a, cu_b);
+                                                       vl, (const bf16_t*)vb, cu_a, cu_b);
   else
     transpose_v_kernel<64><<<grid, 256, 0, stream>>>((const bf16_t*)v, ldv, (bf16_t*)vt, vt_ld, hs, cu_k, nseg,
-                                                      (const bf16_t*)vb, cu_a, cu_b);
+                                                      vl, (const bf16_t*)vb, cu_a, cu_b);
   return ditk_check_launch("ditk_transpose_v");
 }
 }  // namespace
@@ -380,14 +406,16 @@ int transpose_launch(const void* v, const void* vb, int64_t ldv, void* vt, int64
 DITK_EXPORT int ditk_transpose_v(const void* v, int64_t ldv, void* vt, int64_t vt_ld, int Tk,
                                  int heads, int head_dim, const int32_t* cu_k, int nseg,
                                  hipStream_t stream) {
-  return transpose_launch(v, nullptr, ldv, vt, vt_ld, Tk, heads, head_dim, cu_k, nullptr, nullptr, nseg, stream);
+  return transpose_launch(v, nullptr, ldv, vt, vt_ld, Tk, heads, head_dim, cu_k, nullptr, nullptr, nseg,
+                          RowLayout{head_dim, 0}, stream);
 }
 
 DITK_EXPORT int ditk_transpose_v_joint(const void* v_a, const void* v_b, int64_t ldv, void* vt, int64_t vt_ld,
                                        int T_joint, int heads, int head_dim, const int32_t* cu_a,
                                        const int32_t* cu_b, const int32_t* cu_joint, int nseg, hipStream_t stream) {
   DITK_REQUIRE(v_a && v_b && cu_a && cu_b, "ditk_transpose_v_joint: null tensor");
-  return transpose_launch(v_a, v_b, ldv, vt, vt_ld, T_joint, heads, head_dim, cu_joint, cu_a, cu_b, nseg, stream);
+  return transpose_launch(v_a, v_b, ldv, vt, vt_ld, T_joint, heads, head_dim, cu_joint, cu_a, cu_b, nseg,
+                          RowLayout{head_dim, 0}, stream);
 }
 
 namespace {
@@ -395,12 +423,12 @@ namespace {
 // takes q.k to log2 units inside the kernel (unused when pre)
 int flash_launch(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* vt, int64_t vt_ld, void* o,
                  int64_t ldo, float* lse, int64_t lse_ld, const int32_t* cu_q, const int32_t* cu_k, int nseg, int Tq,
-                 int heads, int head_dim, float sl2, bool pre, hipStream_t stream, const void* qb = nullptr,
-                 const void* kb = nullptr, void* ob = nullptr, const int32_t* cu_a = nullptr,
+                 int heads, int head_dim, float sl2, bool pre, RowLayout ql, RowLayout kl, hipStream_t stream,
+                 const void* q2 = nullptr, const void* kb = nullptr, void* ob = nullptr, const int32_t* cu_a = nullptr,
                  const int32_t* cu_b = nullptr) {
   const bool joint = cu_a != nullptr;
-  DITK_REQUIRE(!joint || (pre && qb && kb && ob && cu_b), "ditk_joint_attn: needs both sources and both tables");
-  DITK_REQUIRE(!joint || (((uintptr_t)qb % 16) == 0 && ((uintptr_t)kb % 16) == 0 && ((uintptr_t)ob % 8) == 0),
+  DITK_REQUIRE(!joint || (pre && q2 && kb && ob && cu_b), "ditk_joint_attn: needs both sources and both tables");
+  DITK_REQUIRE(!joint || (((uintptr_t)q2 % 16) == 0 && ((uintptr_t)kb % 16) == 0 && ((uintptr_t)ob % 8) == 0),
                "ditk_joint_attn: misaligned tensor");
   // q and o may be NULL when there are no queries (empty tensors)
   DITK_REQUIRE(k && vt && cu_q && cu_k && (Tq == 0 || (q && o)), "ditk_flash_attn_varlen: null tensor");
@@ -422,16 +450,37 @@ int flash_launch(const void* q, int64_t ldq, const void* k, int64_t ldk, const v
   // next tile's loads hide under the current one's last key tile, as long as
   // the items still fill the CUs at least twice over (512 items at 4 tiles each)
   const int np = (!joint && vt_ld / nseg <= 2048 && (int64_t)((Tq + 255) / 256) * heads >= 2048) ? 4 : 1;
-  const int tiles_bound = ((Tq + 255) / 256 + nseg + np - 1) / np + nseg;
+  // 128-query work items (one 32-query block per wave) when the launch's 256-query
+  // ones would leave CUs idle: an item then takes about kHalfItem of a 256-query
+  // one's time (same key tiles, half the MFMAs; head_dim 64 is bound by its softmax
+  // instructions sooner).  Rounds of items counted as if the segments were equal; the
+  // choice changes no result.  12 heads x 1560 queries and keys of head_dim 128: 46.2
+  // -> 26.5 us, 2 x 1280 37.9 -> 25.3, 2600 69 -> 44, 1560 x 512 19.2 -> 12.6; 24 heads
+  // x 600 of head_dim 64 13.5 -> 10.0, but 2 x 1357 (3 rounds for 2) 43.7 -> 46.8.
+  const float kHalfItem = head_dim == 128 ? 0.57f : 0.72f;
+  auto rounds = [&](int bm) {
+    const int64_t tiles = (int64_t)nseg * (((Tq + nseg - 1) / nseg + bm - 1) / bm);
+    return (float)((tiles * heads + 255) / 256);
+  };
+  const int qb = np == 1 && kHalfItem * rounds(128) < rounds(256) ? 1 : 2;
+  const int bm = 128 * qb;
+  const int tiles_bound = ((Tq + bm - 1) / bm + nseg + np - 1) / np + nseg;
   int64_t nblocks = (int64_t)tiles_bound * heads;
-  nblocks = (nblocks + 8 * kXcdChunk - 1) / (8 * kXcdChunk) * (8 * kXcdChunk);
+  // a launch of less than a round spreads over all XCDs
+  const int chunk = (int)std::min<int64_t>(kXcdChunk, (nblocks + 7) / 8);
+  nblocks = (nblocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
   DITK_REQUIRE(nblocks < (1ll << 31), "ditk_flash_attn_varlen: grid too large");
-  auto kern = joint ? flash_fwd_asm<64, true, true>
-              : head_dim == 128 ? (pre ? flash_fwd_asm<128, true> : flash_fwd_asm<128, false>)
-                                : (pre ? flash_fwd_asm<64, true> : flash_fwd_asm<64, false>);
+  // outputs of 64 MB and more are stored past the caches; smaller ones the next kernel still finds there
+  const bool stream_out = (int64_t)Tq * heads * head_dim * 2 >= (64ll << 20);
+  auto kern = joint ? (qb == 2 ? flash_fwd_asm<64, true, true, 2> : flash_fwd_asm<64, true, true, 1>)
+              : head_dim == 128 ? (pre ? (qb == 2 ? flash_fwd_asm<128, true, false, 2> : flash_fwd_asm<128, true, false, 1>)
+                                       : (qb == 2 ? flash_fwd_asm<128, false, false, 2> : flash_fwd_asm<128, false, false, 1>))
+                                : (pre ? (qb == 2 ? flash_fwd_asm<64, true, false, 2> : flash_fwd_asm<64, true, false, 1>)
+                                       : (qb == 2 ? flash_fwd_asm<64, false, false, 2> : flash_fwd_asm<64, false, false, 1>));
   kern<<<(unsigned)nblocks, 256, 0, stream>>>((const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)vt, vt_ld,
-                                              hs, (bf16_t*)o, ldo, lse, lse_ld, cu_q, cu_k, nseg, heads, np, sl2,
-                                              (const bf16_t*)qb, (const bf16_t*)kb, (bf16_t*)ob, cu_a, cu_b);
+                                              hs, (bf16_t*)o, ldo, lse, lse_ld, cu_q, cu_k, nseg, heads, np, chunk,
+                                              stream_out, sl2, ql, kl, (const bf16_t*)q2, (const bf16_t*)kb,
+                                              (bf16_t*)ob, cu_a, cu_b);
   return ditk_check_launch("ditk_flash_attn_varlen");
 }
 }  // namespace
@@ -443,7 +492,7 @@ DITK_EXPORT int ditk_flash_attn_varlen(const void* q, int64_t ldq, const void* k
                                        int head_dim, float softmax_scale, hipStream_t stream) {
   DITK_REQUIRE(softmax_scale > 0.f, "ditk_flash_attn_varlen: softmax_scale must be > 0");
   return flash_launch(q, ldq, k, ldk, vt, vt_ld, o, ldo, lse, lse_ld, cu_q, cu_k, nseg, Tq, heads, head_dim,
-                      softmax_scale * 1.4426950408889634f, false, stream);
+                      softmax_scale * 1.4426950408889634f, false, RowLayout{head_dim, 0}, RowLayout{head_dim, 0}, stream);
 }
 
 DITK_EXPORT int ditk_flash_attn_varlen_q_prescaled(const void* q, int64_t ldq, const void* k, int64_t ldk,
@@ -452,7 +501,7 @@ DITK_EXPORT int ditk_flash_attn_varlen_q_prescaled(const void* q, int64_t ldq, c
                                                    const int32_t* cu_k, int nseg, int Tq, int heads,
                                                    int head_dim, hipStream_t stream) {
   return flash_launch(q, ldq, k, ldk, vt, vt_ld, o, ldo, lse, lse_ld, cu_q, cu_k, nseg, Tq, heads, head_dim,
-                      1.0f, true, stream);
+                      1.0f, true, RowLayout{head_dim, 0}, RowLayout{head_dim, 0}, stream);
 }
 
 DITK_EXPORT int ditk_joint_attn_q_prescaled(const void* q_a, const void* q_b, int64_t ldq, const void* k_a,
@@ -463,7 +512,34 @@ DITK_EXPORT int ditk_joint_attn_q_prescaled(const void* q_a, const void* q_b, in
   DITK_REQUIRE(head_dim == 64, "ditk_joint_attn_q_prescaled: head_dim must be 64, got %d", head_dim);
   DITK_REQUIRE(cu_a && cu_b, "ditk_joint_attn_q_prescaled: null segment table");
   return flash_launch(q_a, ldq, k_a, ldk, vt, vt_ld, o_a, ldo, nullptr, 0, cu_joint, cu_joint, nseg, T_joint, heads,
-                      head_dim, 1.0f, true, stream, q_b, k_b, o_b, cu_a, cu_b);
+                      head_dim, 1.0f, true, RowLayout{head_dim, 0}, RowLayout{head_dim, 0}, stream, q_b, k_b, o_b, cu_a, cu_b);
+}
+
+// [batch, heads, rows, head_dim] operands read in place: the attention backend's
+// tensors no longer pass through packed copies (three copies of 26 us in all beside
+// 55 us of kernels for 12 x 1560 queries and keys of head_dim 128).
+DITK_EXPORT int ditk_transpose_v_bhsd(const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss, void* vt,
+                                      int64_t vt_ld, int batch, int Sk, int heads, int head_dim,
+                                      const int32_t* cu_k, hipStream_t stream) {
+  DITK_REQUIRE(batch > 0 && Sk >= 0 && (int64_t)batch * Sk < (1ll << 31), "ditk_transpose_v_bhsd: bad sizes");
+  DITK_REQUIRE(v_bs % 8 == 0 && v_hs % 8 == 0, "ditk_transpose_v_bhsd: strides must be multiples of 8");
+  return transpose_launch(v, nullptr, v_ss, vt, vt_ld, batch * Sk, heads, head_dim, cu_k, nullptr, nullptr, batch,
+                          RowLayout{v_hs, v_bs - Sk * v_ss}, stream);
+}
+
+DITK_EXPORT int ditk_flash_attn_bhsd(const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss, const void* k,
+                                     int64_t k_bs, int64_t k_hs, int64_t k_ss, const void* vt, int64_t vt_ld,
+                                     void* o, int64_t ldo, float* lse, int64_t lse_ld, const int32_t* cu_q,
+                                     const int32_t* cu_k, int batch, int Sq, int Sk, int heads, int head_dim,
+                                     float softmax_scale, hipStream_t stream) {
+  DITK_REQUIRE(softmax_scale > 0.f, "ditk_flash_attn_bhsd: softmax_scale must be > 0");
+  DITK_REQUIRE(batch > 0 && Sq >= 0 && Sk >= 0 && (int64_t)batch * Sq < (1ll << 31) &&
+                   (int64_t)batch * Sk < (1ll << 31), "ditk_flash_attn_bhsd: bad sizes");
+  DITK_REQUIRE(q_bs % 8 == 0 && q_hs % 8 == 0 && k_bs % 8 == 0 && k_hs % 8 == 0 && q_ss >= 0 && k_ss >= 0 &&
+                   q_ss < (1ll << 31), "ditk_flash_attn_bhsd: strides must be multiples of 8");
+  return flash_launch(q, q_ss, k, k_ss, vt, vt_ld, o, ldo, lse, lse_ld, cu_q, cu_k, batch, batch * Sq, heads,
+                      head_dim, softmax_scale * 1.4426950408889634f, false, RowLayout{q_hs, q_bs - Sq * q_ss},
+                      RowLayout{k_hs, k_bs - Sk * k_ss}, stream);
 }
 
 // ---------------------------------------------------------------------------

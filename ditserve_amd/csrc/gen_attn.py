@@ -54,11 +54,10 @@ import sys
 # register map (VGPRs: the same for both head dims)
 S_SET = (0, 64)
 P_SET = (128, 160)
-VRING = 6        # Vt fragment ring (read four fragments ahead)
 BN = 64
 
 
-def configure(hd, pre=False, joint=False):
+def configure(hd, pre=False, joint=False, qb=2):
     """Head dim 128 or 64: NC 16-wide chunks of the head dim (K fragments per key
     half), DT 32-row d tiles of O^T, NF Vt fragments per tile (4 key groups x DT),
     ND DMA instructions per wave and operand per tile; AGPRs: O^T, then Q, the K
@@ -79,7 +78,16 @@ def configure(hd, pre=False, joint=False):
     start in two lane-masked rounds (the slotted DMAs of that tile run with an
     empty exec mask).  Q rows are loaded through per-lane 64-bit addresses and
     output rows stored to the source they belong to.  Vt comes in the joint
-    layout.  One query tile per work item."""
+    layout.  One query tile per work item.
+
+    qb: 32-query blocks per wave, 2 or 1 (128-query work items, for launches whose
+    256-query ones would leave CUs idle).  With one block a wave has half the MFMAs
+    per key tile for the same fragment reads, so the reads are issued further ahead
+    (a longer ring, from the registers the second block leaves free).  A query's
+    arithmetic does not depend on it: rescales are decided per block."""
+    global QB, BM, KRING, KA, VRING, VA
+    QB, BM = qb, 128 * qb
+    KRING, KA, VRING, VA = (3, 2, 6, 4) if qb == 2 else (6, 4, 10, 8)
     global HD, NC, DT, NF, ND, KSTAGE_BYTES, VSTAGE_BYTES, O_A, Q_A, KF_A, VF_A, LAST_AGPR
     global PRE, TMP, RING, DTMP, RS0, RS1, NEGM, NEGB, LRUN, KOFF, LAST_VGPR, EPI_T, EPI_L, JOINT
     assert pre or not joint
@@ -100,9 +108,9 @@ def configure(hd, pre=False, joint=False):
     ND = hd // 32
     KSTAGE_BYTES = VSTAGE_BYTES = BN * hd * 2
     O_A = 0
-    Q_A = O_A + 2 * DT * 16
-    KF_A = Q_A + 2 * NC * 4
-    VF_A = KF_A + 3 * 2 * 4
+    Q_A = O_A + QB * DT * 16
+    KF_A = Q_A + QB * NC * 4
+    VF_A = KF_A + KRING * 2 * 4
     LAST_AGPR = VF_A + 4 * VRING - 1
 
 
@@ -117,7 +125,8 @@ S_KT = 66        # s66 tile index kt
 S_NKT1 = 67      # s67 nkt - 1
 S_T0, S_T1 = 68, 69
 S_CMP = 70       # s[70:71] compare mask
-S_EXEC = 72      # s[72:73] saved exec
+S_EXEC = 72      # s[72:73] saved exec (epilogue)
+S_FLAG = 72      # s[72:73] lanes of query block 0 past the rescale threshold (key loop)
 S_VALID = 74     # s74 valid keys of the last tile
 S_THR = 75       # s75 the lazy-rescale threshold 256.0
 S_QOFF = 76      # s76 query-row offset of the current pass (256 per pass)
@@ -258,7 +267,7 @@ class Gen:
 def pair_list(kk):
     """The 16 score pairs of one key half (kk) of a tile for both query blocks,
     in the C++ kernel's order: qb-major, then j, then e."""
-    return [(qb, kk, j, e) for qb in range(2) for j in range(2) for e in range(4)]
+    return [(qb, kk, j, e) for qb in range(QB) for j in range(2) for e in range(4)]
 
 
 def item_order(n):
@@ -391,7 +400,7 @@ def clamp_koff(g, cmp):
 def k_read(g, chunk, kk, stage):
     """ds_read of K fragment (chunk, kk) of K stage `stage`."""
     off = stage * KSTAGE_BYTES + (chunk >> 2) * 8192 + kk * 4096
-    g(f"ds_read_b128 {ar(kf_reg(chunk % 3, kk), 4)}, %[kaddr{chunk & 3}] offset:{off}")
+    g(f"ds_read_b128 {ar(kf_reg(chunk % KRING, kk), 4)}, %[kaddr{chunk & 3}] offset:{off}")
     g.lds_issue(("k", chunk, kk))
 
 
@@ -408,7 +417,7 @@ def mfma_s(g, s_set, qb, kk, chunk, first=False):
         src_c = vr(dst, 16)
     else:
         src_c = vr(negm(qb), 16) if PRE and not first else "0"
-    g(f"v_mfma_f32_32x32x16_bf16 {vr(dst, 16)}, {ar(kf_reg(chunk % 3, kk), 4)}, {ar(q_reg(qb, chunk), 4)}, {src_c}")
+    g(f"v_mfma_f32_32x32x16_bf16 {vr(dst, 16)}, {ar(kf_reg(chunk % KRING, kk), 4)}, {ar(q_reg(qb, chunk), 4)}, {src_c}")
 
 
 def mfma_o(g, p_set, qb, d, grp, ring):
@@ -426,16 +435,16 @@ def s_phase(g, s_set, kstage, vstage=None, items=None, dma=None, first=False):
     for c in range(NC):
         g.lds_wait(("k", c, 1))
         for kk in range(2):
-            for qb in range(2):
+            for qb in range(QB):
                 d = dma[slot] if dma is not None and slot < len(dma) else None
                 if d:
                     d[0]()
                 mfma_s(g, s_set, qb, kk, c, first)
-                if kk == 0 and qb == 0 and c + 2 < NC:
-                    k_read(g, c + 2, 0, kstage)
-                    k_read(g, c + 2, 1, kstage)
+                if kk == 0 and qb == 0 and c + KA < NC:
+                    k_read(g, c + KA, 0, kstage)
+                    k_read(g, c + KA, 1, kstage)
                 if kk == 0 and qb == 0 and c == NC - 1 and vstage is not None:
-                    for f in range(4):
+                    for f in range(VA):
                         v_read(g, f, vstage)
                 if d:
                     d[1]()
@@ -450,12 +459,12 @@ def o_phase(g, p_set, vstage, items=None):
     slot = 0
     for f in range(NF):
         grp, d = f // DT, f % DT
-        for qb in range(2):
+        for qb in range(QB):
             if qb == 0 and f % 2 == 0:
                 g.lds_wait(("v", f + 1))
             mfma_o(g, p_set, qb, d, grp, f % VRING)
-            if qb == 0 and f + 4 < NF:
-                v_read(g, f + 4, vstage)
+            if qb == 0 and f + VA < NF:
+                v_read(g, f + VA, vstage)
             if items is not None:
                 items[slot]()
             slot += 1
@@ -532,14 +541,31 @@ def softmax_tile(g, s_set, p_set, qb, kks, rs_dst, masked=False):
                 g(f"v_add_f32 {vr(rs_dst + qb)}, {vr(rs_dst + qb)}, {vr(t0)}")
 
 
+def flag_blocks(g, rsum):
+    """The lanes of each query block whose row sum (VGPRs rsum + qb) is above 256 or
+    non-finite: S_FLAG (block 0), S_CMP (block 1); vcc = either, for the branch."""
+    if QB == 1:
+        g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(rsum)}")
+        return
+    g(f"v_cmp_nge_f32_e64 {sp(S_FLAG)}, {s_(S_THR)}, {vr(rsum)}")
+    g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(rsum + 1)}")
+    g(f"s_or_b64 vcc, {sp(S_FLAG)}, {sp(S_CMP)}")
+
+
 def exact_rescale(g, s_set, p_set, kks, masked=False, live_next=None):
     """The C++ rescale: m_new = max(m, row max of the tile's scores), O and l
     scaled by exp2(m - m_new), P of the tile recomputed against m_new into rs0.
     (rs1 is cleared.)  Pre: the scores are relative to m_old, so m_new = max(m_old,
     row max + m_old); the tile's S and the next tile's (S set live_next, started
-    from the old -m block) move by -(m_new - m_old) and the block becomes -m_new."""
+    from the old -m block) move by -(m_new - m_old) and the block becomes -m_new.
+    A query block without a flagged lane (flag_blocks) keeps its m, P and sums, so
+    that its results do not depend on the blocks its wave holds beside it."""
     g.nops(20)  # O accumulators read below: MFMA results must have landed
-    for qb in range(2):
+    for qb in range(QB):
+        keep = g.new_label("keep")
+        if QB == 2:
+            g(f"s_cmp_eq_u64 {sp((S_FLAG, S_CMP)[qb])}, 0")
+            g(f"s_cbranch_scc1 {keep}")
         mx, tmp, alpha = DTMP + 1, DTMP + 2, DTMP + 3
         row_max_to(g, s_set, qb, mx, tmp, alpha)
         if PRE:
@@ -571,6 +597,7 @@ def exact_rescale(g, s_set, p_set, kks, masked=False, live_next=None):
         g(f"v_mov_b32 {vr(RS0 + qb)}, 0")
         g(f"v_mov_b32 {vr(RS1 + qb)}, 0")
         softmax_tile(g, s_set, p_set, qb, kks, RS0, masked)
+        g.label(keep)
     g.nops(5 if PRE else 3)  # v_accvgpr_write (and the -m block writes) -> MFMA srcC
 
 
@@ -586,7 +613,7 @@ def tile(g, a):
     b = 1 - a
     after_check = g.new_label("checked")
     resc = g.new_label("rescale")
-    g.lds = [("k", 0, 0), ("k", 0, 1), ("k", 1, 0), ("k", 1, 1)]
+    g.lds = [("k", c, kk) for c in range(KA) for kk in range(2)]
     # K DMA source of tile min(kt+2, nkt-1); the last tile's rows past the end clamp
     g(f"s_add_u32 {s_(S_T0)}, {s_(S_KT)}, 2")
     g(f"s_min_u32 {s_(S_T0)}, {s_(S_T0)}, {s_(S_NKT1)}")
@@ -615,23 +642,22 @@ def tile(g, a):
     dmas = ([(lambda i=i: kdma_m0(g, i, a), lambda i=i: kdma_go(g, i)) for i in range(ND)] +
             [(lambda i=i: vdma_m0(g, i, b), lambda i=i: vdma_go(g, i)) for i in range(ND)])
     # phase 1: S(kt+1) into set b || P(kt) keys 32..63 from set a
-    items = make_items(g, pair_list(1), a, a, RS1, slots=4 * NC)
+    items = make_items(g, pair_list(1), a, a, RS1, slots=2 * QB * NC)
     s_phase(g, b, kstage=b, vstage=a, items=items, dma=dmas)
     # lazy-rescale check on tile kt: rsum = rs0 + rs1 (per lane), flag !(rsum <= 256)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
-    g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(DTMP)}")
-    g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(DTMP + 1)}")
-    g(f"s_or_b64 vcc, vcc, {sp(S_CMP)}")
+    flag_blocks(g, DTMP)
     g(f"s_cbranch_vccnz {resc}")
     g.label(after_check)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(LRUN + qb)}, {vr(LRUN + qb)}, {vr(DTMP + qb)}")
     # phase 2: O += Vt(kt) P(kt) || P(kt+1) keys 0..31 from set b.  The wait
     # covers the VALU reads of the S(kt+1) results of the last MFMAs (already
     # three MFMAs old) and the MFMA reads of the P(kt) just packed.
-    g.nops(2)
-    items = make_items(g, pair_list(0), b, b, RS0, slots=2 * NF)
+    # (one query block: one MFMA old, so the wait is the whole one)
+    g.nops(2 if QB == 2 else 10)
+    items = make_items(g, pair_list(0), b, b, RS0, slots=QB * NF)
     o_phase(g, a, vstage=a, items=items)
     # publish this tile's DMA: own loads landed, then the workgroup barrier
     g("s_waitcnt vmcnt(0)")
@@ -640,7 +666,7 @@ def tile(g, a):
     g(f"s_addc_u32 {s_(S_VDMA + 1)}, {s_(S_VDMA + 1)}, 0")
     g(f"s_add_u32 {s_(S_KT)}, {s_(S_KT)}, 1")
     # the next tile's first K reads: K(kt+2), in stage a
-    for c in range(2):
+    for c in range(KA):
         k_read(g, c, 0, a)
         k_read(g, c, 1, a)
     return resc, after_check
@@ -651,7 +677,7 @@ def rescale_block(g, a, resc, back):
     returns with the tile's row sums in DTMP like the common path."""
     g.label(resc)
     exact_rescale(g, a, a, (0, 1), live_next=1 - a)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
     g(f"s_branch {back}")
 
@@ -662,9 +688,9 @@ def last_tile_prefetch(g, a, nopf):
     g(f"s_cmp_gt_u32 {s_(S_NPASS)}, 1")
     g(f"s_cbranch_scc0 {nopf}")
     tmp = S_SET[1 - a]  # S set of the next tile: free in the last tile
-    g(f"s_add_u32 {s_(S_T0)}, {s_(S_QOFF)}, {BN * 4}")
+    g(f"s_add_u32 {s_(S_T0)}, {s_(S_QOFF)}, {BM}")
     g(f"s_sub_u32 {s_(S_T1)}, %[qend], 1")
-    for qb in range(2):
+    for qb in range(QB):
         ad = tmp + 4 * qb  # even: the address pair, then the row and a temporary
         qrow = opnd(g, f"qrow{qb}", ad + 2)
         g(f"v_add_u32 {vr(ad + 2)}, {s_(S_T0)}, {qrow}")
@@ -707,34 +733,30 @@ def last_tile(g, a):
     g(f"s_cbranch_scc1 {recompute}")
     for it in make_items(g, pair_list(1), a, a, RS1):
         it()
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
-    g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(DTMP)}")
-    g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(DTMP + 1)}")
-    g(f"s_or_b64 vcc, vcc, {sp(S_CMP)}")
+    flag_blocks(g, DTMP)
     g(f"s_cbranch_vccz {reuse_back}")
     exact_rescale(g, a, a, (0, 1))
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
     g.label(reuse_back)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(LRUN + qb)}, {vr(LRUN + qb)}, {vr(DTMP + qb)}")
     g(f"s_branch {common}")
     g.label(recompute)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_mov_b32 {vr(RS0 + qb)}, 0")
     g(f"s_cmp_eq_u32 {s_(S_VALID)}, {BN}")
     g(f"s_cbranch_scc1 {full}")
-    for qb in range(2):
+    for qb in range(QB):
         softmax_tile(g, a, a, qb, (0, 1), RS0, masked=True)
     g(f"s_branch {done_rs}")
     g.label(full)
-    for qb in range(2):
+    for qb in range(QB):
         softmax_tile(g, a, a, qb, (0, 1), RS0, masked=False)
     g.label(done_rs)
-    g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(RS0)}")
-    g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(RS0 + 1)}")
-    g(f"s_or_b64 vcc, vcc, {sp(S_CMP)}")
+    flag_blocks(g, RS0)
     g(f"s_cbranch_vccz {checked}")
     # rescale against the exact tile max (masked sums)
     g(f"s_cmp_eq_u32 {s_(S_VALID)}, {BN}")
@@ -744,11 +766,11 @@ def last_tile(g, a):
     g.label(resc)
     exact_rescale(g, a, a, (0, 1), masked=False)
     g.label(checked)
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_add_f32 {vr(LRUN + qb)}, {vr(LRUN + qb)}, {vr(RS0 + qb)}")
     g.label(common)
     g("s_nop 2")
-    for f in range(4):
+    for f in range(VA):
         v_read(g, f, a)
     o_phase(g, a, vstage=a, items=None)
     # another pass: its loads landed and published, this tile's Vt reads done
@@ -820,7 +842,7 @@ def prologue(g, empty):
     # before the first wait so that their latencies overlap
     if PRE:
         g("s_nop 4")  # the AGPR operands were written just before the body
-    for qb in range(2):
+    for qb in range(QB):
         if JOINT:  # per-lane 64-bit row address in its source
             qa = S_SET[0] + 2 * qb
             g(f"v_accvgpr_read_b32 {vr(qa)}, %[qa{qb}lo]")
@@ -847,9 +869,9 @@ def prologue(g, empty):
 
 def clear_state(g):
     """O = 0, l = 0, row sums 0, tile 0."""
-    for i in range(2 * DT * 16):
+    for i in range(QB * DT * 16):
         g(f"v_accvgpr_write_b32 {ar(O_A + i)}, 0")
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_mov_b32 {vr(LRUN + qb)}, 0")
         g(f"v_mov_b32 {vr(RS0 + qb)}, 0")
         g(f"v_mov_b32 {vr(RS1 + qb)}, 0")
@@ -861,13 +883,13 @@ def pass_start(g):
     0, then the wait for K(1) and Vt(0)."""
     # S(0) = K(0) Q^T into set A
     g.lds = []
-    for c in range(2):
+    for c in range(KA):
         k_read(g, c, 0, 0)
         k_read(g, c, 1, 0)
     s_phase(g, 0, kstage=0, first=True)
     g.nops(20)
     # m = exact max of tile 0 (pre: S(0) -= m, and the -m blocks)
-    for qb in range(2):
+    for qb in range(QB):
         row_max_to(g, 0, qb, DTMP + 1, DTMP + 2, DTMP + 3)
         if PRE:
             for kk in range(2):
@@ -883,7 +905,7 @@ def pass_start(g):
     g("s_barrier")
     # tile 0 reads K(1) from K stage 1; its first reads are issued here
     g.lds = []
-    for c in range(2):
+    for c in range(KA):
         k_read(g, c, 0, 1)
         k_read(g, c, 1, 1)
 
@@ -895,8 +917,8 @@ def epilogue(g, negm_of=None):
     Each 32-query block goes through this wave's LDS staging rows (pitch HD * 2 +
     8 bytes, query q at row q) so that the global stores write whole row
     segments: a lane owns 4 consecutive dims of one query in the accumulators,
-    but stores 16 bytes of one row, HD / 8 lanes per row.  The stores are
-    non-temporal: nothing in the kernel reads the output again."""
+    but stores 16 bytes of one row, HD / 8 lanes per row.  %[ont] says whether
+    the stores are non-temporal: nothing in the kernel reads the output again."""
     g.nops(20)
     T = EPI_T
     # temporaries from register EB on: S set B past the EPI registers (dead in
@@ -923,7 +945,7 @@ def epilogue(g, negm_of=None):
     g(f"v_lshl_add_u32 {vr(ra)}, {vr(t0)}, 4, {vr(ra)}")
     g(f"v_add_u32 {vr(ra)}, %[lds_o], {vr(ra)}")
     g(f"s_lshl_b32 {s_(S_T1)}, %[ldob], {rpr.bit_length() - 1}")   # rpr rows of output
-    for qb in range(2):
+    for qb in range(QB):
         lt, inv, t = EPI_L + 0, EPI_L + 1, EPI_L + 2
         xa = xaddr_to(g, EPI_L + 3, lane)
         qrow = vr(EB + 51)  # this lane's query row in this pass
@@ -994,24 +1016,32 @@ def epilogue(g, negm_of=None):
             g(f"v_addc_co_u32 {vr(addr + 1)}, vcc, 0, {vr(addr + 1)}, vcc")
         g("s_waitcnt lgkmcnt(0)")
         g(f"s_mov_b64 {sp(S_EXEC)}, exec")
-        for i in range(32 // rpr):
-            if JOINT:
-                if i:
+        plain, stored = g.new_label("plainst"), g.new_label("stored")
+        g("s_cmp_eq_u32 %[ont], 0")
+        g(f"s_cbranch_scc1 {plain}")
+        for nt in (" nt", ""):         # streamed past the caches, or left in them
+            if not nt:
+                g(f"s_branch {stored}")
+                g.label(plain)
+            for i in range(32 // rpr):
+                if JOINT:
+                    if i:
+                        g(f"s_mov_b64 exec, {sp(S_EXEC)}")
+                        g(f"v_add_u32 {vr(j0)}, {rpr}, {vr(j0)}")
+                    g(f"v_mad_u64_u32 {vr(addr, 2)}, {sp(S_CMP)}, {vr(j0)}, %[ldob], 0")
+                    g(f"v_cmp_gt_i32 vcc, %[lena], {vr(j0)}")
+                    g(f"v_cndmask_b32 {vr(EB + 57)}, {vr(tb)}, {vr(ib)}, vcc")
+                    g(f"v_cndmask_b32 {vr(EB + 58)}, {vr(tb + 1)}, {vr(ib + 1)}, vcc")
+                    g(f"v_add_co_u32 {vr(addr)}, vcc, {vr(EB + 57)}, {vr(addr)}")
+                    g(f"v_addc_co_u32 {vr(addr + 1)}, vcc, {vr(EB + 58)}, {vr(addr + 1)}, vcc")
+                elif i:
                     g(f"s_mov_b64 exec, {sp(S_EXEC)}")
-                    g(f"v_add_u32 {vr(j0)}, {rpr}, {vr(j0)}")
-                g(f"v_mad_u64_u32 {vr(addr, 2)}, {sp(S_CMP)}, {vr(j0)}, %[ldob], 0")
-                g(f"v_cmp_gt_i32 vcc, %[lena], {vr(j0)}")
-                g(f"v_cndmask_b32 {vr(EB + 57)}, {vr(tb)}, {vr(ib)}, vcc")
-                g(f"v_cndmask_b32 {vr(EB + 58)}, {vr(tb + 1)}, {vr(ib + 1)}, vcc")
-                g(f"v_add_co_u32 {vr(addr)}, vcc, {vr(EB + 57)}, {vr(addr)}")
-                g(f"v_addc_co_u32 {vr(addr + 1)}, vcc, {vr(EB + 58)}, {vr(addr + 1)}, vcc")
-            elif i:
-                g(f"s_mov_b64 exec, {sp(S_EXEC)}")
-                g(f"v_add_co_u32 {vr(addr)}, vcc, {s_(S_T1)}, {vr(addr)}")
-                g(f"v_addc_co_u32 {vr(addr + 1)}, vcc, 0, {vr(addr + 1)}, vcc")
-            g(f"v_cmp_lt_i32 vcc, {i * rpr}, {vr(left)}")
-            g("s_and_b64 exec, exec, vcc")
-            g(f"global_store_dwordx4 {vr(addr, 2)}, {vr(data + 4 * i, 4)}, off nt")  # streamed
+                    g(f"v_add_co_u32 {vr(addr)}, vcc, {s_(S_T1)}, {vr(addr)}")
+                    g(f"v_addc_co_u32 {vr(addr + 1)}, vcc, 0, {vr(addr + 1)}, vcc")
+                g(f"v_cmp_lt_i32 vcc, {i * rpr}, {vr(left)}")
+                g("s_and_b64 exec, exec, vcc")
+                g(f"global_store_dwordx4 {vr(addr, 2)}, {vr(data + 4 * i, 4)}, off{nt}")
+        g.label(stored)
         g(f"s_mov_b64 exec, {sp(S_EXEC)}")
         # lse = (m + log2 l) * ln 2 for lanes of the first half-wave, when asked
         skip = g.new_label("nolse")
@@ -1076,26 +1106,27 @@ def generate():
     g(f"s_sub_u32 {s_(S_NPASS)}, {s_(S_NPASS)}, 1")
     g(f"s_cmp_eq_u32 {s_(S_NPASS)}, 0")
     g(f"s_cbranch_scc1 {done}")
-    g(f"s_add_u32 {s_(S_QOFF)}, {s_(S_QOFF)}, {BN * 4}")
+    g(f"s_add_u32 {s_(S_QOFF)}, {s_(S_QOFF)}, {BM}")
     clear_state(g)
     g(f"s_branch {npass}")
     # no keys: every pass stores zero rows
     g.label(empty)
-    for i in range(2 * DT * 16):
+    for i in range(QB * DT * 16):
         g(f"v_accvgpr_write_b32 {ar(O_A + i)}, 0")
-    for qb in range(2):
+    for qb in range(QB):
         g(f"v_mov_b32 {vr(LRUN + qb)}, 0")
     epilogue(g)
     g(f"s_sub_u32 {s_(S_NPASS)}, {s_(S_NPASS)}, 1")
     g(f"s_cmp_eq_u32 {s_(S_NPASS)}, 0")
     g(f"s_cbranch_scc1 {done}")
-    g(f"s_add_u32 {s_(S_QOFF)}, {s_(S_QOFF)}, {BN * 4}")
+    g(f"s_add_u32 {s_(S_QOFF)}, {s_(S_QOFF)}, {BM}")
     g(f"s_branch {empty}")
     g.label(done)
     return g.lines
 
 
 def clobbers(hd, pre=False, joint=False):
+    """One header for both block counts: the two-block body owns more registers."""
     configure(hd, pre, joint)
     regs = ([f"v{i}" for i in range(LAST_VGPR + 1)] + [f"a{i}" for i in range(LAST_AGPR + 1)] +
             [f"s{i}" for i in (SGPRS_JOINT if joint else SGPRS)])
@@ -1105,12 +1136,12 @@ def clobbers(hd, pre=False, joint=False):
             f"#define DITK_D{name.upper()}_CLOBBERS \\\n" + "".join(f"  {r}, \\\n" for r in rows) + "\n")
 
 
-def write_body(path, hd, pre=False, joint=False):
-    configure(hd, pre, joint)
+def write_body(path, hd, pre=False, joint=False, qb=2):
+    configure(hd, pre, joint, qb)
     lines = generate()
     with open(path, "w") as f:
         f.write(f"// Generated by gen_attn.py -- the instruction body of flash_fwd_asm<{hd}, {str(pre).lower()}, "
-                f"{str(joint).lower()}>.\n")
+                f"{str(joint).lower()}, {qb}>.\n")
         for line in lines:
             esc = line.replace("\\", "\\\\").replace('"', '\\"')
             f.write(f'"{esc}\\n"\n')
@@ -1122,7 +1153,8 @@ def main(argv):
     for hd, pre, joint in ((128, False, False), (128, True, False), (64, False, False), (64, True, False),
                            (64, True, True)):
         name = f"d{hd}{'j' if joint else 'p' if pre else ''}"
-        write_body(os.path.join(out, f"attn_{name}_body.inc"), hd, pre, joint)
+        for qb in (2, 1):
+            write_body(os.path.join(out, f"attn_{name}{'' if qb == 2 else 'q1'}_body.inc"), hd, pre, joint, qb)
         with open(os.path.join(out, f"attn_{name}_clobbers.h"), "w") as f:
             f.write(clobbers(hd, pre, joint))
     return 0

@@ -626,6 +626,40 @@ def flash_attn_varlen(q, k, v, seg_q, seg_k, heads, head_dim, softmax_scale=None
     return (out, lse) if return_lse else out
 
 
+def flash_attn_bhsd(q, k, v, softmax_scale=None):
+    """Attention over q [B, H, Sq, D], k / v [B, H, Sk, D] bf16 of any strides, read in
+    place where they are kernel-addressable (unit stride along D, the others
+    multiples of 8, 16-byte aligned), else from a contiguous copy.  Returns out
+    [B * Sq, H * D] and lse [H, B * Sq] fp32, as flash_attn_varlen does for B
+    equal segments."""
+    for t, name in ((q, "q"), (k, "k"), (v, "v")):
+        _check(t, name, _BF16, 4)
+    B, H, Sq, D = q.shape
+    Sk = k.shape[2]
+    if k.shape != (B, H, Sk, D) or v.shape != k.shape:
+        raise ValueError(f"k and v must be [{B}, {H}, Sk, {D}], got {tuple(k.shape)} and {tuple(v.shape)}")
+    # (a clone: contiguous() keeps the odd strides that dimensions of size 1 may have)
+    q, k, v = (t if _bhsd_in_place(t) else t.clone(memory_format=torch.contiguous_format) for t in (q, k, v))
+    seg_q, seg_k = Segments.uniform(B, Sq, q.device), Segments.uniform(B, Sk, q.device)
+    cols = vt_columns(B * Sk, B)
+    vt = torch.empty((H, D, cols), dtype=_BF16, device=q.device)
+    (qb, qh, qs, _), (kb, kh, ks, _), (vb, vh, vs, _) = q.stride(), k.stride(), v.stride()
+    stream = _stream()
+    _lib.call("ditk_transpose_v_bhsd", _ptr(v), vb, vh, vs, _ptr(vt), cols, B, Sk, H, D, _ptr(seg_k.dev), stream)
+    out = torch.empty((B * Sq, H * D), dtype=_BF16, device=q.device)
+    lse = torch.empty((H, B * Sq), dtype=torch.float32, device=q.device)
+    scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
+    # with no keys at all no K tile is read: any valid address stands in for the empty K
+    _lib.call("ditk_flash_attn_bhsd", _ptr(q), qb, qh, qs, _ptr(k) if Sk else _ptr(vt), kb, kh, ks, _ptr(vt), cols,
+              _ptr(out), H * D, _ptr(lse), B * Sq, _ptr(seg_q.dev), _ptr(seg_k.dev), B, Sq, Sk, H, D, scale, stream)
+    return out, lse
+
+
+def _bhsd_in_place(t):
+    b, h, s, d = t.stride()
+    return d == 1 and not (b % 8 or h % 8 or s % 8 or t.data_ptr() % 16) and s < 1 << 23
+
+
 # ---------------------------------------------------------------------------
 # prelude / epilogue glue
 # ---------------------------------------------------------------------------

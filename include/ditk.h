@@ -195,6 +195,23 @@ int ditk_flash_attn_varlen(const void* q, int64_t ldq, const void* k, int64_t ld
                            ditk_stream_t stream);
 
 /*
+ * ditk_transpose_v and ditk_flash_attn_varlen over [batch, heads, rows, head_dim]
+ * operands read in place: strides in elements (bs between batches, hs between heads,
+ * ss between rows; multiples of 8, unit stride along head_dim), batch b being
+ * segment b of Sq queries and Sk keys (cu_q = [0, Sq, 2 Sq, ...], cu_k likewise).
+ * The output stays packed: o [batch * Sq, heads * head_dim] with row stride ldo, lse
+ * [heads][lse_ld].  Results are those of the packed calls.
+ * Replaces: the attention backend call Spec.run on BHSD tensors —
+ *   workers/xfuser/core/attention/spec.py:283-304.
+ */
+int ditk_transpose_v_bhsd(const void* v, int64_t v_bs, int64_t v_hs, int64_t v_ss, void* vt, int64_t vt_ld, int batch,
+                          int Sk, int heads, int head_dim, const int32_t* cu_k, ditk_stream_t stream);
+int ditk_flash_attn_bhsd(const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss, const void* k, int64_t k_bs,
+                         int64_t k_hs, int64_t k_ss, const void* vt, int64_t vt_ld, void* o, int64_t ldo, float* lse,
+                         int64_t lse_ld, const int32_t* cu_q, const int32_t* cu_k, int batch, int Sq, int Sk,
+                         int heads, int head_dim, float softmax_scale, ditk_stream_t stream);
+
+/*
  * ditk_flash_attn_varlen with q already multiplied by softmax_scale * log2(e)
  * (head_dim 64 or 128).  A producer that folds that factor into its QK-norm
  * weight still rounds q to bf16 once, and the kernel then starts its score
