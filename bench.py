@@ -336,7 +336,8 @@ def _wan_kernel_spec(cfg, seqs, text_len):
         "attn_cross": ("mfma", 4.0 * M * text_len * D, f"cross-attention over {text_len} text keys per segment"),
         "gemm_qkv": ("mfma", 2.0 * M * 3 * D * D, f"fused QKV projection {M}x{3 * D}x{D}, bias"),
         "gemm_o_gate": ("mfma", 2.0 * M * D * D, f"self-attention output projection {M}x{D}x{D}, gated residual"),
-        "gemm_cross_q": ("mfma", 2.0 * M * D * D, f"cross-attention q projection {M}x{D}x{D}, bias"),
+        "gemm_cross_qkv": ("mfma", 2.0 * (M + 2 * text_len * len(seqs)) * D * D,
+                           f"cross-attention q {M}x{D}x{D} and text K/V {text_len * len(seqs)}x{2 * D}x{D}, bias"),
         "gemm_o_res": ("mfma", 2.0 * M * D * D, f"cross-attention output projection {M}x{D}x{D}, residual"),
         "gemm_ffn_up_gelu": ("mfma", 2.0 * M * F * D, f"FFN up {M}x{F}x{D}, GELU-tanh"),
         "gemm_ffn_down_gate": ("mfma", 2.0 * M * D * F, f"FFN down {M}x{D}x{F}, gated residual"),
@@ -354,8 +355,7 @@ def _sd35_kernel_spec(cfg, img_counts, txt_counts):
     return {
         "attn_joint": ("mfma", 4.0 * joint * D, "joint image+text attention, head_dim 64"),
         "attn_dual_core": ("mfma", 4.0 * sum(n * n for n in img_counts) * D, "dual image-only attention, head_dim 64"),
-        "gemm_qkv_img": ("mfma", 2.0 * Mi * 3 * D * D, f"image QKV {Mi}x{3 * D}x{D}, bias"),
-        "gemm_qkv_txt": ("mfma", 2.0 * Mt * 3 * D * D, f"text QKV {Mt}x{3 * D}x{D}, bias"),
+        "gemm_qkv_pair": ("mfma", 2.0 * (Mi + Mt) * 3 * D * D, f"image + text QKV {Mi} + {Mt} x {3 * D} x {D}, bias"),
         "gemm_out_pair": ("mfma", 2.0 * (Mi + Mt) * D * D,
                           f"image + text output projections ({Mi} + {Mt})x{D}x{D}, gated residual, one pair call"),
         "gemm_ffn_up_img": ("mfma", 2.0 * Mi * F * D, f"image FFN up {Mi}x{F}x{D}, GELU-tanh"),

@@ -488,34 +488,33 @@ struct L4Prob {
   const float* gate;
   int64_t gate_stride;
   const int32_t* cu;
-  int nseg, M, tiles_m, group_m;
+  int nseg, M, N, tiles_m, tiles_n, group_m;
 };
 
-// Two products of the same N, K and epilogue (their own inputs, weights, bias,
-// residual, gate and segments) in one persistent launch: the tile list is the
+// Two products of the same K and epilogue (their own inputs, features, weights,
+// bias, residual, gate and segments) in one persistent launch: the tile list is the
 // first product's tiles, then the second's, taken per XCD as gemm_kernel_l4
 // takes one product's.  Each tile is computed exactly as a launch of its own
 // product would compute it.
 template <int EPI, int FI, int FJ>
-__global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob p1, int N, int K, int tiles_n,
-                                                           bool prefetch, bool stream_out) {
+__global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob p1, int K, bool prefetch, bool stream_out) {
   __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   const int nb = gridDim.x, b = blockIdx.x;
-  const int t0 = p0.tiles_m * tiles_n, ntiles = t0 + p1.tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
+  const int t0 = p0.tiles_m * p0.tiles_n, ntiles = t0 + p1.tiles_m * p1.tiles_n, per_xcd = (ntiles + 7) / 8;
   const int tlo = (b & 7) * per_xcd, thi = min(tlo + per_xcd, ntiles);
   // Workgroups in the order of their first tiles: the first c0 start in product 0
   // and prefetch its weights, the others product 1's.
   const int wpx = nb >> 3, x0 = t0 / per_xcd, rank = (b & 7) * wpx + (b >> 3);
   const int c0 = min(nb, x0 * wpx + min(t0 - x0 * per_xcd, wpx));
-  L4Prefetch pf = rank < c0 ? l4_prefetch(rank, c0, N, K, prefetch)
-                            : l4_prefetch(rank - c0, nb - c0, N, K, prefetch);
+  L4Prefetch pf = rank < c0 ? l4_prefetch(rank, c0, p0.N, K, prefetch)
+                            : l4_prefetch(rank - c0, nb - c0, p1.N, K, prefetch);
   for (int L = tlo + (b >> 3); L < thi; L += nb >> 3) {
     const bool s = L >= t0;  // wave-uniform: the fields below are scalar selects
     l4_tile<EPI, FI, FJ>(lds, s ? L - t0 : L, s ? p1.A : p0.A, s ? p1.lda : p0.lda, s ? p1.W : p0.W,
                      s ? p1.ldw : p0.ldw, s ? p1.bias : p0.bias, s ? p1.C : p0.C, s ? p1.ldc : p0.ldc,
-                     s ? p1.M : p0.M, N, K, s ? p1.R : p0.R, s ? p1.ldr : p0.ldr, s ? p1.gate : p0.gate,
+                     s ? p1.M : p0.M, s ? p1.N : p0.N, K, s ? p1.R : p0.R, s ? p1.ldr : p0.ldr, s ? p1.gate : p0.gate,
                      s ? p1.gate_stride : p0.gate_stride, s ? p1.cu : p0.cu, s ? p1.nseg : p0.nseg,
-                     s ? p1.tiles_m : p0.tiles_m, tiles_n, s ? p1.group_m : p0.group_m, pf,
+                     s ? p1.tiles_m : p0.tiles_m, s ? p1.tiles_n : p0.tiles_n, s ? p1.group_m : p0.group_m, pf,
                          stream_out);
     pf.n = 0;
   }
@@ -792,18 +791,18 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
 }
 
 template <int EPI, int FI, int FJ>
-int launch_l4_pair(L4Prob p0, L4Prob p1, int N, int K, hipStream_t stream) {
+int launch_l4_pair(L4Prob p0, L4Prob p1, int K, hipStream_t stream) {
   constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
-  const int tiles_n = (N + GBN - 1) / GBN;
-  p0.tiles_m = (p0.M + GBM - 1) / GBM;
-  p1.tiles_m = (p1.M + GBM - 1) / GBM;
-  p0.group_m = l4_group_m(p0.tiles_m, tiles_n, GBM, GBN, K);
-  p1.group_m = l4_group_m(p1.tiles_m, tiles_n, GBM, GBN, K);
-  const int64_t tiles = (int64_t)(p0.tiles_m + p1.tiles_m) * tiles_n;
+  for (L4Prob* p : {&p0, &p1}) {
+    p->tiles_m = (p->M + GBM - 1) / GBM;
+    p->tiles_n = (p->N + GBN - 1) / GBN;
+    p->group_m = l4_group_m(p->tiles_m, p->tiles_n, GBM, GBN, K);
+  }
+  const int64_t tiles = (int64_t)p0.tiles_m * p0.tiles_n + (int64_t)p1.tiles_m * p1.tiles_n;
   const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
   gemm_kernel_l4_pair<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
-      p0, p1, N, K, tiles_n, l4_prefetch_on(p0.M, N, K, p0.ldw, GBM) && (int64_t)N * p1.ldw * 2 < (1ll << 31),
-      l4_stream_out(p0.M + (int64_t)p1.M, N));
+      p0, p1, K, l4_prefetch_on(p0.M, p0.N, K, p0.ldw, GBM) && (int64_t)p1.N * p1.ldw * 2 < (1ll << 31),
+      l4_stream_out((int64_t)p0.M * p0.N + (int64_t)p1.M * p1.N, 1));
   return ditk_check_launch("ditk_gemm_pair");
 }
 
@@ -838,14 +837,14 @@ int launch_l4_cfg(int cfg, const void* A, int64_t lda, const void* W, int64_t ld
 }
 
 template <int EPI>
-int launch_l4_pair_cfg(int cfg, const L4Prob& p0, const L4Prob& p1, int N, int K, hipStream_t stream) {
+int launch_l4_pair_cfg(int cfg, const L4Prob& p0, const L4Prob& p1, int K, hipStream_t stream) {
   switch (cfg) {
-    case 0: return launch_l4_pair<EPI, 8, 8>(p0, p1, N, K, stream);
-    case 1: return launch_l4_pair<EPI, 6, 8>(p0, p1, N, K, stream);
-    case 2: return launch_l4_pair<EPI, 8, 4>(p0, p1, N, K, stream);
-    case 3: return launch_l4_pair<EPI, 6, 4>(p0, p1, N, K, stream);
-    case 4: return launch_l4_pair<EPI, 4, 4>(p0, p1, N, K, stream);
-    default: return launch_l4_pair<EPI, 3, 4>(p0, p1, N, K, stream);
+    case 0: return launch_l4_pair<EPI, 8, 8>(p0, p1, K, stream);
+    case 1: return launch_l4_pair<EPI, 6, 8>(p0, p1, K, stream);
+    case 2: return launch_l4_pair<EPI, 8, 4>(p0, p1, K, stream);
+    case 3: return launch_l4_pair<EPI, 6, 4>(p0, p1, K, stream);
+    case 4: return launch_l4_pair<EPI, 4, 4>(p0, p1, K, stream);
+    default: return launch_l4_pair<EPI, 3, 4>(p0, p1, K, stream);
   }
 }
 
@@ -987,17 +986,17 @@ DITK_EXPORT int ditk_gemm(const void* A, int64_t lda, const void* W, int64_t ldw
                   stream);
 }
 
-DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0,
+DITK_EXPORT int ditk_gemm_pair_n(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0,
                                void* C0, int64_t ldc0, int M0, const void* R0, int64_t ldr0, const float* gate0,
                                int64_t gate_stride0, const int32_t* cu_seqlens0, int nseg0, const void* A1,
                                int64_t lda1, const void* W1, int64_t ldw1, const float* bias1, void* C1,
                                int64_t ldc1, int M1, const void* R1, int64_t ldr1, const float* gate1,
-                               int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N, int K,
-                               int epilogue, hipStream_t stream) {
-  if (int rc = gemm_validate(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N, K, epilogue, R0, ldr0, gate0,
+                               int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N0, int N1,
+                                 int K, int epilogue, hipStream_t stream) {
+  if (int rc = gemm_validate(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N0, K, epilogue, R0, ldr0, gate0,
                              gate_stride0, cu_seqlens0, nseg0))
     return rc;
-  if (int rc = gemm_validate(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N, K, epilogue, R1, ldr1, gate1,
+  if (int rc = gemm_validate(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N1, K, epilogue, R1, ldr1, gate1,
                              gate_stride1, cu_seqlens1, nseg1))
     return rc;
   // the one-wave-per-SIMD kernel addresses a wave tile's output and residual rows by 32-bit offsets
@@ -1005,10 +1004,12 @@ DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int
   if (M0 > 0 && M1 > 0 && epilogue != EPI_F32 && K % 64 == 0 && strides) {
     // one launch over both tile lists where its rounds cost less than two launches
     int cfg = -1;
-    float us = gemm_plan(M0, N, K).us + gemm_plan(M1, N, K).us;
+    float us = gemm_plan(M0, N0, K).us + gemm_plan(M1, N1, K).us;
     for (int c = 0; c < kL4Cfgs; ++c) {
-      const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn;
-      const float t = l4_cost(c, ((M0 + kL4[c].gbm - 1) / kL4[c].gbm + (M1 + kL4[c].gbm - 1) / kL4[c].gbm) * tn, K);
+      auto tiles = [&](int M, int N) {
+        return (int64_t)((M + kL4[c].gbm - 1) / kL4[c].gbm) * ((N + kL4[c].gbn - 1) / kL4[c].gbn);
+      };
+      const float t = l4_cost(c, tiles(M0, N0) + tiles(M1, N1), K);
       if (t < us) {
         us = t;
         cfg = c;
@@ -1016,21 +1017,33 @@ DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int
     }
     if (cfg >= 0) {
       const L4Prob p0{(const bf16_t*)A0, lda0, (const bf16_t*)W0, ldw0, bias0, C0, ldc0, (const bf16_t*)R0, ldr0,
-                      gate0, gate_stride0, cu_seqlens0, nseg0, M0, 0, 0};
+                      gate0, gate_stride0, cu_seqlens0, nseg0, M0, N0, 0, 0, 0};
       const L4Prob p1{(const bf16_t*)A1, lda1, (const bf16_t*)W1, ldw1, bias1, C1, ldc1, (const bf16_t*)R1, ldr1,
-                      gate1, gate_stride1, cu_seqlens1, nseg1, M1, 0, 0};
+                      gate1, gate_stride1, cu_seqlens1, nseg1, M1, N1, 0, 0, 0};
       switch (epilogue) {
-        case EPI_BIAS: return launch_l4_pair_cfg<EPI_BIAS>(cfg, p0, p1, N, K, stream);
-        case EPI_GELU: return launch_l4_pair_cfg<EPI_GELU>(cfg, p0, p1, N, K, stream);
-        case EPI_GATE_RES: return launch_l4_pair_cfg<EPI_GATE_RES>(cfg, p0, p1, N, K, stream);
-        case EPI_RES: return launch_l4_pair_cfg<EPI_RES>(cfg, p0, p1, N, K, stream);
-        default: return launch_l4_pair_cfg<EPI_SILU>(cfg, p0, p1, N, K, stream);
+        case EPI_BIAS: return launch_l4_pair_cfg<EPI_BIAS>(cfg, p0, p1, K, stream);
+        case EPI_GELU: return launch_l4_pair_cfg<EPI_GELU>(cfg, p0, p1, K, stream);
+        case EPI_GATE_RES: return launch_l4_pair_cfg<EPI_GATE_RES>(cfg, p0, p1, K, stream);
+        case EPI_RES: return launch_l4_pair_cfg<EPI_RES>(cfg, p0, p1, K, stream);
+        default: return launch_l4_pair_cfg<EPI_SILU>(cfg, p0, p1, K, stream);
       }
     }
   }
-  if (int rc = gemm_run(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N, K, epilogue, R0, ldr0, gate0, gate_stride0,
+  if (int rc = gemm_run(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N0, K, epilogue, R0, ldr0, gate0, gate_stride0,
                         cu_seqlens0, nseg0, stream))
     return rc;
-  return gemm_run(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N, K, epilogue, R1, ldr1, gate1, gate_stride1,
+  return gemm_run(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N1, K, epilogue, R1, ldr1, gate1, gate_stride1,
                   cu_seqlens1, nseg1, stream);
+}
+
+DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0,
+                               void* C0, int64_t ldc0, int M0, const void* R0, int64_t ldr0, const float* gate0,
+                               int64_t gate_stride0, const int32_t* cu_seqlens0, int nseg0, const void* A1,
+                               int64_t lda1, const void* W1, int64_t ldw1, const float* bias1, void* C1,
+                               int64_t ldc1, int M1, const void* R1, int64_t ldr1, const float* gate1,
+                               int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N, int K,
+                               int epilogue, hipStream_t stream) {
+  return ditk_gemm_pair_n(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, R0, ldr0, gate0, gate_stride0, cu_seqlens0, nseg0,
+                          A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, R1, ldr1, gate1, gate_stride1, cu_seqlens1, nseg1,
+                          N, N, K, epilogue, stream);
 }

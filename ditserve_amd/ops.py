@@ -520,13 +520,22 @@ def linear_pair(p0, p1, epilogue="bias"):
     residual, gate, segments, out).  Returns (out0, out1), each bitwise what
     linear() returns for it.  Each output may alias its own residual, but neither
     output may overlap any operand or the output of the other product."""
+    return _linear_pair(p0, p1, epilogue, True)
+
+
+def linear_pair_n(p0, p1, epilogue="bias"):
+    """linear_pair() of products that share K but may differ in N."""
+    return _linear_pair(p0, p1, epilogue, False)
+
+
+def _linear_pair(p0, p1, epilogue, one_n):
     def args(p):
         return _linear_args(p["x"], p["w"], p.get("b"), epilogue, p.get("residual"), p.get("gate"),
                             p.get("segments"), p.get("out"))
     o0, a0, N0, K0 = args(p0)
     o1, a1, N1, K1 = args(p1)
-    if (N0, K0) != (N1, K1):
-        raise ValueError(f"linear_pair needs one N and K (got {N0}x{K0} and {N1}x{K1})")
+    if K0 != K1 or (one_n and N0 != N1):
+        raise ValueError(f"linear_pair needs one {'N and ' if one_n else ''}K (got {N0}x{K0} and {N1}x{K1})")
     # the two products' tiles run concurrently in one launch or in order in two,
     # whichever pays: one product's output may not overlap the other's operands
     e0, e1 = _extent(o0), _extent(o1)
@@ -537,7 +546,7 @@ def linear_pair(p0, p1, epilogue="bias"):
                 raise ValueError(f"linear_pair: an output overlaps the {name} product's {key}")
         if _meet(out, other_out):
             raise ValueError(f"linear_pair: an output overlaps the {name} product's out")
-    _lib.call("ditk_gemm_pair", *a0, *a1, N0, K0, EPILOGUES[epilogue], _stream())
+    _lib.call("ditk_gemm_pair_n", *a0, *a1, N0, N1, K0, EPILOGUES[epilogue], _stream())
     return o0, o1
 
 

@@ -287,10 +287,9 @@ class SD35Transformer:
             nh, nc = normed[0], normed[1]
             nh2 = normed[2] if blk["dual"] else None
         with prof.region("gemm_qkv"):
-            with prof.region("gemm_qkv_img"):
-                qkv_i = ops.linear(nh, *blk["qkv"])
-            with prof.region("gemm_qkv_txt"):
-                qkv_t = ops.linear(nc, *blk["qkv_t"])
+            with prof.region("gemm_qkv_pair"):  # image and text, one launch where that pays
+                qkv_i, qkv_t = ops.linear_pair(dict(x=nh, w=blk["qkv"][0], b=blk["qkv"][1]),
+                                               dict(x=nc, w=blk["qkv_t"][0], b=blk["qkv_t"][1]))
         with prof.region("joint_prep"):
             q_i, k_i, v_i = qkv_i.split(D, 1)
             q_t, k_t, v_t = qkv_t.split(D, 1)

@@ -351,9 +351,9 @@ class WanTransformer:
         # cross-attention (_stage2, block.py:288-290)
         with prof.region("cross_prep"):
             x = ops.adaln(h, weight=blk["n2_w"], bias=blk["n2_b"], eps=cfg.eps)
-            with prof.region("gemm_cross_q"):
-                q2 = ops.linear(x, blk["q2_w"], blk["q2_b"])
-            kv2 = ops.linear(packet["encoder"], blk["kv2_w"], blk["kv2_b"])
+            with prof.region("gemm_cross_qkv"):  # image q and text K/V, one launch where that pays
+                q2, kv2 = ops.linear_pair_n(dict(x=x, w=blk["q2_w"], b=blk["q2_b"]),
+                                            dict(x=packet["encoder"], w=blk["kv2_w"], b=blk["kv2_b"]))
             k2, v2 = kv2.split(D, 1)
             # RMSNorm across heads of the image queries and the text keys, in place, one launch
             ops.adaln_multi([dict(x=q2, weight=blk["nq2_pre"], eps=cfg.eps, kind="rms", out=q2),

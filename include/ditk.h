@@ -164,6 +164,14 @@ int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, c
                    int64_t ldw1, const float* bias1, void* C1, int64_t ldc1, int M1, const void* R1, int64_t ldr1,
                    const float* gate1, int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N, int K,
                    int epilogue, ditk_stream_t stream);
+/* ditk_gemm_pair with features N0 and N1 of their own (e.g. Wan's cross-attention q of
+ * the image rows and K/V of the text rows). */
+int ditk_gemm_pair_n(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0, void* C0,
+                     int64_t ldc0, int M0, const void* R0, int64_t ldr0, const float* gate0, int64_t gate_stride0,
+                     const int32_t* cu_seqlens0, int nseg0, const void* A1, int64_t lda1, const void* W1,
+                     int64_t ldw1, const float* bias1, void* C1, int64_t ldc1, int M1, const void* R1, int64_t ldr1,
+                     const float* gate1, int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N0, int N1,
+                     int K, int epilogue, ditk_stream_t stream);
 
 /* Columns of the transposed-V buffer for Tk keys in nseg segments (upper bound). */
 int64_t ditk_vt_columns(int64_t Tk, int nseg);

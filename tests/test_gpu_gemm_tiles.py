@@ -80,3 +80,13 @@ def test_paired_tiles_match_single_launches(m0, m1, n, k, epi):
     got = ops.linear_pair(*probs, epi)
     for g, p in zip(got, probs):
         assert torch.equal(g, ops.linear(epilogue=epi, **p))
+
+
+@pytest.mark.parametrize("m0,n0,m1,n1,k", [(1560, 1536, 512, 3072, 1536), (2560, 1536, 1024, 3072, 1536),
+                                           (77, 200, 1300, 1544, 64), (1300, 4616, 1, 8, 128)])
+def test_paired_tiles_of_two_widths_match_single_launches(m0, n0, m1, n1, k):
+    ps = [dict(zip("xwb", _operands(m, n, k, n + m)[:3])) for m, n in ((m0, n0), (m1, n1))]
+    for g, p in zip(ops.linear_pair_n(*ps), ps):
+        assert torch.equal(g, ops.linear(**p))
+    with pytest.raises(ValueError, match="one N and K"):
+        ops.linear_pair(*ps)
