@@ -450,13 +450,15 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m, L4Prefetch pf, bool stream_out);
+                                        int group_m, L4Prefetch pf, bool stream_out,
+                                        int row_base);
 template <int EPI, int FI, int FJ>
 __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
     const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
     const float* __restrict__ bias, void* __restrict__ Cv, int64_t ldc, int M, int N, int K,
     const bf16_t* R, int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
-    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m, bool prefetch, bool stream_out) {
+    const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n, int group_m, bool prefetch, bool stream_out,
+    int row_base) {
   __shared__ u32x4_t lds[L4<FI, FJ>::LDS_BYTES / 16];
   // Persistent: XCD x (= blockIdx % 8) owns the tiles [x * per_xcd, (x + 1) *
   // per_xcd), which its workgroups take in turn (the order a one-tile-per-
@@ -466,10 +468,16 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_l4(
   const int nb = gridDim.x, b = blockIdx.x;
   const int ntiles = tiles_m * tiles_n, per_xcd = (ntiles + 7) / 8;
   const int tlo = (b & 7) * per_xcd, thi = min(tlo + per_xcd, ntiles);
+  // the epilogue's arguments are loaded here, under the first stages' DMA: first
+  // touched after the k loop, they cost a trip to memory (2 us of 18 at
+  // 2560 x 1536 x 1536)
+  if (EPI == EPI_GATE_RES) asm volatile("" ::"s"(R), "s"(ldr), "s"(gate), "s"(gate_stride), "s"(cu), "s"(nseg), "s"(row_base));
+  if (EPI == EPI_RES) asm volatile("" ::"s"(R), "s"(ldr));
+  asm volatile("" ::"s"(Cv), "s"(ldc));
   L4Prefetch pf = l4_prefetch(b, nb, N, K, prefetch);
   for (int L = tlo + (b >> 3); L < thi; L += nb >> 3) {
     l4_tile<EPI, FI, FJ>(lds, L, A, lda, W, ldw, bias, Cv, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, tiles_m,
-                     tiles_n, group_m, pf, stream_out);
+                     tiles_n, group_m, pf, stream_out, row_base);
     pf.n = 0;  // once per workgroup
   }
 }
@@ -515,7 +523,7 @@ __global__ __launch_bounds__(256, 1) void gemm_kernel_l4_pair(L4Prob p0, L4Prob 
                      s ? p1.M : p0.M, s ? p1.N : p0.N, K, s ? p1.R : p0.R, s ? p1.ldr : p0.ldr, s ? p1.gate : p0.gate,
                      s ? p1.gate_stride : p0.gate_stride, s ? p1.cu : p0.cu, s ? p1.nseg : p0.nseg,
                      s ? p1.tiles_m : p0.tiles_m, s ? p1.tiles_n : p0.tiles_n, s ? p1.group_m : p0.group_m, pf,
-                         stream_out);
+                         stream_out, 0);
     pf.n = 0;
   }
 }
@@ -526,7 +534,8 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
                                         void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
                                         int64_t ldr, const float* __restrict__ gate, int64_t gate_stride,
                                         const int32_t* __restrict__ cu, int nseg, int tiles_m, int tiles_n,
-                                        int group_m, L4Prefetch pf, bool stream_out) {
+                                        int group_m, L4Prefetch pf, bool stream_out,
+                                        int row_base) {
   using G = L4<FI, FJ>;
   constexpr int GBM = G::GBM, GBN = G::GBN, WTM = G::WTM, WTN = G::WTN, STG_ROW = G::STG_ROW;
   const int group = L / (group_m * tiles_n);
@@ -643,8 +652,8 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   bool one_seg = true;
   f32x4_t g0 = {0.f, 0.f, 0.f, 0.f}, g1 = {0.f, 0.f, 0.f, 0.f};
   if (EPI == EPI_GATE_RES) {
-    seg_lo = find_segment(cu, nseg, min(row0, M - 1));
-    one_seg = seg_lo == find_segment(cu, nseg, min(row0 + WTM, M) - 1);
+    seg_lo = find_segment(cu, nseg, row_base + min(row0, M - 1));
+    one_seg = seg_lo == find_segment(cu, nseg, row_base + min(row0 + WTM, M) - 1);
     if (one_seg) {
       const float* gp = gate + (int64_t)seg_lo * gate_stride + min(n, N - 8);
       g0 = *reinterpret_cast<const f32x4_t*>(gp);
@@ -690,7 +699,7 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
             f32x4_t h0 = g0, h1 = g1;
             if (!one_seg) {
               const int m = min(row0 + (r0 + q) * RPP + lane / CPR, M - 1);
-              const float* gp = gate + (int64_t)find_segment(cu, nseg, m) * gate_stride + min(n, N - 8);
+              const float* gp = gate + (int64_t)find_segment(cu, nseg, row_base + m) * gate_stride + min(n, N - 8);
               h0 = *reinterpret_cast<const f32x4_t*>(gp);
               h1 = *reinterpret_cast<const f32x4_t*>(gp + 4);
             }
@@ -778,7 +787,7 @@ bool l4_stream_out(int64_t M, int N) { return M * N * 2 >= (64ll << 20); }
 template <int EPI, int FI, int FJ>
 int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
               int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
-              const int32_t* cu, int nseg, hipStream_t stream) {
+              const int32_t* cu, int nseg, hipStream_t stream, int row_base) {
   constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
   const int tiles_m = (M + GBM - 1) / GBM, tiles_n = (N + GBN - 1) / GBN;
   // one persistent workgroup per CU (a multiple of 8: the same number per XCD)
@@ -786,7 +795,7 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
   gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM),
-      l4_stream_out(M, N));
+      l4_stream_out(M, N), row_base);
   return ditk_check_launch("ditk_gemm");
 }
 
@@ -825,14 +834,14 @@ int launch_tile(const void* A, int64_t lda, const void* W, int64_t ldw, const fl
 template <int EPI>
 int launch_l4_cfg(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
                   int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
-                  int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
+                  int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream, int row_base) {
   switch (cfg) {
-    case 0: return launch_l4<EPI, 8, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-    case 1: return launch_l4<EPI, 6, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-    case 2: return launch_l4<EPI, 8, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-    case 3: return launch_l4<EPI, 6, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-    case 4: return launch_l4<EPI, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-    default: return launch_l4<EPI, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+    case 0: return launch_l4<EPI, 8, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    case 1: return launch_l4<EPI, 6, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    case 2: return launch_l4<EPI, 8, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    case 3: return launch_l4<EPI, 6, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    case 4: return launch_l4<EPI, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    default: return launch_l4<EPI, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
   }
 }
 
@@ -860,27 +869,45 @@ float small_cost(int M, int N, int K) {
   return tiles <= cu_count() ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
 }
 
-// How one product runs: configuration cfg of gemm_kernel_l4 (-1: gemm_kernel's
-// 64 x 128 tiles) for the first M - tail rows, 64 x 128 tiles for the tail.  The
-// tail is a short last tile row, left to a second launch when that saves the
-// persistent kernel more (a round of tiles) than it costs.  Every row is computed
-// the same way whichever tile holds it, so the choice changes no result.  Against
-// the fastest of all configurations at each measured size the choice loses 0.4% on
-// average.
+// How one product runs: the first `rows` rows on configuration cfg of gemm_kernel_l4
+// (-1: gemm_kernel's 64 x 128 tiles), the rest in a second launch on rest_cfg.  A
+// second launch pays where the tiles of one configuration leave the last round of
+// CUs mostly idle: full rounds of it, then smaller tiles for the remaining rows
+// (14336 x 1536 x 8960: 336 tiles of 256 x 256 are 1.3 rounds, 367 -> 314 us;
+// 54560 x 3072 x 14336, whose last tile row has 32 rows, 3.89 -> 3.56 ms).  A short
+// last tile row is split off for any predicted gain, more rows at long K from
+// kSplitGain on: over several rounds the workgroups drift apart and the last round
+// costs less than a whole one (7000 x 4608 x 1536, 0.3% predicted: 78 -> 82 us; 28080
+// x 1536 x 1536, 8% predicted: 126 -> 133 us).
+// Every row is computed the same way whichever tile holds it, so the choice changes
+// no result.  Without splits the choice loses 0.4% on average against the fastest of
+// all configurations at each measured size.
 struct GemmPlan {
-  int cfg, tail;
+  int cfg, rows, rest_cfg;
   float us;
 };
-GemmPlan gemm_plan(int M, int N, int K) {
-  GemmPlan best{-1, 0, small_cost(M, N, K)};
+GemmPlan gemm_plan_one(int M, int N, int K) {
+  GemmPlan best{-1, M, -1, small_cost(M, N, K)};
   for (int c = 0; c < kL4Cfgs; ++c) {
-    const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn;
-    const int tm = (M + kL4[c].gbm - 1) / kL4[c].gbm, rem = M % kL4[c].gbm;
-    const float us = l4_cost(c, tm * tn, K);
-    if (us < best.us) best = GemmPlan{c, 0, us};
-    if (rem == 0 || tm < 2) continue;
-    const float split = l4_cost(c, (tm - 1) * tn, K) + small_cost(rem, N, K);
-    if (split < best.us) best = GemmPlan{c, rem, split};
+    const int64_t tiles = (int64_t)((M + kL4[c].gbm - 1) / kL4[c].gbm) * ((N + kL4[c].gbn - 1) / kL4[c].gbn);
+    const float us = l4_cost(c, tiles, K);
+    if (us < best.us) best = GemmPlan{c, M, -1, us};
+  }
+  return best;
+}
+constexpr float kSplitGain = 0.92f;
+GemmPlan gemm_plan(int M, int N, int K) {
+  GemmPlan best = gemm_plan_one(M, N, K);
+  const float one = best.us;
+  const int64_t ncu = std::max(8, cu_count() / 8 * 8);
+  for (int c = 0; c < kL4Cfgs; ++c) {
+    const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn, tm = (M + kL4[c].gbm - 1) / kL4[c].gbm;
+    const int64_t main_m = tm * tn / ncu * ncu / tn;  // tile rows of the full rounds
+    if (main_m == 0 || main_m >= tm || tm * tn % ncu == 0) continue;
+    const int rows = (int)main_m * kL4[c].gbm;
+    const GemmPlan rest = gemm_plan_one(M - rows, N, K);
+    const float us = l4_cost(c, main_m * tn, K) + rest.us;
+    if (us < best.us && (main_m == tm - 1 || (K >= 4096 && us < kSplitGain * one))) best = GemmPlan{c, rows, rest.cfg, us};
   }
   return best;
 }
@@ -897,21 +924,25 @@ int launch(const void* A, int64_t lda, const void* W, int64_t ldw, const float* 
   if constexpr (EPI != EPI_F32 && BK == 64) {
     if (ldc < (1 << 22) && ldr < (1 << 22)) {
       const GemmPlan p = gemm_plan(M, N, K);
-      // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
-      // more of the residual and gate reads (28000 x 1536 x 1536 129 -> 123 us, 9300
-      // 46.9 -> 44.6; at N = K = 3072 it is 0-3% slower)
-      if (EPI == EPI_GATE_RES && p.cfg == 0 && K < 3072)
-        return launch_tile<EPI, BK, TILE_LARGE>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-      const int Mm = p.cfg < 0 ? 0 : M - p.tail;
-      if (p.cfg >= 0)
-        if (int rc = launch_l4_cfg<EPI>(p.cfg, A, lda, W, ldw, bias, C, ldc, Mm, N, K, R, ldr, gate, gate_stride, cu,
-                                        nseg, stream))
-          return rc;
-      if (Mm == M) return 0;
-      return launch_tile<EPI, BK, TILE_SMALL>(static_cast<const bf16_t*>(A) + (int64_t)Mm * lda, lda, W, ldw, bias,
-                                              static_cast<bf16_t*>(C) + (int64_t)Mm * ldc, ldc, M - Mm, N, K,
-                                              R ? static_cast<const bf16_t*>(R) + (int64_t)Mm * ldr : nullptr, ldr,
-                                              gate, gate_stride, cu, nseg, stream, Mm);
+      // rows [m0, m0 + m) on configuration cfg
+      auto part = [&](int cfg, int m0, int m) {
+        const bf16_t* Am = static_cast<const bf16_t*>(A) + (int64_t)m0 * lda;
+        bf16_t* Cm = static_cast<bf16_t*>(C) + (int64_t)m0 * ldc;
+        const bf16_t* Rm = R ? static_cast<const bf16_t*>(R) + (int64_t)m0 * ldr : nullptr;
+        if (cfg < 0)
+          return launch_tile<EPI, BK, TILE_SMALL>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
+                                                  cu, nseg, stream, m0);
+        // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
+        // more of the residual and gate reads (28000 x 1536 x 1536 129 -> 123 us, 9300
+        // 46.9 -> 44.6; at N = K = 3072 it is 0-3% slower)
+        if (EPI == EPI_GATE_RES && cfg == 0 && K < 3072)
+          return launch_tile<EPI, BK, TILE_LARGE>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
+                                                  cu, nseg, stream, m0);
+        return launch_l4_cfg<EPI>(cfg, Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu, nseg,
+                                  stream, m0);
+      };
+      const int rc = part(p.cfg, 0, p.rows);
+      return rc != 0 || p.rows == M ? rc : part(p.rest_cfg, p.rows, M - p.rows);
     }
   }
   const int64_t large_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
