@@ -68,6 +68,7 @@ SIGNATURES = {
     "ditk_silu": (c_int, [_P, _P, c_int64, _P]),
     "ditk_adaln_multi": (c_int, [ctypes.POINTER(AdalnJob), c_int, _P]),
     "ditk_qk_norm_multi": (c_int, [ctypes.POINTER(QkNormJob), c_int, _P]),
+    "ditk_check_cu_seqlens_pair": (c_int, [_P, c_int, _P, _P, c_int, _P, c_int, _P, _P]),
     "ditk_check_cu_seqlens": (c_int, [_P, c_int, c_int, _P, _P, _P]),
     "ditk_solver_step": (c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, c_int64, _P, _P]),
     "ditk_flash_attn_varlen_noalloc": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64,

@@ -126,8 +126,7 @@ def flash_attn_varlen_func(q, k, v, cu_q, cu_k, max_q, max_k, dropout_p=0.0, cau
     tq, h, d = q.shape
     if cu_q.numel() != cu_k.numel():
         raise ValueError("cu_seqlens_q and cu_seqlens_k must have the same length")
-    seg_q = ops.Segments.from_device(cu_q.to(torch.int32), tq)
-    seg_k = ops.Segments.from_device(cu_k.to(torch.int32), k.shape[0])
+    seg_q, seg_k = ops.Segments.pair_from_device(cu_q.to(torch.int32), tq, cu_k.to(torch.int32), k.shape[0])
     out = ops.flash_attn_varlen(q.reshape(tq, h * d), k.reshape(k.shape[0], h * d),
                                 v.reshape(v.shape[0], h * d).contiguous(), seg_q, seg_k, h, d)
     return out.view(tq, h, d)

@@ -143,10 +143,21 @@ inline unsigned grid_for(int64_t n) {
 // A valid table (cu[0] = 0, nondecreasing, cu[n-1] = total) comes out unchanged;
 // any other sets bit 0 of *status (sticky: this kernel never clears it).  One
 // workgroup; chunks of 256 entries, each a block-wide running max on LDS.
-__global__ __launch_bounds__(256) void check_cu_kernel(const int32_t* __restrict__ cu, int n, int total,
-                                                       int32_t* __restrict__ out, int32_t* __restrict__ status) {
+// A workgroup per table (one or two in a launch).  The status may be in pinned host
+// memory: it is only written, and only for a bad table, so that a caller can poll it
+// without a copy per call.
+struct CuTable {
+  const int32_t* cu;
+  int32_t* out;
+  int n, total;
+};
+__global__ __launch_bounds__(256) void check_cu_kernel(CuTable t0, CuTable t1, int32_t* __restrict__ status) {
   __shared__ int32_t sm[256];
   const int tid = threadIdx.x;
+  const CuTable& t = blockIdx.x == 0 ? t0 : t1;
+  const int32_t* __restrict__ cu = t.cu;
+  int32_t* __restrict__ out = t.out;
+  const int n = t.n, total = t.total;
   int carry = 0, bad = 0;
   for (int base = 0; base < n; base += 256) {
     const int i = base + tid;
@@ -159,7 +170,7 @@ __global__ __launch_bounds__(256) void check_cu_kernel(const int32_t* __restrict
     }
     sm[tid] = v;
     __syncthreads();
-    for (int off = 1; off < 256; off <<= 1) {
+    for (int off = 1; off < min(256, n - base); off <<= 1) {
       const int x = tid >= off ? sm[tid - off] : 0;
       __syncthreads();
       sm[tid] = max(sm[tid], x);
@@ -169,7 +180,8 @@ __global__ __launch_bounds__(256) void check_cu_kernel(const int32_t* __restrict
     carry = max(carry, sm[255]);
     __syncthreads();
   }
-  if (__syncthreads_or(bad) && tid == 0) atomicOr(status, 1);
+  if (__syncthreads_or(bad) && tid == 0)
+    __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace
@@ -180,8 +192,22 @@ DITK_EXPORT int ditk_check_cu_seqlens(const int32_t* cu, int nseg, int total, in
   DITK_REQUIRE(cu != cu_out, "ditk_check_cu_seqlens: cu_out must not be cu");
   DITK_REQUIRE(nseg > 0 && nseg < (1 << 24) && total >= 0, "ditk_check_cu_seqlens: bad sizes (nseg %d, total %d)",
                nseg, total);
-  check_cu_kernel<<<1, 256, 0, stream>>>(cu, nseg + 1, total, cu_out, status);
+  const CuTable t{cu, cu_out, nseg + 1, total};
+  check_cu_kernel<<<1, 256, 0, stream>>>(t, t, status);
   return ditk_check_launch("ditk_check_cu_seqlens");
+}
+
+DITK_EXPORT int ditk_check_cu_seqlens_pair(const int32_t* cu0, int total0, int32_t* cu_out0, const int32_t* cu1,
+                                           int total1, int32_t* cu_out1, int nseg, int32_t* status,
+                                           hipStream_t stream) {
+  DITK_REQUIRE(cu0 && cu_out0 && cu1 && cu_out1 && status, "ditk_check_cu_seqlens_pair: null pointer");
+  DITK_REQUIRE(cu0 != cu_out0 && cu1 != cu_out1 && cu_out0 != cu_out1,
+               "ditk_check_cu_seqlens_pair: the outputs must be tables of their own");
+  DITK_REQUIRE(nseg > 0 && nseg < (1 << 24) && total0 >= 0 && total1 >= 0,
+               "ditk_check_cu_seqlens_pair: bad sizes (nseg %d, totals %d and %d)", nseg, total0, total1);
+  check_cu_kernel<<<2, 256, 0, stream>>>(CuTable{cu0, cu_out0, nseg + 1, total0}, CuTable{cu1, cu_out1, nseg + 1, total1},
+                                         status);
+  return ditk_check_launch("ditk_check_cu_seqlens_pair");
 }
 
 DITK_EXPORT int ditk_patchify(const void* latent, void* out, int C, int F, int H, int W, int pt, int ph,

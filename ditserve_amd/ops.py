@@ -107,17 +107,41 @@ class Segments:
         valid (cu[0] != 0, a decrease, cu[-1] != total) sets the device's sticky
         status, which the next call made after that kernel has finished raises
         (table_status(...).poll()), or check_tables() raises after a sync."""
-        if cu_dev.dtype != torch.int32 or cu_dev.dim() != 1 or cu_dev.numel() < 2 or cu_dev.device.type != "cuda":
-            raise ValueError("cu_seqlens must be a 1-D int32 cuda tensor with at least 2 entries")
+        cls._check_table(cu_dev)
         status = table_status(cu_dev.device)
         status.poll()
-        obj = cls.__new__(cls)
-        obj.cu = None
-        obj.dev = torch.empty_like(cu_dev, memory_format=torch.contiguous_format)
-        obj._nseg, obj._total = cu_dev.numel() - 1, int(total)
+        obj = cls._clamped(torch.empty_like(cu_dev, memory_format=torch.contiguous_format), total)
         _lib.call("ditk_check_cu_seqlens", _ptr(cu_dev.contiguous()), obj._nseg, obj._total, _ptr(obj.dev),
-                  _ptr(status.dev), _stream())
-        status.queue_read()
+                  _ptr(status.host), _stream())
+        return obj
+
+    @classmethod
+    def pair_from_device(cls, cu_q, total_q, cu_k, total_k):
+        """from_device() of a varlen call's query and key tables (equally long) in one launch."""
+        cls._check_table(cu_q)
+        cls._check_table(cu_k)
+        if cu_q.numel() != cu_k.numel():
+            raise ValueError("cu_seqlens_q and cu_seqlens_k must have the same length")
+        status = table_status(cu_q.device)
+        status.poll()
+        own = torch.empty((2, cu_q.numel()), dtype=torch.int32, device=cu_q.device).unbind(0)
+        q, k = cls._clamped(own[0], total_q), cls._clamped(own[1], total_k)
+        cu_q, cu_k = cu_q.contiguous(), cu_k.contiguous()
+        _lib.call("ditk_check_cu_seqlens_pair", _ptr(cu_q), q._total, _ptr(q.dev), _ptr(cu_k), k._total, _ptr(k.dev),
+                  q._nseg, _ptr(status.host), _stream())
+        return q, k
+
+    @staticmethod
+    def _check_table(cu_dev):
+        if cu_dev.dtype != torch.int32 or cu_dev.dim() != 1 or cu_dev.numel() < 2 or cu_dev.device.type != "cuda":
+            raise ValueError("cu_seqlens must be a 1-D int32 cuda tensor with at least 2 entries")
+
+    @classmethod
+    def _clamped(cls, dev, total):
+        """A table whose device copy `dev` a check kernel is about to write."""
+        obj = cls.__new__(cls)
+        obj.cu, obj.dev = None, dev
+        obj._nseg, obj._total = dev.numel() - 1, int(total)
         return obj
 
     @classmethod
@@ -166,38 +190,25 @@ _UNIFORM = {}
 
 
 class TableStatus:
-    """Sticky per-device flag of ditk_check_cu_seqlens.  After each check a copy of
-    the flag goes to pinned host memory without blocking; poll() looks at it only
-    once that copy has completed (an event query, never a wait) and raises if a
-    table was invalid.  check() waits for the device and raises likewise."""
+    """Sticky per-device flag of the cu_seqlens checks, in pinned host memory that the
+    check kernels write only for an invalid table: poll() looks at it without a
+    copy, an event or a wait and raises if a finished check (at the latest) set it;
+    check() waits for the device first."""
 
     def __init__(self, device):
-        self.dev = torch.zeros(1, dtype=torch.int32, device=device)
+        self.device = device
         self.host = torch.zeros(1, dtype=torch.int32).pin_memory()
-        self.event = None
 
-    def queue_read(self):
-        self.host.copy_(self.dev, non_blocking=True)
-        self.event = torch.cuda.Event()
-        self.event.record()
-
-    def _raise_if_set(self):
-        if int(self.host[0]) != 0:
+    def poll(self):
+        if self.host.item() != 0:
             self.host.zero_()
-            self.dev.zero_()
-            self.event = None
             raise _lib.DitkError("an invalid cu_seqlens table reached the attention kernels (cu[0] != 0, "
                                  "decreasing, or its last entry != the packed token count); it was clamped "
                                  "into bounds, so those outputs are not attention over the intended segments")
 
-    def poll(self):
-        if self.event is not None and self.event.query():
-            self._raise_if_set()
-
     def check(self):
-        torch.cuda.synchronize(self.dev.device)
-        self.host.copy_(self.dev)
-        self._raise_if_set()
+        torch.cuda.synchronize(self.device)
+        self.poll()
 
 
 _STATUS = {}

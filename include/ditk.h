@@ -312,6 +312,10 @@ int ditk_silu(const void* x, void* y, int64_t n, ditk_stream_t stream);
  */
 int ditk_check_cu_seqlens(const int32_t* cu, int nseg, int total, int32_t* cu_out, int32_t* status,
                           ditk_stream_t stream);
+/* ditk_check_cu_seqlens of two tables of nseg segments (a varlen call's queries and
+ * keys) in one launch.  In both, status may be pinned host memory. */
+int ditk_check_cu_seqlens_pair(const int32_t* cu0, int total0, int32_t* cu_out0, const int32_t* cu1, int total1,
+                               int32_t* cu_out1, int nseg, int32_t* status, ditk_stream_t stream);
 
 /*
  * Fused CFG combine + solver step for one request's fp32 latent of n elements,
