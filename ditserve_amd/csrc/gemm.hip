@@ -382,6 +382,96 @@ __global__ __launch_bounds__(Tile<T>::WM * Tile<T>::WN * 64, Tile<T>::WAVES_PER_
   }
 }
 
+// Up to 16 rows by many features (SD3.5's stacked modulations of a step: 2 rows by
+// 499 k features of K = 1536, 1.5 GB of weights): bound by streaming the weights
+// once.  One wave computes 16 features for all rows with the weights straight from
+// global memory into MFMA operands (no LDS, no barriers, no tile of 254 idle rows):
+// lane l loads 16 bytes of weight row n0 + l % 16 at k 8 (l / 16), a batch of SK_U
+// 32-k chunks ahead of the MFMAs: 341 -> 292 us, 4.5 -> 5.25 TB/s.  Fewer features
+// are bound by one wave's walk along K and gain nothing (9216: 10.8 against 11.0 us,
+// 1536: 5.5 against 6.2).  Same MFMA, k order, bias add and rounding as gemm_kernel:
+// bitwise its results.
+constexpr int kSkinnyM = 16, kSkinnyN = 16384;
+constexpr int SK_U = 8;
+template <int EPI>
+__global__ __launch_bounds__(256) void gemm_skinny(
+    const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
+    const float* __restrict__ bias, void* __restrict__ Cv, int64_t ldc, int M, int N, int K, const bf16_t* R,
+    int64_t ldr, const float* __restrict__ gate, int64_t gate_stride, const int32_t* __restrict__ cu, int nseg) {
+  const int lane = threadIdx.x & 63, ql = lane & 15, g = lane >> 4;
+  const int n0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+  if (n0 >= N) return;
+  const bf16_t* wp = W + (int64_t)min(n0 + ql, N - 1) * ldw + g * 8;
+  const bf16_t* xp = A + (int64_t)min(ql, M - 1) * lda + g * 8;
+  const int chunks = K / 32;
+  bf16x8_t w[2][SK_U], x[2][SK_U];
+  auto load = [&](int set, int c0) {
+#pragma unroll
+    for (int u = 0; u < SK_U; ++u) {
+      const int c = min(c0 + u, chunks - 1);  // past the end: the last chunk again, not used
+      w[set][u] = *reinterpret_cast<const bf16x8_t*>(wp + (int64_t)c * 32);
+      x[set][u] = *reinterpret_cast<const bf16x8_t*>(xp + (int64_t)c * 32);
+    }
+  };
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  auto use = [&](int set, int c0) {
+#pragma unroll
+    for (int u = 0; u < SK_U; ++u)
+      if (c0 + u < chunks) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[set][u], x[set][u], acc, 0, 0, 0);
+  };
+  load(0, 0);
+  for (int c = 0; c < chunks; c += 2 * SK_U) {
+    load(1, c + SK_U);
+    use(0, c);
+    load(0, c + 2 * SK_U);
+    use(1, c + SK_U);
+  }
+  // this lane: row ql, features n .. n + 3
+  const int n = n0 + 4 * g;
+  if (ql >= M || n >= N) return;
+  const f32x4_t y = acc + (bias != nullptr ? *reinterpret_cast<const f32x4_t*>(bias + n) : f32x4_t{0.f, 0.f, 0.f, 0.f});
+  if (EPI == EPI_F32) {
+    *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(Cv) + (int64_t)ql * ldc + n) = y;
+    return;
+  }
+  auto lo = [](uint32_t w2) { return __uint_as_float(w2 << 16); };
+  auto hi = [](uint32_t w2) { return __uint_as_float(w2 & 0xffff0000u); };
+  u32x2_t v{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+  if (EPI != EPI_BIAS) {
+    float f[4] = {lo(v[0]), hi(v[0]), lo(v[1]), hi(v[1])};
+    if (EPI == EPI_GELU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] = gelu_tanh_f(f[e]);
+    } else if (EPI == EPI_SILU) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f[e] = silu_f(f[e]);
+    } else {
+      const u32x2_t r = *reinterpret_cast<const u32x2_t*>(R + (int64_t)ql * ldr + n);
+      const float rv[4] = {lo(r[0]), hi(r[0]), lo(r[1]), hi(r[1])};
+      if (EPI == EPI_GATE_RES) {
+        const f32x4_t h = *reinterpret_cast<const f32x4_t*>(gate + (int64_t)find_segment(cu, nseg, ql) * gate_stride + n);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = fmaf(f[e], h[e], rv[e]);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) f[e] = rv[e] + f[e];
+      }
+    }
+    v = u32x2_t{pack_bf2(f[0], f[1]), pack_bf2(f[2], f[3])};
+  }
+  *reinterpret_cast<u32x2_t*>(reinterpret_cast<bf16_t*>(Cv) + (int64_t)ql * ldc + n) = v;
+}
+
+template <int EPI>
+int launch_skinny(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
+                  int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
+                  const int32_t* cu, int nseg, hipStream_t stream) {
+  gemm_skinny<EPI><<<(unsigned)((N + 63) / 64), 256, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C,
+                                                                 ldc, M, N, K, (const bf16_t*)R, ldr, gate,
+                                                                 gate_stride, cu, nseg);
+  return ditk_check_launch("ditk_gemm");
+}
+
 // One wave per SIMD (every epilogue but fp32, K % 64 == 0): a workgroup tile as
 // four wave tiles, their accumulators in the AGPRs (all 256 of them for the
 // 256 x 256 tile's 128 x 128 wave tiles).  The k loop and the bf16 staging are
@@ -920,6 +1010,8 @@ template <int EPI, int BK>
 int launch(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
            int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
            int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
+  if (M <= kSkinnyM && N >= kSkinnyN)
+    return launch_skinny<EPI>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
   // the one-wave-per-SIMD kernel's epilogue addresses a wave tile's rows by 32-bit offsets
   if constexpr (EPI != EPI_F32 && BK == 64) {
     if (ldc < (1 << 22) && ldr < (1 << 22)) {

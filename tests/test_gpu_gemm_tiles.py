@@ -66,6 +66,25 @@ def test_tiles_match_the_fp32_output_kernel(m, n, k):
         assert bool((out[m] == 7.0).all())  # nothing past the last row
 
 
+@pytest.mark.parametrize("m", [1, 2, 15, 16])
+@pytest.mark.parametrize("n,k", [(16384, 32), (16392, 96), (16440, 544), (20000, 1536)])
+def test_few_rows_match_the_tiles(m, n, k):
+    """Up to 16 rows run without LDS tiles: bit for bit the rows of a taller product."""
+    x, w, b, res, gate = _operands(40, n, k, m + n + k)
+    few, tall = ops.Segments([0, m // 2, m], "cuda"), ops.Segments([0, m // 2, 40], "cuda")
+    for epi in ("f32", "bias", "gelu", "silu", "res", "gate_res"):
+        kw = [dict(residual=res[:r]) if epi in ("res", "gate_res") else {} for r in (m, 40)]
+        if epi == "gate_res":
+            for d, seg in zip(kw, (few, tall)):
+                d.update(gate=gate, segments=seg)
+        out = torch.full((m + 1, n), 7.0, device="cuda", dtype=torch.float32 if epi == "f32" else torch.bfloat16)
+        ops.linear(x[:m], w, b, epi, out=out[:m], **kw[0])
+        assert torch.equal(out[:m], ops.linear(x, w, b, epi, **kw[1])[:m]), epi
+        assert bool((out[m] == 7.0).all())
+    y = x[:m].double() @ w.double().t() + b.double()
+    assert float((ops.linear(x[:m], w, b, "f32").double() - y).norm() / y.norm()) < 1e-6  # fp32 sums of k products
+
+
 @pytest.mark.parametrize("m0,m1,n,k", [(2048, 666, 1536, 6144), (2048, 666, 4608, 1536), (256, 100, 1536, 1536),
                                        (64, 2048, 1544, 64), (8192, 666, 1536, 256), (129, 1, 200, 128)])
 @pytest.mark.parametrize("epi", ["bias", "gelu", "gate_res"])
