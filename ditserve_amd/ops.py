@@ -687,11 +687,21 @@ def _bhsd_in_place(t):
 def patchify(latent, patch):
     """latent [C, F, H, W] bf16 -> [S, C*pt*ph*pw] bf16 (Conv3d-weight feature order)."""
     _check(latent, "latent", _BF16, 4)
+    return _patchify("ditk_patchify", latent, patch)
+
+
+def patchify_f32(latent, patch):
+    """patchify() of an fp32 latent: each value rounded to bf16 as .to(bfloat16) does."""
+    _check(latent, "latent", torch.float32, 4)
+    return _patchify("ditk_patchify_f32", latent, patch)
+
+
+def _patchify(entry, latent, patch):
     latent = latent.contiguous()
     C, F, H, W = latent.shape
     pt, ph, pw = patch
     out = torch.empty(((F // pt) * (H // ph) * (W // pw), C * pt * ph * pw), dtype=_BF16, device=latent.device)
-    _lib.call("ditk_patchify", _ptr(latent), _ptr(out), C, F, H, W, pt, ph, pw, _stream())
+    _lib.call(entry, _ptr(latent), _ptr(out), C, F, H, W, pt, ph, pw, _stream())
     return out
 
 

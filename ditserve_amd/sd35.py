@@ -376,7 +376,9 @@ class SD35Transformer:
         # prelude: patch embed (+ cropped 2D sin-cos positions), context embedder, temb
         h = torch.empty((seg_img.total, D), dtype=_BF16, device=dev)
         for m, (l, (hp, wp)) in enumerate(zip(lats, hw)):
-            patches = ops.patchify(l.reshape(cfg.in_ch, 1, *l.shape[1:]).to(_BF16), (1, P, P))
+            lat = l.reshape(cfg.in_ch, 1, *l.shape[1:])
+            patches = (ops.patchify_f32(lat, (1, P, P)) if lat.dtype == torch.float32 else
+                       ops.patchify(lat.to(_BF16), (1, P, P)))
             rows = h[seg_img.cu[m]:seg_img.cu[m + 1]]
             ops.linear(patches, self.pe_w, self.pe_b, "res", residual=self._pos(hp, wp), out=rows)
         c = ops.linear(torch.cat([x.to(device=dev, dtype=_BF16) for x in txts]), *self.ctx)

@@ -270,7 +270,9 @@ class WanTransformer:
             if key in cache:  # CFG pairs share the latent: patchify once
                 hidden[seg.cu[i]:seg.cu[i + 1]] = hidden[cache[key][0]:cache[key][1]]
                 continue
-            patches = ops.patchify(lat.reshape(lat.shape[-4:]).to(_BF16), cfg.patch)
+            lat = lat.reshape(lat.shape[-4:])
+            patches = (ops.patchify_f32(lat, cfg.patch) if lat.dtype == torch.float32 else
+                       ops.patchify(lat.to(_BF16), cfg.patch))
             ops.linear(patches, self.patch_w, self.patch_b, out=hidden[seg.cu[i]:seg.cu[i + 1]])
             cache[key] = (seg.cu[i], seg.cu[i + 1])
         text = torch.cat([x.reshape(-1, cfg.text_dim).to(device=dev, dtype=_BF16) for x in texts])

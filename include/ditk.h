@@ -266,6 +266,9 @@ int ditk_transpose_v_joint(const void* v_a, const void* v_b, int64_t ldv, void* 
  */
 int ditk_patchify(const void* latent, void* out, int C, int F, int H, int W, int pt, int ph, int pw,
                   ditk_stream_t stream);
+/* ditk_patchify of an fp32 latent, rounded to bf16 on the way (one launch). */
+int ditk_patchify_f32(const float* latent, void* out, int C, int F, int H, int W, int pt, int ph, int pw,
+                      ditk_stream_t stream);
 
 /*
  * x [S, pt*ph*pw*C] bf16 -> fp32 latent [C, F'*pt, H'*ph, W'*pw].
