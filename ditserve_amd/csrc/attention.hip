@@ -111,7 +111,7 @@ __device__ __forceinline__ int padded_key_start(const int32_t* __restrict__ cu, 
       [koff0] "v"(koff[0]), [koff1] "v"(koff[1]), [koff2] "v"(koff[2]), [koff3] "v"(koff[3]),                     \
       [koffl0] "v"(koffl[0]), [koffl1] "v"(koffl[1]), [koffl2] "v"(koffl[2]), [koffl3] "v"(koffl[3]),             \
       [voff0] "v"(voff[0]), [voff1] "v"(voff[1]), [voff2] "v"(voff[2]), [voff3] "v"(voff[3]),                     \
-      [lane] "v"(lanev), [qrow0] "v"(qrow0), [qrow1] "v"(qrow1)
+      [flag] "s"(su(lds_f)), [lane] "v"(lanev), [qrow0] "v"(qrow0), [qrow1] "v"(qrow1)
 // Pre-scaled q: the body's -m blocks take 32 more VGPRs, so the per-lane values
 // it reads only outside the key loop arrive in AGPRs
 #define DITK_ATTN_ASM_OPERANDS_PRE                                                                                  \
@@ -126,7 +126,7 @@ __device__ __forceinline__ int padded_key_start(const int32_t* __restrict__ cu, 
       [koff0] "a"(koff[0]), [koff1] "a"(koff[1]), [koff2] "a"(koff[2]), [koff3] "a"(koff[3]),                     \
       [koffl0] "a"(koffl[0]), [koffl1] "a"(koffl[1]), [koffl2] "a"(koffl[2]), [koffl3] "a"(koffl[3]),             \
       [voff0] "v"(voff[0]), [voff1] "v"(voff[1]), [voff2] "v"(voff[2]), [voff3] "v"(voff[3]),                     \
-      [lane] "a"(lanev), [qrow0] "a"(qrow0), [qrow1] "a"(qrow1)
+      [flag] "s"(su(lds_f)), [lane] "a"(lanev), [qrow0] "a"(qrow0), [qrow1] "a"(qrow1)
 // Joint sources (with pre-scaled q): the two K and O source bases of the segment
 // (the text ones shifted back by len_img rows), len_img, the segment's first
 // joint row, per-lane Q row addresses and the K rows of each DMA instruction
@@ -160,6 +160,7 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
   __shared__ u32x4_t Vs[2][HD * 8];
   constexpr int OPITCH = HD * 2 + 8;  // output staging row pitch (bytes), 32 rows per wave
   __shared__ u32x4_t Os[4 * 32 * OPITCH / 16];
+  __shared__ __align__(16) uint32_t Fs[NW];  // rescale flags of one-block waves
   // A work item is np consecutive BM-query tiles of one (segment, head), run as
   // passes of the body (the next pass's loads issued under the current pass's
   // last key tile).  Items in segment-major order (segment, then head, then
@@ -234,6 +235,7 @@ __global__ __launch_bounds__(256, 1) void flash_fwd_asm(
   const uint32_t lds_v = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4_t*)&Vs[0][0];
   const uint32_t lds_o = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) u32x4_t*)&Os[0] +
                          (uint32_t)wave_u * (32 * OPITCH);
+  const uint32_t lds_f = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint32_t*)&Fs[wave_u];
   uint32_t kaddr[4], vaddr[4], koff[4] = {}, koffl[4] = {}, voff[4] = {};
   const int lrow = lane >> 3;
   const int lsw0 = ((lane & 7) ^ ((lane >> 4) & 7)) * 8;

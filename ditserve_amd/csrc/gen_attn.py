@@ -84,7 +84,8 @@ def configure(hd, pre=False, joint=False, qb=2):
     256-query ones would leave CUs idle).  With one block a wave has half the MFMAs
     per key tile for the same fragment reads, so the reads are issued further ahead
     (a longer ring, from the registers the second block leaves free).  A query's
-    arithmetic does not depend on it: rescales are decided per block."""
+    arithmetic does not depend on it: rescales are decided for 64 queries, the blocks
+    of a wave or of a pair of one-block waves (flag_queries)."""
     global QB, BM, KRING, KA, VRING, VA
     QB, BM = qb, 128 * qb
     KRING, KA, VRING, VA = (3, 2, 6, 4) if qb == 2 else (6, 4, 10, 8)
@@ -126,7 +127,7 @@ S_NKT1 = 67      # s67 nkt - 1
 S_T0, S_T1 = 68, 69
 S_CMP = 70       # s[70:71] compare mask
 S_EXEC = 72      # s[72:73] saved exec (epilogue)
-S_FLAG = 72      # s[72:73] lanes of query block 0 past the rescale threshold (key loop)
+S_FLAG = 72      # s72 one-block waves: this wave's rescale flag (key loop)
 S_VALID = 74     # s74 valid keys of the last tile
 S_THR = 75       # s75 the lazy-rescale threshold 256.0
 S_QOFF = 76      # s76 query-row offset of the current pass (256 per pass)
@@ -541,15 +542,53 @@ def softmax_tile(g, s_set, p_set, qb, kks, rs_dst, masked=False):
                 g(f"v_add_f32 {vr(rs_dst + qb)}, {vr(rs_dst + qb)}, {vr(t0)}")
 
 
-def flag_blocks(g, rsum):
-    """The lanes of each query block whose row sum (VGPRs rsum + qb) is above 256 or
-    non-finite: S_FLAG (block 0), S_CMP (block 1); vcc = either, for the branch."""
-    if QB == 1:
+def flag_queries(g, rsum):
+    """Whether a lane's row sum (VGPRs rsum + qb) of these 64 queries is above 256 or
+    non-finite.  Returns the branches taken if one is and if none is."""
+    if QB == 2:
         g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(rsum)}")
-        return
-    g(f"v_cmp_nge_f32_e64 {sp(S_FLAG)}, {s_(S_THR)}, {vr(rsum)}")
-    g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(rsum + 1)}")
-    g(f"s_or_b64 vcc, {sp(S_FLAG)}, {sp(S_CMP)}")
+        g(f"v_cmp_nge_f32_e64 {sp(S_CMP)}, {s_(S_THR)}, {vr(rsum + 1)}")
+        g(f"s_or_b64 vcc, vcc, {sp(S_CMP)}")
+        return "s_cbranch_vccnz", "s_cbranch_vccz"
+    flag_post(g, rsum)
+    flag_fetch(g)
+    return flag_read(g)
+
+
+# One block per wave: waves 2 i and 2 i + 1 hold the 64 queries, and tell each other
+# through a word of LDS each (%[flag], the other wave's at ^ 4) around a barrier of their
+# own: post, fetch, read.  A word is posted again only past the barrier that ends the
+# tile, when the other wave has read it.  Exchanged right after the phase, the flags cost
+# about 200 cycles a key tile; P is therefore finished in three quarters of the phase's
+# MFMA slots and the exchange runs under the others (head_dim 64: 3-6% of the kernel back,
+# 128: 0-3%).  12 heads x 1560 of head_dim 128: 23.6 us without an exchange, 26.2 with it.
+FLAG_V, FLAG_A = 2, 3  # of DTMP: the word, its address
+
+
+def flag_post(g, rsum):
+    g(f"v_cmp_nge_f32 vcc, {s_(S_THR)}, {vr(rsum)}")
+    g(f"v_mov_b32 {vr(DTMP + FLAG_A)}, %[flag]")
+    g("s_cmp_lg_u64 vcc, 0")
+    g(f"s_cselect_b32 {s_(S_FLAG)}, 1, 0")
+    g(f"v_mov_b32 {vr(DTMP + FLAG_V)}, {s_(S_FLAG)}")
+    g(f"ds_write_b32 {vr(DTMP + FLAG_A)}, {vr(DTMP + FLAG_V)}")
+    g.lds_issue("flag posted")
+    g(f"v_xor_b32 {vr(DTMP + FLAG_A)}, 4, {vr(DTMP + FLAG_A)}")
+
+
+def flag_fetch(g):
+    g.lds_wait("flag posted")
+    g("s_barrier")
+    g(f"ds_read_b32 {vr(DTMP + FLAG_V)}, {vr(DTMP + FLAG_A)}")
+    g.lds_issue("flag fetched")
+
+
+def flag_read(g):
+    g.lds_wait("flag fetched")
+    g(f"v_readfirstlane_b32 {s_(S_CMP)}, {vr(DTMP + FLAG_V)}")
+    g(f"s_or_b32 {s_(S_CMP)}, {s_(S_CMP)}, {s_(S_FLAG)}")
+    g(f"s_cmp_lg_u32 {s_(S_CMP)}, 0")
+    return "s_cbranch_scc1", "s_cbranch_scc0"
 
 
 def exact_rescale(g, s_set, p_set, kks, masked=False, live_next=None):
@@ -557,15 +596,9 @@ def exact_rescale(g, s_set, p_set, kks, masked=False, live_next=None):
     scaled by exp2(m - m_new), P of the tile recomputed against m_new into rs0.
     (rs1 is cleared.)  Pre: the scores are relative to m_old, so m_new = max(m_old,
     row max + m_old); the tile's S and the next tile's (S set live_next, started
-    from the old -m block) move by -(m_new - m_old) and the block becomes -m_new.
-    A query block without a flagged lane (flag_blocks) keeps its m, P and sums, so
-    that its results do not depend on the blocks its wave holds beside it."""
+    from the old -m block) move by -(m_new - m_old) and the block becomes -m_new."""
     g.nops(20)  # O accumulators read below: MFMA results must have landed
     for qb in range(QB):
-        keep = g.new_label("keep")
-        if QB == 2:
-            g(f"s_cmp_eq_u64 {sp((S_FLAG, S_CMP)[qb])}, 0")
-            g(f"s_cbranch_scc1 {keep}")
         mx, tmp, alpha = DTMP + 1, DTMP + 2, DTMP + 3
         row_max_to(g, s_set, qb, mx, tmp, alpha)
         if PRE:
@@ -597,7 +630,6 @@ def exact_rescale(g, s_set, p_set, kks, masked=False, live_next=None):
         g(f"v_mov_b32 {vr(RS0 + qb)}, 0")
         g(f"v_mov_b32 {vr(RS1 + qb)}, 0")
         softmax_tile(g, s_set, p_set, qb, kks, RS0, masked)
-        g.label(keep)
     g.nops(5 if PRE else 3)  # v_accvgpr_write (and the -m block writes) -> MFMA srcC
 
 
@@ -642,13 +674,24 @@ def tile(g, a):
     dmas = ([(lambda i=i: kdma_m0(g, i, a), lambda i=i: kdma_go(g, i)) for i in range(ND)] +
             [(lambda i=i: vdma_m0(g, i, b), lambda i=i: vdma_go(g, i)) for i in range(ND)])
     # phase 1: S(kt+1) into set b || P(kt) keys 32..63 from set a
-    items = make_items(g, pair_list(1), a, a, RS1, slots=2 * QB * NC)
-    s_phase(g, b, kstage=b, vstage=a, items=items, dma=dmas)
-    # lazy-rescale check on tile kt: rsum = rs0 + rs1 (per lane), flag !(rsum <= 256)
-    for qb in range(QB):
-        g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
-    flag_blocks(g, DTMP)
-    g(f"s_cbranch_vccnz {resc}")
+    # and the lazy-rescale check on tile kt: rsum = rs0 + rs1 (per lane), flag !(rsum <= 256)
+    def row_sums():
+        for qb in range(QB):
+            g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
+    slots = 2 * QB * NC
+    if QB == 2:
+        s_phase(g, b, kstage=b, vstage=a, items=make_items(g, pair_list(1), a, a, RS1, slots=slots), dma=dmas)
+        row_sums()
+        flagged, _ = flag_queries(g, DTMP)
+    else:  # P done in three quarters of the slots, the flag exchange under the last MFMAs
+        most = slots * 3 // 4
+        items = make_items(g, pair_list(1), a, a, RS1, slots=most) + [lambda: None] * (slots - most)
+        last = items[most - 1]
+        items[most - 1] = lambda: (last(), row_sums(), flag_post(g, DTMP))
+        items[(most + slots) // 2 - 1] = lambda: flag_fetch(g)
+        s_phase(g, b, kstage=b, vstage=a, items=items, dma=dmas)
+        flagged, _ = flag_read(g)
+    g(f"{flagged} {resc}")
     g.label(after_check)
     for qb in range(QB):
         g(f"v_add_f32 {vr(LRUN + qb)}, {vr(LRUN + qb)}, {vr(DTMP + qb)}")
@@ -735,8 +778,8 @@ def last_tile(g, a):
         it()
     for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
-    flag_blocks(g, DTMP)
-    g(f"s_cbranch_vccz {reuse_back}")
+    _, clear = flag_queries(g, DTMP)
+    g(f"{clear} {reuse_back}")
     exact_rescale(g, a, a, (0, 1))
     for qb in range(QB):
         g(f"v_add_f32 {vr(DTMP + qb)}, {vr(RS0 + qb)}, {vr(RS1 + qb)}")
@@ -756,8 +799,8 @@ def last_tile(g, a):
     for qb in range(QB):
         softmax_tile(g, a, a, qb, (0, 1), RS0, masked=False)
     g.label(done_rs)
-    flag_blocks(g, RS0)
-    g(f"s_cbranch_vccz {checked}")
+    _, clear = flag_queries(g, RS0)
+    g(f"{clear} {checked}")
     # rescale against the exact tile max (masked sums)
     g(f"s_cmp_eq_u32 {s_(S_VALID)}, {BN}")
     g(f"s_cbranch_scc1 {resc}")
