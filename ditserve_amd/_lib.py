@@ -52,6 +52,7 @@ SIGNATURES = {
     "ditk_transpose_v": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, c_int, _P]),
     "ditk_flash_attn_varlen": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P,
                                        _P, c_int, c_int, c_int, c_int, c_float, _P]),
+    "ditk_attn_item_queries": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "ditk_transpose_v_bhsd": (c_int, [_P, c_int64, c_int64, c_int64, _P, c_int64, c_int, c_int, c_int, c_int, _P, _P]),
     "ditk_flash_attn_bhsd": (c_int, [_P, c_int64, c_int64, c_int64, _P, c_int64, c_int64, c_int64, _P, c_int64, _P,
                                      c_int64, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, _P]),

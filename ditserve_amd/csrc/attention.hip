@@ -421,13 +421,53 @@ DITK_EXPORT int ditk_transpose_v_joint(const void* v_a, const void* v_b, int64_t
 }
 
 namespace {
+// Workgroups of a launch with items of np tiles of bm queries (at least the items of any
+// tables with these totals), and its XCD chunk: a launch of less than a round
+// spreads over all XCDs.
+int64_t item_grid(int Tq, int nseg, int heads, int bm, int np, int* chunk) {
+  const int tiles_bound = ((Tq + bm - 1) / bm + nseg + np - 1) / np + nseg;
+  const int64_t nblocks = (int64_t)tiles_bound * heads;
+  *chunk = (int)std::min<int64_t>(kXcdChunk, (nblocks + 7) / 8);
+  return (nblocks + 8 * *chunk - 1) / (8 * *chunk) * (8 * *chunk);
+}
+
+// query tiles per work item, see flash_launch
+int item_passes(int64_t keys_per_seg, int Tq, int heads, bool joint) {
+  return !joint && keys_per_seg <= 2048 && (int64_t)((Tq + 255) / 256) * heads >= 2048 ? 4 : 1;
+}
+
+// Queries per work item: 128 (one 32-query block per wave) when 256-query items would
+// leave CUs idle, else 256.  The choice changes no result.  A 128-query item takes 0.60
+// (head_dim 128) to 0.66 (64) of a 256-query one's time with the CUs all busy (same key
+// tiles, half the MFMAs, the rescale flags of two waves exchanged), and CUs that are not
+// busy speed the others up, so 128-query items win while all of them run in one round
+// of CUs: 12 heads x 1536 queries and keys of head_dim 128 34.4 -> 27.2 us, 24 heads x
+// 1280 of head_dim 64 20.3 -> 18.0; not in 3 rounds for 2 (12 x 5888: 242 -> 250 us,
+// 6912: 326 -> 317; 24 x 3328 91.6 -> 99.1), nor in 2 for 1 (12 x 3584 78 -> 109).  One
+// segment or equal ones: rounds are compared at 0.75.  Segments of any lengths, which
+// only the device knows: 128-query items if they are at most a round however the Tq
+// queries are cut (at most one per 128 queries and segment); counted as if equal, 24
+// heads of 978 + 985 + 75 + 157 ran two rounds of them for one (20.8 -> 27.8 us), 12 of
+// 9000 + 3000 500 -> 563.
+int item_queries(int Tq, int nseg, int heads, int np, bool equal) {
+  if (np != 1) return 256;
+  const int64_t ncu = ditk_cu_count(), len = ((int64_t)Tq + nseg - 1) / nseg;
+  if (nseg == 1 || equal) {
+    auto rounds = [&](int64_t bm) { return (nseg * ((len + bm - 1) / bm) * heads + ncu - 1) / ncu; };
+    return 3 * rounds(128) < 4 * rounds(256) ? 128 : 256;
+  }
+  const int64_t most = std::max<int64_t>((int64_t)Tq - nseg, 0) / 128 + nseg;
+  return most * heads <= ncu ? 128 : 256;
+}
+
 // shared checks and launch of both attention entry points; sl2 = the factor that
-// takes q.k to log2 units inside the kernel (unused when pre)
+// takes q.k to log2 units inside the kernel (unused when pre); equal = the
+// segments are known to have Tq / nseg queries each
 int flash_launch(const void* q, int64_t ldq, const void* k, int64_t ldk, const void* vt, int64_t vt_ld, void* o,
                  int64_t ldo, float* lse, int64_t lse_ld, const int32_t* cu_q, const int32_t* cu_k, int nseg, int Tq,
                  int heads, int head_dim, float sl2, bool pre, RowLayout ql, RowLayout kl, hipStream_t stream,
-                 const void* q2 = nullptr, const void* kb = nullptr, void* ob = nullptr, const int32_t* cu_a = nullptr,
-                 const int32_t* cu_b = nullptr) {
+                 bool equal = false, const void* q2 = nullptr, const void* kb = nullptr, void* ob = nullptr,
+                 const int32_t* cu_a = nullptr, const int32_t* cu_b = nullptr) {
   const bool joint = cu_a != nullptr;
   DITK_REQUIRE(!joint || (pre && q2 && kb && ob && cu_b), "ditk_joint_attn: needs both sources and both tables");
   DITK_REQUIRE(!joint || (((uintptr_t)q2 % 16) == 0 && ((uintptr_t)kb % 16) == 0 && ((uintptr_t)ob % 8) == 0),
@@ -451,26 +491,10 @@ int flash_launch(const void* q, int64_t ldq, const void* k, int64_t ldk, const v
   // have few keys (vt_ld / nseg bounds the mean key count from above), so the
   // next tile's loads hide under the current one's last key tile, as long as
   // the items still fill the CUs at least twice over (512 items at 4 tiles each)
-  const int np = (!joint && vt_ld / nseg <= 2048 && (int64_t)((Tq + 255) / 256) * heads >= 2048) ? 4 : 1;
-  // 128-query work items (one 32-query block per wave) when the launch's 256-query
-  // ones would leave CUs idle: an item then takes about kHalfItem of a 256-query
-  // one's time (same key tiles, half the MFMAs; head_dim 64 is bound by its softmax
-  // instructions sooner).  Rounds of items counted as if the segments were equal; the
-  // choice changes no result.  12 heads x 1560 queries and keys of head_dim 128: 46.2
-  // -> 26.5 us, 2 x 1280 37.9 -> 25.3, 2600 69 -> 44, 1560 x 512 19.2 -> 12.6; 24 heads
-  // x 600 of head_dim 64 13.5 -> 10.0, but 2 x 1357 (3 rounds for 2) 43.7 -> 46.8.
-  const float kHalfItem = head_dim == 128 ? 0.57f : 0.72f;
-  auto rounds = [&](int bm) {
-    const int64_t tiles = (int64_t)nseg * (((Tq + nseg - 1) / nseg + bm - 1) / bm);
-    return (float)((tiles * heads + 255) / 256);
-  };
-  const int qb = np == 1 && kHalfItem * rounds(128) < rounds(256) ? 1 : 2;
-  const int bm = 128 * qb;
-  const int tiles_bound = ((Tq + bm - 1) / bm + nseg + np - 1) / np + nseg;
-  int64_t nblocks = (int64_t)tiles_bound * heads;
-  // a launch of less than a round spreads over all XCDs
-  const int chunk = (int)std::min<int64_t>(kXcdChunk, (nblocks + 7) / 8);
-  nblocks = (nblocks + 8 * chunk - 1) / (8 * chunk) * (8 * chunk);
+  const int np = item_passes(vt_ld / nseg, Tq, heads, joint);
+  const int qb = item_queries(Tq, nseg, heads, np, equal) / 128;
+  int chunk = 0;
+  const int64_t nblocks = item_grid(Tq, nseg, heads, 128 * qb, np, &chunk);
   DITK_REQUIRE(nblocks < (1ll << 31), "ditk_flash_attn_varlen: grid too large");
   // outputs of 64 MB and more are stored past the caches; smaller ones the next kernel still finds there
   const bool stream_out = (int64_t)Tq * heads * head_dim * 2 >= (64ll << 20);
@@ -514,7 +538,13 @@ DITK_EXPORT int ditk_joint_attn_q_prescaled(const void* q_a, const void* q_b, in
   DITK_REQUIRE(head_dim == 64, "ditk_joint_attn_q_prescaled: head_dim must be 64, got %d", head_dim);
   DITK_REQUIRE(cu_a && cu_b, "ditk_joint_attn_q_prescaled: null segment table");
   return flash_launch(q_a, ldq, k_a, ldk, vt, vt_ld, o_a, ldo, nullptr, 0, cu_joint, cu_joint, nseg, T_joint, heads,
-                      head_dim, 1.0f, true, RowLayout{head_dim, 0}, RowLayout{head_dim, 0}, stream, q_b, k_b, o_b, cu_a, cu_b);
+                      head_dim, 1.0f, true, RowLayout{head_dim, 0}, RowLayout{head_dim, 0}, stream, false, q_b, k_b, o_b,
+                      cu_a, cu_b);
+}
+
+DITK_EXPORT int ditk_attn_item_queries(int Tq, int Tk, int nseg, int heads, int equal, int joint) {
+  if (Tq < 0 || Tk < 0 || nseg <= 0 || heads <= 0) return 0;
+  return item_queries(Tq, nseg, heads, item_passes(ditk_vt_columns(Tk, nseg) / nseg, Tq, heads, joint != 0), equal != 0);
 }
 
 // [batch, heads, rows, head_dim] operands read in place: the attention backend's
@@ -541,7 +571,7 @@ DITK_EXPORT int ditk_flash_attn_bhsd(const void* q, int64_t q_bs, int64_t q_hs, 
                    q_ss < (1ll << 31), "ditk_flash_attn_bhsd: strides must be multiples of 8");
   return flash_launch(q, q_ss, k, k_ss, vt, vt_ld, o, ldo, lse, lse_ld, cu_q, cu_k, batch, batch * Sq, heads,
                       head_dim, softmax_scale * 1.4426950408889634f, false, RowLayout{q_hs, q_bs - Sq * q_ss},
-                      RowLayout{k_hs, k_bs - Sk * k_ss}, stream);
+                      RowLayout{k_hs, k_bs - Sk * k_ss}, stream, true);
 }
 
 // ---------------------------------------------------------------------------

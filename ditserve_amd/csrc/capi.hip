@@ -2,6 +2,8 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
+
 #include "ditk_common.h"
 
 namespace {
@@ -22,6 +24,21 @@ int ditk_check_launch(const char* what) {
     return 2;
   }
   return 0;
+}
+
+// Cached per device (callers on several host threads may race to fill an entry; they
+// store the same value).
+int ditk_cu_count() {
+  static std::atomic<int> cached[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int c = cached[dev].load(std::memory_order_relaxed);
+  if (c == 0) {
+    int n = 0;
+    c = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+    cached[dev].store(c, std::memory_order_relaxed);
+  }
+  return c;
 }
 
 DITK_EXPORT const char* ditk_last_error(void) { return g_err; }

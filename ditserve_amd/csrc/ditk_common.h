@@ -27,6 +27,7 @@ typedef __attribute__((__vector_size__(2 * sizeof(uint32_t)))) uint32_t u32x2_t;
 // ---------------------------------------------------------------------------
 void ditk_set_error(const char* fmt, ...);
 int ditk_check_launch(const char* what);
+int ditk_cu_count();  // CUs of the current device (256 without one)
 
 // Jobs of the multi-job row-kernel entry points; the same layout as the
 // declarations of include/ditk.h (C ABI).

@@ -811,20 +811,6 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   }
 }
 
-// CUs of the current device, cached per device (callers on several host
-// threads may race to fill an entry; they store the same value)
-int cu_count() {
-  static std::atomic<int> cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  int c = cached[dev].load(std::memory_order_relaxed);
-  if (c == 0) {
-    int n = 0;
-    c = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-    cached[dev].store(c, std::memory_order_relaxed);
-  }
-  return c;
-}
 // The tile configurations of gemm_kernel_l4: workgroup tile (tokens x features)
 // and its measured time in us, start + rounds x (tile + stage x K / 64) with a round
 // one tile per CU (least squares over 14 weight shapes of the Wan and SD3.5 blocks,
@@ -847,7 +833,7 @@ constexpr L4Cfg kL4[kL4Cfgs] = {{256, 256, -4.4f, 10.2f, 1.207f}, {256, 192, -2.
 // gemm_group_m's orders.
 int l4_group_m(int64_t tiles_m, int64_t tiles_n, int gbm, int gbn, int K) {
   const int64_t tiles = tiles_m * tiles_n, per_xcd = (tiles + 7) / 8;
-  if (tiles > 2 * cu_count()) return gemm_group_m(K, (int)tiles_n);
+  if (tiles > 2 * ditk_cu_count()) return gemm_group_m(K, (int)tiles_n);
   int64_t g = 1;
   while (g < tiles_m && (g + 1) * (g + 1) * gbm <= per_xcd * gbn) ++g;
   const int64_t groups = (tiles_m + g - 1) / g;
@@ -881,7 +867,7 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
   constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
   const int tiles_m = (M + GBM - 1) / GBM, tiles_n = (N + GBN - 1) / GBN;
   // one persistent workgroup per CU (a multiple of 8: the same number per XCD)
-  const int64_t nblocks = std::min<int64_t>(((int64_t)tiles_m * tiles_n + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
+  const int64_t nblocks = std::min<int64_t>(((int64_t)tiles_m * tiles_n + 7) / 8 * 8, std::max(8, ditk_cu_count() / 8 * 8));
   gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM),
@@ -898,7 +884,7 @@ int launch_l4_pair(L4Prob p0, L4Prob p1, int K, hipStream_t stream) {
     p->group_m = l4_group_m(p->tiles_m, p->tiles_n, GBM, GBN, K);
   }
   const int64_t tiles = (int64_t)p0.tiles_m * p0.tiles_n + (int64_t)p1.tiles_m * p1.tiles_n;
-  const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, cu_count() / 8 * 8));
+  const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, ditk_cu_count() / 8 * 8));
   gemm_kernel_l4_pair<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       p0, p1, K, l4_prefetch_on(p0.M, p0.N, K, p0.ldw, GBM) && (int64_t)p1.N * p1.ldw * 2 < (1ll << 31),
       l4_stream_out((int64_t)p0.M * p0.N + (int64_t)p1.M * p1.N, 1));
@@ -951,12 +937,12 @@ int launch_l4_pair_cfg(int cfg, const L4Prob& p0, const L4Prob& p1, int K, hipSt
 // tiles of gemm_kernel while each has a CU to itself (two sharing one run at half
 // the rate each, where the configurations above are the faster ones).
 float l4_cost(int c, int64_t tiles, int K) {
-  const int64_t ncu = std::max(8, cu_count() / 8 * 8), rounds = (tiles + ncu - 1) / ncu;
+  const int64_t ncu = std::max(8, ditk_cu_count() / 8 * 8), rounds = (tiles + ncu - 1) / ncu;
   return kL4[c].start + (float)rounds * (kL4[c].tile + kL4[c].stage * (float)(K / 64));
 }
 float small_cost(int M, int N, int K) {
   const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-  return tiles <= cu_count() ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
+  return tiles <= ditk_cu_count() ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
 }
 
 // How one product runs: the first `rows` rows on configuration cfg of gemm_kernel_l4
@@ -989,7 +975,7 @@ constexpr float kSplitGain = 0.92f;
 GemmPlan gemm_plan(int M, int N, int K) {
   GemmPlan best = gemm_plan_one(M, N, K);
   const float one = best.us;
-  const int64_t ncu = std::max(8, cu_count() / 8 * 8);
+  const int64_t ncu = std::max(8, ditk_cu_count() / 8 * 8);
   for (int c = 0; c < kL4Cfgs; ++c) {
     const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn, tm = (M + kL4[c].gbm - 1) / kL4[c].gbm;
     const int64_t main_m = tm * tn / ncu * ncu / tn;  // tile rows of the full rounds

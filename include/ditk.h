@@ -219,6 +219,11 @@ int ditk_flash_attn_bhsd(const void* q, int64_t q_bs, int64_t q_hs, int64_t q_ss
                          int64_t lse_ld, const int32_t* cu_q, const int32_t* cu_k, int batch, int Sq, int Sk,
                          int heads, int head_dim, float softmax_scale, ditk_stream_t stream);
 
+/* Queries per work item (128 or 256) of an attention launch over Tq queries and Tk keys in
+ * nseg segments (equal: ditk_flash_attn_bhsd; joint: ditk_joint_attn_q_prescaled); 0 for
+ * bad sizes.  For tests and tuning: the size changes no result. */
+int ditk_attn_item_queries(int Tq, int Tk, int nseg, int heads, int equal, int joint);
+
 /*
  * ditk_flash_attn_varlen with q already multiplied by softmax_scale * log2(e)
  * (head_dim 64 or 128).  A producer that folds that factor into its QK-norm
