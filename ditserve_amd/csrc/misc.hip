@@ -162,11 +162,12 @@ inline unsigned grid_for(int64_t n) {
 // and out[i] = max over j <= i of clamp(cu[j], 0, total), so the table is
 // nondecreasing inside [0, total] and every row a kernel derives from it exists.
 // A valid table (cu[0] = 0, nondecreasing, cu[n-1] = total) comes out unchanged;
-// any other sets bit 0 of *status (sticky: this kernel never clears it).  One
-// workgroup; chunks of 256 entries, each a block-wide running max on LDS.
+// any other sets bit 0 of *status (sticky: this kernel never clears it).  Chunks
+// of 256 entries, each a block-wide running max on LDS.
 // A workgroup per table (one or two in a launch).  The status may be in pinned host
-// memory: it is only written, and only for a bad table, so that a caller can poll it
-// without a copy per call.
+// memory, so that a caller can poll it without a copy per call: it is touched for a bad
+// table only, and by a load and a store, not by an atomic or, which the bus to the
+// host need not have (both tables set the same bit, so their order does not matter).
 struct CuTable {
   const int32_t* cu;
   int32_t* out;
@@ -201,8 +202,10 @@ __global__ __launch_bounds__(256) void check_cu_kernel(CuTable t0, CuTable t1, i
     carry = max(carry, sm[255]);
     __syncthreads();
   }
-  if (__syncthreads_or(bad) && tid == 0)
-    __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (__syncthreads_or(bad) && tid == 0) {
+    const int32_t old = __hip_atomic_load(status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(status, old | 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 }  // namespace

@@ -313,7 +313,8 @@ int ditk_silu(const void* x, void* y, int64_t n, ditk_stream_t stream);
  * cu_out[i] = the running max of cu[0..i] clamped into [0, total], so every row
  * the kernels derive from cu_out exists.  A valid table (cu[0] = 0,
  * nondecreasing, cu[nseg] = total) is copied unchanged; any other sets bit 0 of
- * *status, which the kernel never clears (the host reads it after a later sync).
+ * *status, which the kernel never clears (the host reads it after a later sync); the
+ * other bits stay as they are (nobody else may change them meanwhile).
  * No host synchronisation; cu_out must not be cu.
  * Replaces: the trust the reference's varlen slot places in its device tables
  *   (sd35_batch.py:448-486 passes cu_seqlens straight to the flash kernel).

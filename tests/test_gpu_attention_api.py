@@ -145,3 +145,35 @@ def test_backend_uniform_tables_are_cached():
     a = ops.Segments.uniform(2, 77, DEV)
     api.ditk_attention(x, x, x)
     assert ops.Segments.uniform(2, 77, DEV) is a and a.dev.tolist() == [0, 77, 154]
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+def test_table_check_sets_bit_0_and_keeps_the_others(pinned):
+    """ditk_check_cu_seqlens(_pair): an invalid table sets bit 0 of the status word, in
+    device or pinned host memory, and leaves the caller's other bits; a valid one
+    leaves it all."""
+    from ditserve_amd import _lib, ops
+    good = torch.tensor([0, 3, 10], dtype=torch.int32, device="cuda")
+    bad = torch.tensor([0, 12, 10], dtype=torch.int32, device="cuda")
+    out = torch.empty((2, 3), dtype=torch.int32, device="cuda")
+
+    def status(word):
+        t = torch.tensor([word], dtype=torch.int32)
+        return t.pin_memory() if pinned else t.cuda()
+
+    def check(tables, word):
+        st = status(word)
+        if len(tables) == 1:
+            _lib.call("ditk_check_cu_seqlens", tables[0].data_ptr(), 2, 10, out[0].data_ptr(), st.data_ptr(),
+                      ops._stream())
+        else:
+            _lib.call("ditk_check_cu_seqlens_pair", tables[0].data_ptr(), 10, out[0].data_ptr(), tables[1].data_ptr(),
+                      10, out[1].data_ptr(), 2, st.data_ptr(), ops._stream())
+        torch.cuda.synchronize()
+        return int(st.cpu()[0])
+
+    for word in (0, 6, 1 << 30):
+        assert check((good,), word) == word and check((good, good), word) == word
+        for tables in ((bad,), (bad, good), (good, bad), (bad, bad)):
+            assert check(tables, word) == word | 1, (word, len(tables))
+    assert out.tolist() == [[0, 10, 10], [0, 10, 10]]
