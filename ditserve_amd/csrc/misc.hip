@@ -225,7 +225,7 @@ DITK_EXPORT int ditk_check_cu_seqlens_pair(const int32_t* cu0, int total0, int32
                                            int total1, int32_t* cu_out1, int nseg, int32_t* status,
                                            hipStream_t stream) {
   DITK_REQUIRE(cu0 && cu_out0 && cu1 && cu_out1 && status, "ditk_check_cu_seqlens_pair: null pointer");
-  DITK_REQUIRE(cu0 != cu_out0 && cu1 != cu_out1 && cu_out0 != cu_out1,
+  DITK_REQUIRE(cu0 != cu_out0 && cu1 != cu_out1 && cu_out0 != cu_out1 && cu0 != cu_out1 && cu1 != cu_out0,
                "ditk_check_cu_seqlens_pair: the outputs must be tables of their own");
   DITK_REQUIRE(nseg > 0 && nseg < (1 << 24) && total0 >= 0 && total1 >= 0,
                "ditk_check_cu_seqlens_pair: bad sizes (nseg %d, totals %d and %d)", nseg, total0, total1);

@@ -39,3 +39,16 @@ def test_ops_reject_cpu_tensors_before_launch():
         ops.adaln(x)
     with pytest.raises(ValueError):
         ops.linear(x, torch.zeros(8, 64, dtype=torch.bfloat16))
+
+
+def test_table_pair_check_refuses_shared_outputs():
+    """The two workgroups of ditk_check_cu_seqlens_pair run at once: an output may be no
+    input and not the other output (refused before any launch; addresses only)."""
+    from ditserve_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("libditk.so not built (run python -m ditserve_amd.build)")
+    lib = _lib.load()
+    a, b, c, d, st = (0x1000 * i for i in range(1, 6))
+    for cu0, out0, cu1, out1 in ((a, a, b, c), (a, b, c, c), (a, b, c, b), (a, b, b, c), (a, b, c, a)):
+        assert lib.ditk_check_cu_seqlens_pair(cu0, 10, out0, cu1, 10, out1, 2, st, None) == 1
+        assert b"tables of their own" in lib.ditk_last_error()
