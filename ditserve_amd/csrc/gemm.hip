@@ -109,7 +109,9 @@ __device__ __forceinline__ void lds_dma16(const bf16_t* gsrc, u32x4_t* lds_slot0
 // features f = i*16 + 4*(lane/16) + e, token t = j*16 + lane % 16 of the wave
 // tile.  The bias is loaded after the k loop (holding it through the loop would
 // spill).
-template <int EPI, int BK, int T>
+// STREAM: output stored past the caches (see stream_output; a run-time choice in the
+// epilogue's stores costs 3% at 65520 x 1536 x 1536).
+template <int EPI, int BK, int T, bool STREAM>
 __global__ __launch_bounds__(Tile<T>::WM * Tile<T>::WN * 64, Tile<T>::WAVES_PER_EU) void gemm_kernel(
     const bf16_t* __restrict__ A, int64_t lda, const bf16_t* __restrict__ W, int64_t ldw,
     const float* __restrict__ bias, void* __restrict__ Cv, int64_t ldc, int M, int N, int K,
@@ -374,10 +376,7 @@ __global__ __launch_bounds__(Tile<T>::WM * Tile<T>::WN * 64, Tile<T>::WAVES_PER_
       v = pack8(x);
     }
     u32x4_t* dst = reinterpret_cast<u32x4_t*>(reinterpret_cast<bf16_t*>(Cv) + (int64_t)m * ldc + n);
-    // large-tile outputs (>= 16 MB) are streamed: the next kernel reads them back
-    // from HBM anyway, and non-temporal stores measured 2.6-3.6% faster on the
-    // K = 1536 block GEMMs (qkv, ffn up, o-proj), unchanged on ffn down
-    if (T == TILE_LARGE) __builtin_nontemporal_store(v, dst);
+    if (STREAM) __builtin_nontemporal_store(v, dst);
     else *dst = v;
   }
 }
@@ -854,12 +853,14 @@ bool l4_prefetch_on(int M, int N, int K, int64_t ldw, int gbm) {
   if (tiles_m < (K >= 4096 ? 4 : 8)) return false;
   return (int64_t)N * ldw * 2 < (1ll << 31) && (rem == 0 || (3 * rem > gbm && (gbm == 128 || K >= 4096)));
 }
-// Whether the output is stored past the caches.  Outputs of 64 MB and more are
-// (2.6-3.6% faster on the K = 1536 products of 65520 rows: they would not stay
+// Whether the output is stored past the caches (either kernel).  Outputs of 64 MB and more
+// are (2.6-3.6% faster on the K = 1536 products of 65520 rows: they would not stay
 // cached until the next kernel reads them); smaller ones stay, and the next kernel
 // finds them (one-frame Wan block 300 -> 281 us, preview step of 2 x 1280 rows
-// 11.20 -> 10.90 ms, SD3.5 512 step 8.65 -> 8.37 ms).
-bool l4_stream_out(int64_t M, int N) { return M * N * 2 >= (64ll << 20); }
+// 11.20 -> 10.90 ms, SD3.5 512 step 8.65 -> 8.37 ms; gated residual of K = N = 1536 on
+// gemm_kernel and the AdaLN after it: 9300 rows 59.1 -> 57.8 us, 20000 113.2 -> 110.7,
+// but 21800, just below the line, 129 -> 132).
+bool stream_output(int64_t M, int N) { return M * N * 2 >= (64ll << 20); }
 template <int EPI, int FI, int FJ>
 int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
               int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
@@ -871,7 +872,7 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
   gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM),
-      l4_stream_out(M, N), row_base);
+      stream_output(M, N), row_base);
   return ditk_check_launch("ditk_gemm");
 }
 
@@ -887,7 +888,7 @@ int launch_l4_pair(L4Prob p0, L4Prob p1, int K, hipStream_t stream) {
   const int64_t nblocks = std::min<int64_t>((tiles + 7) / 8 * 8, std::max(8, ditk_cu_count() / 8 * 8));
   gemm_kernel_l4_pair<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       p0, p1, K, l4_prefetch_on(p0.M, p0.N, K, p0.ldw, GBM) && (int64_t)p1.N * p1.ldw * 2 < (1ll << 31),
-      l4_stream_out((int64_t)p0.M * p0.N + (int64_t)p1.M * p1.N, 1));
+      stream_output((int64_t)p0.M * p0.N + (int64_t)p1.M * p1.N, 1));
   return ditk_check_launch("ditk_gemm_pair");
 }
 
@@ -900,7 +901,9 @@ int launch_tile(const void* A, int64_t lda, const void* W, int64_t ldw, const fl
   const int64_t tiles = (int64_t)tiles_m * tiles_n;
   const int64_t nblocks = (tiles + 7) / 8 * 8;
   DITK_REQUIRE(nblocks < (1ll << 31), "ditk_gemm: grid too large");
-  gemm_kernel<EPI, BK, T><<<(unsigned)nblocks, S::GW * 64, 0, stream>>>(
+  constexpr bool kMayStream = T == TILE_LARGE && EPI != EPI_F32;
+  auto kern = kMayStream && stream_output(M, N) ? gemm_kernel<EPI, BK, T, kMayStream> : gemm_kernel<EPI, BK, T, false>;
+  kern<<<(unsigned)nblocks, S::GW * 64, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, gemm_group_m(K, tiles_n), row_base);
   return ditk_check_launch("ditk_gemm");
@@ -1011,8 +1014,9 @@ int launch(const void* A, int64_t lda, const void* W, int64_t ldw, const float* 
           return launch_tile<EPI, BK, TILE_SMALL>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
                                                   cu, nseg, stream, m0);
         // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
-        // more of the residual and gate reads (28000 x 1536 x 1536 129 -> 123 us, 9300
-        // 46.9 -> 44.6; at N = K = 3072 it is 0-3% slower)
+        // more of the residual and gate reads (1536 x 1536, with the AdaLN that reads the
+        // output next: 28080 rows 175 -> 166 us, 20000 115 -> 110, 9300 62 -> 58; at N = K = 3072
+        // it is 0-3% slower)
         if (EPI == EPI_GATE_RES && cfg == 0 && K < 3072)
           return launch_tile<EPI, BK, TILE_LARGE>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
                                                   cu, nseg, stream, m0);

@@ -15,8 +15,8 @@ SHAPES = [(m, n, k) for n, k in ((1536, 64), (200, 192), (1544, 320), (4616, 128
 SHAPES += [(1560, 1536, 1536), (2048, 1536, 2048), (2560, 4608, 448), (1024, 8968, 256), (666, 6144, 576),
            (3480, 1536, 4160), (16416, 3072, 256), (4096, 1536, 4096),
            (1560, 4608, 1536), (666, 8960, 704), (5001, 3080, 64), (5001, 1544, 128), (1500, 4616, 192),
-           (2500, 1544, 64), (1500, 1544, 192)]
-
+           (2500, 1544, 64), (1500, 1544, 192),
+           (21000, 1536, 1536), (22000, 1536, 1536)]  # outputs of 62 MB, left in the caches, and 64 MB, stored past them
 
 
 def _operands(m, n, k, seed):
