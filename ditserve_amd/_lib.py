@@ -48,6 +48,8 @@ SIGNATURES = {
     "ditk_gemm_pair_n": (c_int, [_P, c_int64, _P, c_int64, _P, _P, c_int64, c_int, _P, c_int64, _P, c_int64, _P, c_int,
                                  _P, c_int64, _P, c_int64, _P, _P, c_int64, c_int, _P, c_int64, _P, c_int64, _P, c_int,
                                  c_int, c_int, c_int, c_int, _P]),
+    "ditk_gemm_plan": (c_int, [c_int, c_int, c_int, c_int, ctypes.POINTER(c_int)]),
+    "ditk_gemm_pair_plan": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int]),
     "ditk_vt_columns": (c_int64, [c_int64, c_int]),
     "ditk_transpose_v": (c_int, [_P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, c_int, _P]),
     "ditk_flash_attn_varlen": (c_int, [_P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P,

@@ -936,22 +936,32 @@ int launch_l4_pair_cfg(int cfg, const L4Prob& p0, const L4Prob& p1, int K, hipSt
   }
 }
 
-// Estimated time (us) of `tiles` tiles of configuration c, and of M x N on the 64 x 128
-// tiles of gemm_kernel while each has a CU to itself (two sharing one run at half
-// the rate each, where the configurations above are the faster ones).
-float l4_cost(int c, int64_t tiles, int K) {
-  const int64_t ncu = std::max(8, ditk_cu_count() / 8 * 8), rounds = (tiles + ncu - 1) / ncu;
+// Estimated time (us) of `tiles` tiles of configuration c on `cus` CUs, and of M x N on
+// the 64 x 128 tiles of gemm_kernel while each has a CU to itself (two sharing one run at
+// half the rate each, where the configurations above are the faster ones).
+float l4_cost(int c, int64_t tiles, int K, int cus) {
+  const int64_t ncu = std::max(8, cus / 8 * 8), rounds = (tiles + ncu - 1) / ncu;
   return kL4[c].start + (float)rounds * (kL4[c].tile + kL4[c].stage * (float)(K / 64));
 }
-float small_cost(int M, int N, int K) {
+float small_cost(int M, int N, int K, int cus) {
   const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 127) / 128);
-  return tiles <= ditk_cu_count() ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
+  return tiles <= cus ? 2.8f + 0.411f * (float)(K / 64) : 1e30f;
+}
+int64_t l4_tiles(int c, int M, int N) {
+  return (int64_t)((M + kL4[c].gbm - 1) / kL4[c].gbm) * ((N + kL4[c].gbn - 1) / kL4[c].gbn);
 }
 
-// How one product runs: the first `rows` rows on configuration cfg of gemm_kernel_l4
-// (-1: gemm_kernel's 64 x 128 tiles), the rest in a second launch on rest_cfg.  A
-// second launch pays where the tiles of one configuration leave the last round of
-// CUs mostly idle: full rounds of it, then smaller tiles for the remaining rows
+// The kernels and tiles a product can run on (as numbered by ditk_gemm_plan).
+enum GemmTile : int {
+  GT_SMALL = 0,                    // gemm_kernel, 64 x 128
+  GT_LARGE = 1,                    // gemm_kernel, 256 x 256
+  GT_L4 = 2,                       // + a configuration of kL4: gemm_kernel_l4
+  GT_SKINNY = GT_L4 + kL4Cfgs,     // gemm_skinny
+};
+
+// How one product runs: the first `rows` rows on `tile`, the others in a second launch
+// on `rest`.  A second launch pays where the tiles of one configuration leave the last
+// round of CUs mostly idle: full rounds of it, then smaller tiles for the remaining rows
 // (14336 x 1536 x 8960: 336 tiles of 256 x 256 are 1.3 rounds, 367 -> 314 us;
 // 54560 x 3072 x 14336, whose last tile row has 32 rows, 3.89 -> 3.56 ms).  A short
 // last tile row is split off for any predicted gain, more rows at long K from
@@ -962,85 +972,93 @@ float small_cost(int M, int N, int K) {
 // no result.  Without splits the choice loses 0.4% on average against the fastest of
 // all configurations at each measured size.
 struct GemmPlan {
-  int cfg, rows, rest_cfg;
+  int tile, rows, rest;
   float us;
 };
-GemmPlan gemm_plan_one(int M, int N, int K) {
-  GemmPlan best{-1, M, -1, small_cost(M, N, K)};
+GemmPlan gemm_plan_one(int M, int N, int K, int cus) {
+  GemmPlan best{GT_SMALL, M, GT_SMALL, small_cost(M, N, K, cus)};
   for (int c = 0; c < kL4Cfgs; ++c) {
-    const int64_t tiles = (int64_t)((M + kL4[c].gbm - 1) / kL4[c].gbm) * ((N + kL4[c].gbn - 1) / kL4[c].gbn);
-    const float us = l4_cost(c, tiles, K);
-    if (us < best.us) best = GemmPlan{c, M, -1, us};
+    const float us = l4_cost(c, l4_tiles(c, M, N), K, cus);
+    if (us < best.us) best = GemmPlan{GT_L4 + c, M, GT_SMALL, us};
   }
   return best;
 }
 constexpr float kSplitGain = 0.92f;
-GemmPlan gemm_plan(int M, int N, int K) {
-  GemmPlan best = gemm_plan_one(M, N, K);
+GemmPlan gemm_plan_l4(int M, int N, int K, int cus) {
+  GemmPlan best = gemm_plan_one(M, N, K, cus);
   const float one = best.us;
-  const int64_t ncu = std::max(8, ditk_cu_count() / 8 * 8);
+  const int64_t ncu = std::max(8, cus / 8 * 8);
   for (int c = 0; c < kL4Cfgs; ++c) {
     const int64_t tn = (N + kL4[c].gbn - 1) / kL4[c].gbn, tm = (M + kL4[c].gbm - 1) / kL4[c].gbm;
     const int64_t main_m = tm * tn / ncu * ncu / tn;  // tile rows of the full rounds
     if (main_m == 0 || main_m >= tm || tm * tn % ncu == 0) continue;
     const int rows = (int)main_m * kL4[c].gbm;
-    const GemmPlan rest = gemm_plan_one(M - rows, N, K);
-    const float us = l4_cost(c, main_m * tn, K) + rest.us;
-    if (us < best.us && (main_m == tm - 1 || (K >= 4096 && us < kSplitGain * one))) best = GemmPlan{c, rows, rest.cfg, us};
+    const GemmPlan rest = gemm_plan_one(M - rows, N, K, cus);
+    const float us = l4_cost(c, main_m * tn, K, cus) + rest.us;
+    if (us < best.us && (main_m == tm - 1 || (K >= 4096 && us < kSplitGain * one)))
+      best = GemmPlan{GT_L4 + c, rows, rest.tile, us};
   }
   return best;
 }
 
-// fp32 outputs and K % 64 != 0: gemm_kernel, on small tiles when the large ones
-// would number fewer than kSmallBelow (666 rows 1.3-3x faster at 54-72 large tiles,
-// 8192 x 1536 1.25-1.5x slower at 192).
+// narrow: every output and residual row stride below 2^22 (the one-wave-per-SIMD kernel's
+// epilogue addresses a wave tile's rows by 32-bit offsets).  fp32 outputs and K % 64 != 0:
+// gemm_kernel, on small tiles when the large ones would number fewer than
+// kSmallBelow (666 rows 1.3-3x faster at 54-72 large tiles, 8192 x 1536 1.25-1.5x
+// slower at 192).
 constexpr int64_t kSmallBelow = 128;
+GemmPlan gemm_plan(int M, int N, int K, int epilogue, bool narrow, int cus) {
+  if (M <= kSkinnyM && N >= kSkinnyN)  // its weights at 5.25 TB/s
+    return GemmPlan{GT_SKINNY, M, GT_SMALL, 2.f + (float)N * (float)K * (2.f / 5.25e6f)};
+  if (epilogue == EPI_F32 || K % 64 != 0 || !narrow) {
+    const int64_t large_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
+    return GemmPlan{large_tiles < kSmallBelow ? GT_SMALL : GT_LARGE, M, GT_SMALL, 0.f};
+  }
+  GemmPlan p = gemm_plan_l4(M, N, K, cus);
+  // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
+  // more of the residual and gate reads (1536 x 1536, with the AdaLN that reads the
+  // output next: 28080 rows 175 -> 166 us, 20000 115 -> 110, 9300 62 -> 58; at N = K = 3072
+  // it is 0-3% slower)
+  if (epilogue == EPI_GATE_RES && K < 3072)
+    for (int* t : {&p.tile, &p.rest})
+      if (*t == GT_L4) *t = GT_LARGE;
+  return p;
+}
+
 template <int EPI, int BK>
-int launch(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
+int launch(const GemmPlan& plan, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
            int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
            int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
-  if (M <= kSkinnyM && N >= kSkinnyN)
-    return launch_skinny<EPI>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-  // the one-wave-per-SIMD kernel's epilogue addresses a wave tile's rows by 32-bit offsets
-  if constexpr (EPI != EPI_F32 && BK == 64) {
-    if (ldc < (1 << 22) && ldr < (1 << 22)) {
-      const GemmPlan p = gemm_plan(M, N, K);
-      // rows [m0, m0 + m) on configuration cfg
-      auto part = [&](int cfg, int m0, int m) {
-        const bf16_t* Am = static_cast<const bf16_t*>(A) + (int64_t)m0 * lda;
-        bf16_t* Cm = static_cast<bf16_t*>(C) + (int64_t)m0 * ldc;
-        const bf16_t* Rm = R ? static_cast<const bf16_t*>(R) + (int64_t)m0 * ldr : nullptr;
-        if (cfg < 0)
-          return launch_tile<EPI, BK, TILE_SMALL>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
-                                                  cu, nseg, stream, m0);
-        // the gated residual at short K: the 8-wave kernel's two waves per SIMD hide
-        // more of the residual and gate reads (1536 x 1536, with the AdaLN that reads the
-        // output next: 28080 rows 175 -> 166 us, 20000 115 -> 110, 9300 62 -> 58; at N = K = 3072
-        // it is 0-3% slower)
-        if (EPI == EPI_GATE_RES && cfg == 0 && K < 3072)
-          return launch_tile<EPI, BK, TILE_LARGE>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
-                                                  cu, nseg, stream, m0);
-        return launch_l4_cfg<EPI>(cfg, Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu, nseg,
-                                  stream, m0);
-      };
-      const int rc = part(p.cfg, 0, p.rows);
-      return rc != 0 || p.rows == M ? rc : part(p.rest_cfg, p.rows, M - p.rows);
-    }
-  }
-  const int64_t large_tiles = (int64_t)((M + 255) / 256) * ((N + 255) / 256);
-  if (large_tiles < kSmallBelow)
-    return launch_tile<EPI, BK, TILE_SMALL>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
-  return launch_tile<EPI, BK, TILE_LARGE>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+  // rows [m0, m0 + m) on tile
+  auto part = [&](int tile, int m0, int m) {
+    constexpr int esize = EPI == EPI_F32 ? 4 : 2;
+    const void* Am = static_cast<const bf16_t*>(A) + (int64_t)m0 * lda;
+    void* Cm = static_cast<char*>(C) + (int64_t)m0 * ldc * esize;
+    const void* Rm = R ? static_cast<const bf16_t*>(R) + (int64_t)m0 * ldr : nullptr;
+    if (tile == GT_SKINNY)
+      return launch_skinny<EPI>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu, nseg, stream);
+    if (tile == GT_SMALL)
+      return launch_tile<EPI, BK, TILE_SMALL>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
+                                              cu, nseg, stream, m0);
+    if constexpr (EPI != EPI_F32 && BK == 64)
+      if (tile >= GT_L4)
+        return launch_l4_cfg<EPI>(tile - GT_L4, Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu,
+                                  nseg, stream, m0);
+    return launch_tile<EPI, BK, TILE_LARGE>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
+                                            cu, nseg, stream, m0);
+  };
+  const int rc = part(plan.tile, 0, plan.rows);
+  return rc != 0 || plan.rows == M ? rc : part(plan.rest, plan.rows, M - plan.rows);
 }
 
 template <int EPI>
-int launch_k(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
+int launch_k(const GemmPlan& plan, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
              int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
              int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
   // 64-k stages when K allows (half the barriers); the MFMA k order is the
   // same for both, so results do not depend on the choice
-  return K % 64 == 0 ? launch<EPI, 64>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream)
-                     : launch<EPI, 32>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
+  return K % 64 == 0 ? launch<EPI, 64>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream)
+                     : launch<EPI, 32>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream);
 }
 
 }  // namespace
@@ -1073,17 +1091,36 @@ int gemm_validate(const void* A, int64_t lda, const void* W, int64_t ldw, const 
   return 0;
 }
 
-int gemm_run(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
-             int M, int N, int K, int epilogue, const void* R, int64_t ldr, const float* gate,
+bool narrow(int64_t ldc, int64_t ldr) { return ldc < (1 << 22) && ldr < (1 << 22); }
+
+// The configuration of kL4 that takes two products in one launch, where its rounds over
+// both tile lists cost less than the two launches p0 and p1; -1 where none does.
+int pair_plan(const GemmPlan& p0, const GemmPlan& p1, int M0, int N0, int M1, int N1, int K, int epilogue, bool narrow,
+              int cus) {
+  if (M0 <= 0 || M1 <= 0 || epilogue == EPI_F32 || K % 64 != 0 || !narrow) return -1;
+  int cfg = -1;
+  float us = p0.us + p1.us;
+  for (int c = 0; c < kL4Cfgs; ++c) {
+    const float t = l4_cost(c, l4_tiles(c, M0, N0) + l4_tiles(c, M1, N1), K, cus);
+    if (t < us) {
+      us = t;
+      cfg = c;
+    }
+  }
+  return cfg;
+}
+
+int gemm_run(const GemmPlan& plan, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
+             int64_t ldc, int M, int N, int K, int epilogue, const void* R, int64_t ldr, const float* gate,
              int64_t gate_stride, const int32_t* cu_seqlens, int nseg, hipStream_t stream) {
   if (M == 0) return 0;
   switch (epilogue) {
-    case EPI_BIAS: return launch_k<EPI_BIAS>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
-    case EPI_GELU: return launch_k<EPI_GELU>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
-    case EPI_GATE_RES: return launch_k<EPI_GATE_RES>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
-    case EPI_RES: return launch_k<EPI_RES>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
-    case EPI_F32: return launch_k<EPI_F32>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
-    default: return launch_k<EPI_SILU>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    case EPI_BIAS: return launch_k<EPI_BIAS>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    case EPI_GELU: return launch_k<EPI_GELU>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    case EPI_GATE_RES: return launch_k<EPI_GATE_RES>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    case EPI_RES: return launch_k<EPI_RES>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    case EPI_F32: return launch_k<EPI_F32>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
+    default: return launch_k<EPI_SILU>(plan, A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
   }
 }
 }  // namespace
@@ -1095,8 +1132,8 @@ DITK_EXPORT int ditk_gemm(const void* A, int64_t lda, const void* W, int64_t ldw
   if (int rc = gemm_validate(A, lda, W, ldw, bias, C, ldc, M, N, K, epilogue, R, ldr, gate, gate_stride,
                              cu_seqlens, nseg))
     return rc;
-  return gemm_run(A, lda, W, ldw, bias, C, ldc, M, N, K, epilogue, R, ldr, gate, gate_stride, cu_seqlens, nseg,
-                  stream);
+  return gemm_run(gemm_plan(M, N, K, epilogue, narrow(ldc, ldr), ditk_cu_count()), A, lda, W, ldw, bias, C, ldc, M, N,
+                  K, epilogue, R, ldr, gate, gate_stride, cu_seqlens, nseg, stream);
 }
 
 DITK_EXPORT int ditk_gemm_pair_n(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0,
@@ -1112,41 +1149,46 @@ DITK_EXPORT int ditk_gemm_pair_n(const void* A0, int64_t lda0, const void* W0, i
   if (int rc = gemm_validate(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N1, K, epilogue, R1, ldr1, gate1,
                              gate_stride1, cu_seqlens1, nseg1))
     return rc;
-  // the one-wave-per-SIMD kernel addresses a wave tile's output and residual rows by 32-bit offsets
-  const bool strides = ldc0 < (1 << 22) && ldr0 < (1 << 22) && ldc1 < (1 << 22) && ldr1 < (1 << 22);
-  if (M0 > 0 && M1 > 0 && epilogue != EPI_F32 && K % 64 == 0 && strides) {
-    // one launch over both tile lists where its rounds cost less than two launches
-    int cfg = -1;
-    float us = gemm_plan(M0, N0, K).us + gemm_plan(M1, N1, K).us;
-    for (int c = 0; c < kL4Cfgs; ++c) {
-      auto tiles = [&](int M, int N) {
-        return (int64_t)((M + kL4[c].gbm - 1) / kL4[c].gbm) * ((N + kL4[c].gbn - 1) / kL4[c].gbn);
-      };
-      const float t = l4_cost(c, tiles(M0, N0) + tiles(M1, N1), K);
-      if (t < us) {
-        us = t;
-        cfg = c;
-      }
-    }
-    if (cfg >= 0) {
-      const L4Prob p0{(const bf16_t*)A0, lda0, (const bf16_t*)W0, ldw0, bias0, C0, ldc0, (const bf16_t*)R0, ldr0,
-                      gate0, gate_stride0, cu_seqlens0, nseg0, M0, N0, 0, 0, 0};
-      const L4Prob p1{(const bf16_t*)A1, lda1, (const bf16_t*)W1, ldw1, bias1, C1, ldc1, (const bf16_t*)R1, ldr1,
-                      gate1, gate_stride1, cu_seqlens1, nseg1, M1, N1, 0, 0, 0};
-      switch (epilogue) {
-        case EPI_BIAS: return launch_l4_pair_cfg<EPI_BIAS>(cfg, p0, p1, K, stream);
-        case EPI_GELU: return launch_l4_pair_cfg<EPI_GELU>(cfg, p0, p1, K, stream);
-        case EPI_GATE_RES: return launch_l4_pair_cfg<EPI_GATE_RES>(cfg, p0, p1, K, stream);
-        case EPI_RES: return launch_l4_pair_cfg<EPI_RES>(cfg, p0, p1, K, stream);
-        default: return launch_l4_pair_cfg<EPI_SILU>(cfg, p0, p1, K, stream);
-      }
+  const int cus = ditk_cu_count();
+  const bool narrow0 = narrow(ldc0, ldr0), narrow1 = narrow(ldc1, ldr1);
+  const GemmPlan g0 = gemm_plan(M0, N0, K, epilogue, narrow0, cus), g1 = gemm_plan(M1, N1, K, epilogue, narrow1, cus);
+  const int cfg = pair_plan(g0, g1, M0, N0, M1, N1, K, epilogue, narrow0 && narrow1, cus);
+  if (cfg >= 0) {
+    const L4Prob p0{(const bf16_t*)A0, lda0, (const bf16_t*)W0, ldw0, bias0, C0, ldc0, (const bf16_t*)R0, ldr0,
+                    gate0, gate_stride0, cu_seqlens0, nseg0, M0, N0, 0, 0, 0};
+    const L4Prob p1{(const bf16_t*)A1, lda1, (const bf16_t*)W1, ldw1, bias1, C1, ldc1, (const bf16_t*)R1, ldr1,
+                    gate1, gate_stride1, cu_seqlens1, nseg1, M1, N1, 0, 0, 0};
+    switch (epilogue) {
+      case EPI_BIAS: return launch_l4_pair_cfg<EPI_BIAS>(cfg, p0, p1, K, stream);
+      case EPI_GELU: return launch_l4_pair_cfg<EPI_GELU>(cfg, p0, p1, K, stream);
+      case EPI_GATE_RES: return launch_l4_pair_cfg<EPI_GATE_RES>(cfg, p0, p1, K, stream);
+      case EPI_RES: return launch_l4_pair_cfg<EPI_RES>(cfg, p0, p1, K, stream);
+      default: return launch_l4_pair_cfg<EPI_SILU>(cfg, p0, p1, K, stream);
     }
   }
-  if (int rc = gemm_run(A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N0, K, epilogue, R0, ldr0, gate0, gate_stride0,
+  if (int rc = gemm_run(g0, A0, lda0, W0, ldw0, bias0, C0, ldc0, M0, N0, K, epilogue, R0, ldr0, gate0, gate_stride0,
                         cu_seqlens0, nseg0, stream))
     return rc;
-  return gemm_run(A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N1, K, epilogue, R1, ldr1, gate1, gate_stride1,
+  return gemm_run(g1, A1, lda1, W1, ldw1, bias1, C1, ldc1, M1, N1, K, epilogue, R1, ldr1, gate1, gate_stride1,
                   cu_seqlens1, nseg1, stream);
+}
+
+DITK_EXPORT int ditk_gemm_plan(int M, int N, int K, int epilogue, int* plan) {
+  DITK_REQUIRE(plan && M > 0 && N > 0 && K > 0 && K % 32 == 0 && epilogue >= 0 && epilogue <= 5,
+               "ditk_gemm_plan: bad arguments");
+  const GemmPlan p = gemm_plan(M, N, K, epilogue, true, ditk_cu_count());
+  plan[0] = p.tile;
+  plan[1] = p.rows;
+  plan[2] = p.rest;
+  return 0;
+}
+
+DITK_EXPORT int ditk_gemm_pair_plan(int M0, int N0, int M1, int N1, int K, int epilogue) {
+  if (M0 <= 0 || M1 <= 0 || N0 <= 0 || N1 <= 0 || K <= 0 || K % 32 != 0) return -1;
+  const int cus = ditk_cu_count();
+  const int cfg = pair_plan(gemm_plan(M0, N0, K, epilogue, true, cus), gemm_plan(M1, N1, K, epilogue, true, cus), M0, N0,
+                            M1, N1, K, epilogue, true, cus);
+  return cfg < 0 ? -1 : GT_L4 + cfg;
 }
 
 DITK_EXPORT int ditk_gemm_pair(const void* A0, int64_t lda0, const void* W0, int64_t ldw0, const float* bias0,

@@ -173,6 +173,15 @@ int ditk_gemm_pair_n(const void* A0, int64_t lda0, const void* W0, int64_t ldw0,
                      const float* gate1, int64_t gate_stride1, const int32_t* cu_seqlens1, int nseg1, int N0, int N1,
                      int K, int epilogue, ditk_stream_t stream);
 
+/* How ditk_gemm runs a product (row strides below 2^22; for tests and tuning: no result
+ * depends on it): the first plan[1] rows on tile plan[0], the others on plan[2].  Tiles in
+ * tokens x features: 0: 64 x 128; 1: 256 x 256, eight waves; 2-7: 256 x 256, 256 x 192,
+ * 128 x 256, 128 x 192, 128 x 128, 128 x 96, four waves; 8: few rows without tiles.
+ * ditk_gemm_pair_plan: the tile both products of ditk_gemm_pair_n share in one launch,
+ * -1 for two launches. */
+int ditk_gemm_plan(int M, int N, int K, int epilogue, int* plan);
+int ditk_gemm_pair_plan(int M0, int N0, int M1, int N1, int K, int epilogue);
+
 /* Columns of the transposed-V buffer for Tk keys in nseg segments (upper bound). */
 int64_t ditk_vt_columns(int64_t Tk, int nseg);
 
