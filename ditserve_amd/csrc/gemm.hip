@@ -853,18 +853,18 @@ bool l4_prefetch_on(int M, int N, int K, int64_t ldw, int gbm) {
   if (tiles_m < (K >= 4096 ? 4 : 8)) return false;
   return (int64_t)N * ldw * 2 < (1ll << 31) && (rem == 0 || (3 * rem > gbm && (gbm == 128 || K >= 4096)));
 }
-// Whether the output is stored past the caches (either kernel).  Outputs of 64 MB and more
+// Whether the output (all of it, where two launches write it) is stored past the caches.  Outputs of 64 MB and more
 // are (2.6-3.6% faster on the K = 1536 products of 65520 rows: they would not stay
 // cached until the next kernel reads them); smaller ones stay, and the next kernel
 // finds them (one-frame Wan block 300 -> 281 us, preview step of 2 x 1280 rows
 // 11.20 -> 10.90 ms, SD3.5 512 step 8.65 -> 8.37 ms; gated residual of K = N = 1536 on
-// gemm_kernel and the AdaLN after it: 9300 rows 59.1 -> 57.8 us, 20000 113.2 -> 110.7,
-// but 21800, just below the line, 129 -> 132).
+// gemm_kernel and the AdaLN after it: 9300 rows 59.1 -> 57.8 us, 20000 113.2 -> 110.7;
+// 21800 rows 129 past the caches, 132 in them).
 bool stream_output(int64_t M, int N) { return M * N * 2 >= (64ll << 20); }
 template <int EPI, int FI, int FJ>
 int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C, int64_t ldc,
               int M, int N, int K, const void* R, int64_t ldr, const float* gate, int64_t gate_stride,
-              const int32_t* cu, int nseg, hipStream_t stream, int row_base) {
+              const int32_t* cu, int nseg, hipStream_t stream, int row_base, bool stream_out) {
   constexpr int GBM = L4<FI, FJ>::GBM, GBN = L4<FI, FJ>::GBN;
   const int tiles_m = (M + GBM - 1) / GBM, tiles_n = (N + GBN - 1) / GBN;
   // one persistent workgroup per CU (a multiple of 8: the same number per XCD)
@@ -872,7 +872,7 @@ int launch_l4(const void* A, int64_t lda, const void* W, int64_t ldw, const floa
   gemm_kernel_l4<EPI, FI, FJ><<<(unsigned)nblocks, 256, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, l4_group_m(tiles_m, tiles_n, GBM, GBN, K), l4_prefetch_on(M, N, K, ldw, GBM),
-      stream_output(M, N), row_base);
+      stream_out, row_base);
   return ditk_check_launch("ditk_gemm");
 }
 
@@ -895,14 +895,14 @@ int launch_l4_pair(L4Prob p0, L4Prob p1, int K, hipStream_t stream) {
 template <int EPI, int BK, int T>
 int launch_tile(const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
                 int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
-                int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream, int row_base = 0) {
+                int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream, int row_base, bool stream_out) {
   using S = Stages<BK, T>;
   const int tiles_m = (M + S::GBM - 1) / S::GBM, tiles_n = (N + S::GBN - 1) / S::GBN;
   const int64_t tiles = (int64_t)tiles_m * tiles_n;
   const int64_t nblocks = (tiles + 7) / 8 * 8;
   DITK_REQUIRE(nblocks < (1ll << 31), "ditk_gemm: grid too large");
   constexpr bool kMayStream = T == TILE_LARGE && EPI != EPI_F32;
-  auto kern = kMayStream && stream_output(M, N) ? gemm_kernel<EPI, BK, T, kMayStream> : gemm_kernel<EPI, BK, T, false>;
+  auto kern = kMayStream && stream_out ? gemm_kernel<EPI, BK, T, kMayStream> : gemm_kernel<EPI, BK, T, false>;
   kern<<<(unsigned)nblocks, S::GW * 64, 0, stream>>>(
       (const bf16_t*)A, lda, (const bf16_t*)W, ldw, bias, C, ldc, M, N, K, (const bf16_t*)R, ldr, gate,
       gate_stride, cu, nseg, tiles_m, tiles_n, gemm_group_m(K, tiles_n), row_base);
@@ -913,14 +913,15 @@ int launch_tile(const void* A, int64_t lda, const void* W, int64_t ldw, const fl
 template <int EPI>
 int launch_l4_cfg(int cfg, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
                   int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
-                  int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream, int row_base) {
+                  int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream, int row_base,
+                  bool stream_out) {
   switch (cfg) {
-    case 0: return launch_l4<EPI, 8, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
-    case 1: return launch_l4<EPI, 6, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
-    case 2: return launch_l4<EPI, 8, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
-    case 3: return launch_l4<EPI, 6, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
-    case 4: return launch_l4<EPI, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
-    default: return launch_l4<EPI, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base);
+    case 0: return launch_l4<EPI, 8, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
+    case 1: return launch_l4<EPI, 6, 8>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
+    case 2: return launch_l4<EPI, 8, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
+    case 3: return launch_l4<EPI, 6, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
+    case 4: return launch_l4<EPI, 4, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
+    default: return launch_l4<EPI, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, R, ldr, gate, gate_stride, cu, nseg, stream, row_base, stream_out);
   }
 }
 
@@ -1029,6 +1030,7 @@ template <int EPI, int BK>
 int launch(const GemmPlan& plan, const void* A, int64_t lda, const void* W, int64_t ldw, const float* bias, void* C,
            int64_t ldc, int M, int N, int K, const void* R, int64_t ldr, const float* gate,
            int64_t gate_stride, const int32_t* cu, int nseg, hipStream_t stream) {
+  const bool stream_out = stream_output(M, N);
   // rows [m0, m0 + m) on tile
   auto part = [&](int tile, int m0, int m) {
     constexpr int esize = EPI == EPI_F32 ? 4 : 2;
@@ -1039,13 +1041,13 @@ int launch(const GemmPlan& plan, const void* A, int64_t lda, const void* W, int6
       return launch_skinny<EPI>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu, nseg, stream);
     if (tile == GT_SMALL)
       return launch_tile<EPI, BK, TILE_SMALL>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
-                                              cu, nseg, stream, m0);
+                                              cu, nseg, stream, m0, stream_out);
     if constexpr (EPI != EPI_F32 && BK == 64)
       if (tile >= GT_L4)
         return launch_l4_cfg<EPI>(tile - GT_L4, Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride, cu,
-                                  nseg, stream, m0);
+                                  nseg, stream, m0, stream_out);
     return launch_tile<EPI, BK, TILE_LARGE>(Am, lda, W, ldw, bias, Cm, ldc, m, N, K, Rm, ldr, gate, gate_stride,
-                                            cu, nseg, stream, m0);
+                                            cu, nseg, stream, m0, stream_out);
   };
   const int rc = part(plan.tile, 0, plan.rows);
   return rc != 0 || plan.rows == M ? rc : part(plan.rest, plan.rows, M - plan.rows);
