@@ -29,3 +29,23 @@ def gen(seed):
 
 def randn(shape, seed, scale=1.0):
     return torch.randn(shape, generator=gen(seed)) * scale
+
+
+# Tiles of a product, as numbered by ditk_gemm_plan (2-7: one wave per SIMD)
+SMALL, EIGHT_WAVES, T256, T128X192, T128X96, SKINNY = 0, 1, 2, 5, 7, 8
+
+
+def gemm_plan(m, n, k, epi="bias"):
+    """(tile, rows, rest tile) ditk_gemm takes for an m x n x k product: host only."""
+    import ctypes
+
+    from ditserve_amd import _lib, ops
+    plan = (ctypes.c_int * 3)()
+    _lib.call("ditk_gemm_plan", m, n, k, ops.EPILOGUES[epi], plan)
+    return tuple(plan)
+
+
+def pair_plan(m0, n0, m1, n1, k, epi="bias"):
+    """The tile of a pair's one launch, -1 for two launches."""
+    from ditserve_amd import _lib, ops
+    return _lib.load().ditk_gemm_pair_plan(m0, n0, m1, n1, k, ops.EPILOGUES[epi])

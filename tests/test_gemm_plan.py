@@ -1,27 +1,12 @@
 """The GEMM's tile choice (host rule, no GPU calls): which plans the GPU tests of splits,
 pairs and store policies run on."""
-import ctypes
-
 import pytest
 
 from ditserve_amd import _lib
-from ditserve_amd.ops import EPILOGUES
+from tests.helpers import EIGHT_WAVES, SKINNY, SMALL, T128X96, T128X192, T256, gemm_plan, pair_plan
 
 if not _lib.LIB_PATH.exists():
     pytest.skip("libditk.so not built (run python -m ditserve_amd.build)", allow_module_level=True)
-
-SMALL, EIGHT_WAVES, T256, SKINNY = 0, 1, 2, 8
-T128X192, T128X96 = 5, 7
-
-
-def gemm_plan(m, n, k, epi="bias"):
-    plan = (ctypes.c_int * 3)()
-    assert _lib.load().ditk_gemm_plan(m, n, k, EPILOGUES[epi], plan) == 0
-    return tuple(plan)
-
-
-def pair_plan(m0, n0, m1, n1, k, epi="bias"):
-    return _lib.load().ditk_gemm_pair_plan(m0, n0, m1, n1, k, EPILOGUES[epi])
 
 
 @pytest.mark.parametrize("shape,want", [

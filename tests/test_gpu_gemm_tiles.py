@@ -3,6 +3,8 @@ tiles, split tail rows, paired launches) against the fp32-output kernel."""
 import pytest
 import torch
 
+from tests.helpers import T128X96, T256, gemm_plan, pair_plan
+
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
@@ -66,6 +68,42 @@ def test_tiles_match_the_fp32_output_kernel(m, n, k):
         assert bool((out[m] == 7.0).all())  # nothing past the last row
 
 
+# full rounds of 256 x 256 tiles, then the other rows on 128 x 96 ones (several tile rows
+# at long K)
+SPLITS = [(10914, 1536, 4096, 10752), (12001, 1536, 6144, 10752), (5505, 3072, 14336, 5376)]
+
+
+@pytest.mark.parametrize("m,n,k,rows", SPLITS)
+@pytest.mark.parametrize("epi", ["bias", "gelu", "res", "gate_res"])
+def test_split_products(m, n, k, rows, epi):
+    """A product in two launches, the second on gemm_kernel_l4 with a row base: against
+    the fp32-output kernel, and bit for bit against the same rows as a product of
+    their own.  The gated residual's segments end inside either part."""
+    assert gemm_plan(m, n, k, epi) == (T256, rows, T128X96)
+    x, w, b, res, gate = _operands(m, n, k, m + k)
+    cut = [0, 4000, rows + 60, m]
+    g = torch.randn((3, n), generator=torch.Generator(device="cuda").manual_seed(3), device="cuda")
+
+    def run(lo, hi, out=None):
+        kw = dict(residual=res[lo:hi]) if epi in ("res", "gate_res") else {}
+        if epi == "gate_res":
+            kw.update(gate=g, segments=ops.Segments([min(max(c - lo, 0), hi - lo) for c in cut], "cuda"))
+        return ops.linear(x[lo:hi], w, b, epi, out=out, **kw)
+
+    out = torch.full((m + 1, n), 7.0, device="cuda", dtype=torch.bfloat16)
+    run(0, m, out[:m])
+    assert bool((out[m] == 7.0).all())
+    y = ops.linear(x, w, b, "f32").bfloat16()
+    f = y.float()
+    seg = torch.bucketize(torch.arange(m, device="cuda"), torch.tensor(cut[1:3], device="cuda"), right=True)
+    want = {"bias": lambda: y, "gelu": lambda: torch.nn.functional.gelu(f, approximate="tanh"),
+            "res": lambda: res.float() + f, "gate_res": lambda: res.float() + f * g[seg]}[epi]()
+    _check(out[:m], want, epi)
+    for lo, hi in ((rows, m), (rows - 200, rows + 100), (3900, 4100)):
+        assert gemm_plan(hi - lo, n, k, epi)[0] != T256
+        assert torch.equal(out[lo:hi], run(lo, hi)), (lo, hi)
+
+
 @pytest.mark.parametrize("m", [1, 2, 15, 16])
 @pytest.mark.parametrize("n,k", [(16384, 32), (16392, 96), (16440, 544), (20000, 1536)])
 def test_few_rows_match_the_tiles(m, n, k):
@@ -96,6 +134,7 @@ def test_paired_tiles_match_single_launches(m0, m1, n, k, epi):
         if epi == "gate_res":
             p.update(residual=res, gate=gate, segments=ops.Segments([0, m // 2, m], "cuda"))
         probs.append(p)
+    assert pair_plan(m0, n, m1, n, k, epi) >= 0  # in one launch
     got = ops.linear_pair(*probs, epi)
     for g, p in zip(got, probs):
         assert torch.equal(g, ops.linear(epilogue=epi, **p))
@@ -105,6 +144,7 @@ def test_paired_tiles_match_single_launches(m0, m1, n, k, epi):
                                            (77, 200, 1300, 1544, 64), (1300, 4616, 1, 8, 128)])
 def test_paired_tiles_of_two_widths_match_single_launches(m0, n0, m1, n1, k):
     ps = [dict(zip("xwb", _operands(m, n, k, n + m)[:3])) for m, n in ((m0, n0), (m1, n1))]
+    assert pair_plan(m0, n0, m1, n1, k) >= 0
     for g, p in zip(ops.linear_pair_n(*ps), ps):
         assert torch.equal(g, ops.linear(**p))
     with pytest.raises(ValueError, match="one N and K"):

@@ -8,7 +8,7 @@ import torch
 
 from oracle import common as oc
 from oracle import wan as ow
-from tests.helpers import assert_close, bf, randn
+from tests.helpers import SMALL, assert_close, bf, gemm_plan, pair_plan, randn
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -80,14 +80,13 @@ def test_gemm_rows_independent_of_packing():
 @pytest.mark.parametrize("epi", ["bias", "gelu", "f32", "gate_res", "res", "silu"])
 @pytest.mark.parametrize("K,N", [(1536, 4096), (1536, 1536), (96, 2048), (4160, 2048), (4160, 1024)])
 def test_gemm_tile_configs_agree(epi, K, N):
-    """Large M runs large workgroup tiles, a few hundred rows the 64x128 ones; all
+    """Large M runs large workgroup tiles, a few hundred rows smaller ones; all
     use the same MFMA, k order and epilogue arithmetic, so rows computed in either
-    are bitwise equal.  At M = 8192 on 256 CUs: N = 4096 and (K = 4160, N = 2048)
-    take the one-wave-per-SIMD 256x256 kernel, N = 1536 and (4160, 1024) its
-    256x192 form (fewer tile rounds), K = 96 (an odd number of 32-k stages) and
-    the fp32 epilogue the 8-wave kernel."""
+    are bitwise equal.  K = 96 (an odd number of 32-k stages) and the fp32 epilogue
+    take the 8-wave kernel, the others mostly one wave per SIMD."""
     ops = _ops()
     M = 8192
+    assert gemm_plan(M, N, K, epi)[:1] != gemm_plan(633, N, K, epi)[:1]
     a = randn((M, K), 40).to(DEV, torch.bfloat16)
     w = randn((N, K), 41, 0.02).to(DEV, torch.bfloat16)
     b = randn((N,), 42).to(DEV)
@@ -98,7 +97,7 @@ def test_gemm_tile_configs_agree(epi, K, N):
     elif epi == "res":
         kw = dict(residual=randn((M, N), 43).to(DEV, torch.bfloat16))
     full = ops.linear(a, w, b, epi, **kw)
-    lo, hi = 4700, 5333  # 633 rows across the segment boundary: at most 3 x 16 large tiles, so small ones run
+    lo, hi = 4700, 5333  # 633 rows across the segment boundary
     if epi == "gate_res":
         kw = dict(residual=kw["residual"][lo:hi].contiguous(), gate=kw["gate"], segments=_seg([0, 5000 - lo, hi - lo]))
     elif epi == "res":
@@ -109,10 +108,10 @@ def test_gemm_tile_configs_agree(epi, K, N):
 
 @pytest.mark.parametrize("epi", ["bias", "res", "gate_res", "gelu"])
 def test_gemm_persistent_tiles_agree(epi):
-    """M = 20000, N = K = 1536: 474 large tiles on at most 256 persistent
-    workgroups (some take two), the last tile row ragged (20000 = 78 x 256 + 32).
-    Rows computed there equal, bitwise, the same rows computed alone by the
-    small-tile kernel: a slice ending at the last row and one across tile rows."""
+    """M = 20000, N = K = 1536: 474 large tiles, on at most 256 persistent
+    workgroups but for the gated residual (some take two), the last tile row ragged (20000 = 78 x 256 + 32).
+    Rows computed there equal, bitwise, the same rows computed alone on
+    other tiles: a slice ending at the last row and one across tile rows."""
     ops = _ops()
     M, N, K = 20000, 1536, 1536
     a = randn((M, K), 50).to(DEV, torch.bfloat16)
@@ -142,10 +141,12 @@ def test_gemm_short_tile_row_split_agrees(epi):
     are 4 rounds of 256 CUs but 42 x 18 = 756 are 3, so the 40 rows of the last
     tile row go to the small-tile kernel in a second launch (rows offset into the
     gated residual's segments: a segment ends 22 rows into them).  The same rows
-    inside an 11008-row product (43 whole tile rows, one launch) are equal
+    inside an 11264-row product (44 whole tile rows, one launch) are equal
     bitwise, and the product is close to an fp32 reference."""
     ops = _ops()
-    M, N, K, M2 = 10792, 4608, 1536, 11008
+    M, N, K, M2 = 10792, 4608, 1536, 11264
+    assert gemm_plan(M, N, K, epi)[1:] == (10752, SMALL)
+    assert gemm_plan(M2, N, K, epi)[0] != SMALL and gemm_plan(M2, N, K, epi)[1] == M2
     a = randn((M2, K), 60).to(DEV, torch.bfloat16)
     w = randn((N, K), 61, 0.02).to(DEV, torch.bfloat16)
     b = randn((N,), 62).to(DEV)
@@ -196,6 +197,7 @@ def test_gemm_pair_matches_separate(epi, M0, M1, N, K):
             p["segments"] = _seg([0, M // 2 + 7, M])
         return p
 
+    assert (pair_plan(M0, N, M1, N, K, epi) >= 0) == (N == 1536)
     p0, p1 = prob(M0, 70), prob(M1, 80)
     y0, y1 = ops.linear_pair(p0, p1, epi)
     assert torch.equal(y0, ops.linear(epilogue=epi, **p0)), "first product"
@@ -221,6 +223,7 @@ def test_gemm_pair_in_place_matches_separate(epi):
             p["segments"] = _seg([0, M // 2 + 7, M])
         return p
 
+    assert pair_plan(8192, N, 666, N, K, epi) >= 0
     p0, p1 = prob(8192, 90), prob(666, 95)
     ref0 = p0["residual"].clone()
     ref1 = p1["residual"].clone()
