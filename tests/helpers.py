@@ -49,3 +49,9 @@ def pair_plan(m0, n0, m1, n1, k, epi="bias"):
     """The tile of a pair's one launch, -1 for two launches."""
     from ditserve_amd import _lib, ops
     return _lib.load().ditk_gemm_pair_plan(m0, n0, m1, n1, k, ops.EPILOGUES[epi])
+
+
+def attn_items(tq, tk, nseg, heads, equal=False, joint=False):
+    """Queries per work item (128 or 256) of an attention launch: host only."""
+    from ditserve_amd import _lib
+    return _lib.load().ditk_attn_item_queries(tq, tk, nseg, heads, equal, joint)

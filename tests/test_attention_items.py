@@ -4,6 +4,7 @@ import random
 import pytest
 
 from ditserve_amd import _lib
+from tests.helpers import attn_items
 
 if not _lib.LIB_PATH.exists():
     pytest.skip("libditk.so not built (run python -m ditserve_amd.build)", allow_module_level=True)
@@ -11,8 +12,8 @@ if not _lib.LIB_PATH.exists():
 CUS = 256  # of an MI355X, and what the library assumes without a GPU
 
 
-def items(lens, heads, equal=False, joint=False, keys=None):
-    return _lib.load().ditk_attn_item_queries(sum(lens), sum(keys or lens), len(lens), heads, equal, joint)
+def items(lens, heads, equal=False, joint=False):
+    return attn_items(sum(lens), sum(lens), len(lens), heads, equal, joint)
 
 
 @pytest.mark.parametrize("lens,heads,want", [

@@ -3,6 +3,8 @@ entry point on packed copies (the same kernel, so bit for bit)."""
 import pytest
 import torch
 
+from tests.helpers import attn_items
+
 pytestmark = pytest.mark.gpu
 
 if torch.cuda.is_available():
@@ -44,7 +46,7 @@ def test_strided_operands_match_packed(b, h, sq, sk, d):
 
 def _spiky(t, h, d, seed):
     """q, k with occasional large rows, so that running maxima rise past the lazy
-    rescale threshold in some 32-query blocks and not in others."""
+    rescale threshold for some queries of a wave and not for others."""
     g = torch.Generator(device="cuda").manual_seed(seed)
     q, k, v = (torch.randn((t, h * d), generator=g, device="cuda") for _ in range(3))
     q[::37] *= 6.0
@@ -60,6 +62,7 @@ def test_work_item_size_does_not_change_results(d, pre, lens):
     with enough others to fill the GPU run as 256-query ones: bit for bit the same,
     rescales and lse included, and each close to softmax attention in fp64."""
     h, total = 3, sum(lens)
+    assert attn_items(total, total, len(lens), h) == 128
     q, k, v = _spiky(total, h, d, total + d)
     cu = [0]
     for n in lens:
@@ -69,6 +72,7 @@ def test_work_item_size_does_not_change_results(d, pre, lens):
     reps = 256 * 256 // max(total, 1) + 2
     cu_many = [0] + [r * total + c for r in range(reps) for c in cu[1:]]
     seg_many = ops.Segments(cu_many, "cuda")
+    assert attn_items(reps * total, reps * total, reps * len(lens), h) == 256
     many, many_lse = ops.flash_attn_varlen(q.repeat(reps, 1), k.repeat(reps, 1), v.repeat(reps, 1), seg_many, seg_many,
                                            h, d, return_lse=True, q_prescaled=pre)
     for r in (0, reps // 2, reps - 1):
@@ -86,3 +90,41 @@ def test_work_item_size_does_not_change_results(d, pre, lens):
         assert float(err) < 8e-3, float(err)
         assert torch.allclose(few_lse[:, a:b].double(), s.logsumexp(-1), atol=2e-3, rtol=1e-5)
 
+
+
+@pytest.mark.parametrize("img,txt", [([260, 64], [77, 33]), ([1], [63]), ([64, 129, 300], [64, 1, 20]), ([1024], [333])])
+def test_joint_work_item_size_does_not_change_results(img, txt):
+    """Joint attention likewise: segments whose last key tile is partial, whose image
+    and text rows meet inside a tile or at its edge, on the one- and the two-block body,
+    each close to softmax attention in fp64."""
+    h, w = 4, 4 * 64
+    def cu(lens, reps=1):
+        out = [0]
+        for n in lens * reps:
+            out.append(out[-1] + n)
+        return out
+    both = [a + b for a, b in zip(img, txt)]
+    total = sum(both)
+    q, k, v = (dict(zip(("img", "txt"), x.split([sum(img), sum(txt)]))) for x in _spiky(total, w // 64, 64, total))
+    q = {n: (x.float() * (64 ** -0.5 * ops.LOG2E)).bfloat16() for n, x in q.items()}
+
+    def run(reps):
+        segs = [ops.Segments(cu(n, reps), "cuda") for n in (img, txt, both)]
+        (qi, qt), (ki, kt), (vi, vt_) = ([x[n].repeat(reps, 1) for n in ("img", "txt")] for x in (q, k, v))
+        vt = ops.transpose_v_joint(vi, vt_, h, 64, *segs)
+        return ops.joint_attention_q_prescaled(qi, qt, ki, kt, vt, *segs, h, 64)
+    reps = 256 * 128 // total + 2
+    assert attn_items(total, total, len(img), h, joint=True) == 128
+    assert attn_items(reps * total, reps * total, reps * len(img), h, joint=True) == 256
+    few, many = run(1), run(reps)
+    for one, all_ in zip(few, many):
+        for r in (0, reps // 2, reps - 1):
+            assert torch.equal(all_[r * one.shape[0]:(r + 1) * one.shape[0]], one)
+    for m in range(len(img)):
+        rows = [slice(cu(n)[m], cu(n)[m + 1]) for n in (img, txt)]
+        qs, ks, vs = (torch.cat([x[n][r] for n, r in zip(("img", "txt"), rows)]).double().view(-1, h, 64).transpose(0, 1)
+                      for x in (q, k, v))
+        want = ((qs @ ks.transpose(1, 2) / ops.LOG2E).softmax(-1) @ vs).transpose(0, 1).reshape(-1, w)
+        got = torch.cat([x[r] for x, r in zip(few, rows)]).double()
+        # P and O round to bf16 (2^-9 each, averaged over keys)
+        assert float((got - want).norm() / want.norm()) < 8e-3
