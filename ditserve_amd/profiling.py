@@ -7,20 +7,42 @@ encloses, so the measured duration is GPU time of exactly those kernels.
 Disabled profilers cost nothing; nothing here synchronises until summary().
 """
 import collections
-import contextlib
+import functools
 
 import torch
 
 
-class _NoRegion:
+class _Region:
+    """A region that is not timed: a context manager, or a decorator, whose function is
+    timed or not as the profiler stands at each call."""
+
+    def __init__(self, profiler, name):
+        self._profiler, self._name = profiler, name
+
     def __enter__(self):
         return None
 
     def __exit__(self, *exc):
         return False
 
+    def __call__(self, fn):
+        @functools.wraps(fn)
+        def inside(*args, **kwargs):
+            with self._profiler.region(self._name):
+                return fn(*args, **kwargs)
+        return inside
 
-_NO_REGION = _NoRegion()  # stateless: shared by every untimed region
+
+class _TimedRegion(_Region):
+    def __enter__(self):
+        self._start = torch.cuda.Event(enable_timing=True)
+        self._end = torch.cuda.Event(enable_timing=True)
+        self._start.record()
+
+    def __exit__(self, *exc):
+        self._end.record()
+        self._profiler._events[self._name].append((self._start, self._end))
+        return False
 
 
 class EventProfiler:
@@ -31,23 +53,18 @@ class EventProfiler:
         self.enabled = enabled
         self.only = None if only is None else frozenset(only)
         self._events = collections.defaultdict(list)
+        self._idle = {}
 
     def region(self, name):
-        """Context manager timing the launches inside it as `name`."""
-        if not self.enabled or (self.only is not None and name not in self.only):
-            return _NO_REGION
-        return self._timed(name)
-
-    @contextlib.contextmanager
-    def _timed(self, name):
-        start = torch.cuda.Event(enable_timing=True)
-        end = torch.cuda.Event(enable_timing=True)
-        start.record()
-        try:
-            yield
-        finally:
-            end.record()
-            self._events[name].append((start, end))
+        """Context manager (or decorator) timing the launches inside it as `name`."""
+        if self.enabled and (self.only is None or name in self.only):
+            return _TimedRegion(self, name)
+        idle = self._idle.get(name)  # stateless: one per name, for the first few hundred names
+        if idle is None:
+            idle = _Region(self, name)
+            if len(self._idle) < 256:
+                self._idle[name] = idle
+        return idle
 
     def reset(self):
         self._events.clear()

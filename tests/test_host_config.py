@@ -152,3 +152,44 @@ def test_attention_plugin_dataclasses_match_reference():
     assert attention.VarlenPacking.from_kwargs({"cu_seqlens_k": 1}) is None
     p = attention.VarlenPacking.from_kwargs({"indices_k": "i", "cu_seqlens_k": "c", "max_seqlen_k": 7})
     assert (p.indices_k, p.cu_seqlens_k, p.max_seqlen_k) == ("i", "c", 7)
+
+
+def test_profiler_regions_decorate(monkeypatch):
+    """A region is a context manager or a decorator; the decorated function is timed
+    as the profiler's switches stand at each call."""
+    import torch
+    from ditserve_amd.profiling import EventProfiler
+
+    class Event:
+        def __init__(self, enable_timing):
+            assert enable_timing
+
+        def record(self):
+            pass
+
+        def elapsed_time(self, end):
+            return 2.0
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    prof = EventProfiler(enabled=False, only=("a", "f"))
+    with prof.region("a"):
+        pass
+    assert prof.summary() == {}
+
+    @prof.region("f")
+    def f(n):
+        return 1 + f(n - 1) if n else 0
+    assert f(2) == 2 and prof.summary() == {}
+    prof.enabled = True
+    with prof.region("a"):
+        assert f(2) == 2
+    with prof.region("b"):
+        pass
+    try:
+        with prof.region("a"):
+            raise KeyError
+    except KeyError:
+        pass
+    prof.enabled = False
+    assert f(1) == 1
+    assert {n: r["count"] for n, r in prof.summary().items()} == {"a": 2, "f": 3}
