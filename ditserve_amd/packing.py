@@ -52,17 +52,22 @@ def token_packing_stats(counts):
     }
 
 
-def joint_layout(img_counts, txt_counts):
-    """Joint image+text layout of a packed MMDiT batch.
-
-    Returns cu_img, cu_txt, cu_joint (cu_joint[m] = cu_img[m] + cu_txt[m]),
-    max_seqlen_img, max_seqlen_joint and the joint row of every image / text
-    token (img_in_joint, txt_in_joint)."""
+def joint_tables(img_counts, txt_counts):
+    """(cu_img, cu_txt, cu_joint) of a packed MMDiT batch: cu_joint[m] = cu_img[m] + cu_txt[m]."""
     if len(img_counts) != len(txt_counts) or not img_counts:
         raise ValueError("image and text counts must be non-empty lists of equal length")
     cu_img = build_cu_seqlens(img_counts)
     cu_txt = [0, *itertools.accumulate(int(n) for n in txt_counts)]
-    cu_joint = [a + b for a, b in zip(cu_img, cu_txt)]
+    return cu_img, cu_txt, [a + b for a, b in zip(cu_img, cu_txt)]
+
+
+def joint_layout(img_counts, txt_counts):
+    """Joint image+text layout of a packed MMDiT batch.
+
+    Returns cu_img, cu_txt and cu_joint (joint_tables), max_seqlen_img,
+    max_seqlen_joint and the joint row of every image / text token (img_in_joint,
+    txt_in_joint)."""
+    cu_img, cu_txt, cu_joint = joint_tables(img_counts, txt_counts)
     img_in_joint, txt_in_joint = [], []
     for m, (ni, nt) in enumerate(zip(img_counts, txt_counts)):
         img_in_joint.extend(range(cu_joint[m], cu_joint[m] + ni))

@@ -19,14 +19,13 @@ Block (sd35_batch.py:647-708), per JointTransformerBlock:
   blocks); gated residuals; GELU-tanh FFNs on image and text.
 """
 import dataclasses
-import itertools
 import math
 
 import torch
 
 from . import ops
 from .ops import Segments
-from .packing import build_cu_seqlens
+from .packing import joint_tables
 from .profiling import NULL as _NULL_PROFILER
 
 _BF16 = torch.bfloat16
@@ -368,9 +367,7 @@ class SD35Transformer:
                 raise ValueError(f"text contexts must be [L, {cfg.text_dim}], got {tuple(t.shape)}")
         txts = [t.reshape(-1, cfg.text_dim) for t in texts]
         txt_counts = [t.shape[0] for t in txts]
-        cu_img, cu_txt = build_cu_seqlens(img_counts), [0, *itertools.accumulate(txt_counts)]
-        cu_joint = [a + b for a, b in zip(cu_img, cu_txt)]
-        cus = (cu_img, cu_txt, cu_joint)
+        cus = cu_img, cu_txt, cu_joint = joint_tables(img_counts, txt_counts)
         *cu_dev, t = ops.to_device_tables([*cus, [float(x) for x in timesteps]], dev)
         seg_img, seg_txt, seg_joint = (Segments(c, dev, d) for c, d in zip(cus, cu_dev))
         # prelude: patch embed (+ cropped 2D sin-cos positions), context embedder, temb

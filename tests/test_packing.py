@@ -51,6 +51,7 @@ def test_joint_index_maps_agree():
         assert o["img_in_joint_idx"] == p["img_in_joint"]
         assert o["txt_in_joint_idx"] == p["txt_in_joint"]
         assert o["cu_joint"] == p["cu_joint"]
+        assert packing.joint_tables(img, txt) == (p["cu_img"], p["cu_txt"], p["cu_joint"])
         # the two maps partition the joint rows
         assert sorted(p["img_in_joint"] + p["txt_in_joint"]) == list(range(p["total_joint"]))
 
