@@ -23,10 +23,6 @@ def _stream():
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def ctypes_stream(stream):
-    return _lib.c_void_p(stream.cuda_stream)
-
-
 def _ptr(t):
     return t.data_ptr() if t is not None else None
 

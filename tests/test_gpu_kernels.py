@@ -206,6 +206,26 @@ def test_gemm_pair_matches_separate(epi, M0, M1, N, K):
         ops.linear_pair(p0, dict(x=p1["x"][:, :K - 32].contiguous(), w=p1["w"][:, :K - 32].contiguous()), epi)
 
 
+def test_gemm_pair_entry_point_of_one_width():
+    """ditk_gemm_pair (products of one N) through the C ABI: ops.linear_pair takes the
+    form with two widths, which gives the same."""
+    from ditserve_amd import _lib
+    ops = _ops()
+    M, N, K = (600, 130), 1536, 256
+    ps = [dict(x=randn((m, K), 70 + m).to(DEV, torch.bfloat16), w=randn((N, K), 71 + m, 0.02).to(DEV, torch.bfloat16),
+               b=randn((N,), 72 + m).to(DEV), residual=randn((m, N), 73 + m).to(DEV, torch.bfloat16),
+               gate=randn((2, N), 74 + m).to(DEV), segments=_seg([0, m // 2, m])) for m in M]
+    outs = [torch.empty((m, N), dtype=torch.bfloat16, device=DEV) for m in M]
+    args = []
+    for p, y in zip(ps, outs):
+        s = p["segments"]
+        args += [p["x"].data_ptr(), K, p["w"].data_ptr(), K, p["b"].data_ptr(), y.data_ptr(), N, y.shape[0],
+                 p["residual"].data_ptr(), N, p["gate"].data_ptr(), N, s.dev.data_ptr(), s.nseg]
+    _lib.call("ditk_gemm_pair", *args, N, K, ops.EPILOGUES["gate_res"], torch.cuda.current_stream().cuda_stream)
+    for got, want in zip(outs, ops.linear_pair(*ps, "gate_res")):
+        assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("epi", ["gate_res", "res"])
 def test_gemm_pair_in_place_matches_separate(epi):
     """SD3.5's block calls the pair in place (out = residual = h for the image rows,
