@@ -30,7 +30,9 @@ attention roofline fraction and CPU baseline:
   * wan21_480p_33f_cfg2   Wan2.1-T2V-1.3B 480x832x33f step (the reference's dev
                           shape), CFG pair of 2 x 14040 tokens.
 
-Prints one JSON line.  ``roofline`` is for the dominant kernel, the self-attention
+Prints one JSON line of a few kilobytes; ``--details FILE`` writes the whole results,
+which the line gives without the kernel tables and with a few numbers per config.
+``roofline`` is for the dominant kernel, the self-attention
 flash kernel, from HIP events recorded on its launch stream over the timed steps.
 ``kernels`` (per config) gives every hot kernel's roofline -- GEMMs and attention
 as TFLOP/s of the 2.5 PFLOP/s bf16 peak, the row kernels as TB/s of 8 TB/s HBM --
@@ -94,6 +96,7 @@ def parse_args():
     ap.add_argument("--breakdown", action="store_true", help="per-op HIP-event breakdown in the JSON")
     ap.add_argument("--surfaces", action="store_true",
                     help="only time the reference-shaped entry points against the engine path (one JSON line)")
+    ap.add_argument("--details", metavar="FILE", help="also write the whole results (kernel tables, every config) as JSON")
     ap.add_argument("--workload", default="wan21_480p", choices=sorted(WORKLOADS),
                     help="the workload of the top-level line (default: the Wan2.1 480p headline)")
     return ap.parse_args()
@@ -741,6 +744,16 @@ def _public(d):
     return {k: v for k, v in d.items() if not k.startswith("_")}
 
 
+def _line(out):
+    """The results as one short line: no kernel tables, and of each config its rate, its
+    time, and how these stand to the reference's and to the CPU's."""
+    short = {k: v for k, v in out.items() if k not in ("kernels", "per_config")}
+    keep = ("value", "unit", "ms_per_step", "vs_reference_a100", "gpu_vs_cpu")
+    if "per_config" in out:
+        short["per_config"] = {n: {k: r[k] for k in keep if k in r} for n, r in out["per_config"].items()}
+    return json.dumps(short)
+
+
 def main():
     args = parse_args()
     world = int(os.environ.get("WORLD_SIZE", "1"))
@@ -829,7 +842,10 @@ def main():
             blk["gpu_vs_cpu"] = blk["cpu_baseline"]["value"] / blk["value"]
         per["wan21_block_1560tok"] = blk
         out["per_config"] = per
-    print(json.dumps(out), flush=True)
+    if args.details:
+        with open(args.details, "w") as f:
+            json.dump(out, f, indent=1)
+    print(_line(out), flush=True)
 
 
 if __name__ == "__main__":

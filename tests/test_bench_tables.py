@@ -1,5 +1,6 @@
 """bench.py's per-kernel roofline tables (host arithmetic only): the algorithmic work
 per launch each kernel is credited with, and the fractions derived from it."""
+import json
 import math
 
 import bench
@@ -41,3 +42,19 @@ def test_kernel_table_fractions():
     assert t["k_mfma"]["unit"] == "TFLOP/s" and t["k_mfma"]["flops_per_launch"] == 2.5e12
     assert math.isclose(t["k_hbm"]["achieved"], 4.0) and math.isclose(t["k_hbm"]["frac"], 0.5)
     assert t["k_hbm"]["unit"] == "TB/s" and t["k_hbm"]["launches"] == 5 and t["k_hbm"]["bytes_per_launch"] == 8e9
+
+
+def test_printed_line_is_short_and_keeps_the_headline():
+    """The printed line leaves out the kernel tables, whatever they hold."""
+    table = {f"kernel_{i}": {"what": "x" * 80, "achieved": 1234.5678901234, "frac": 0.5} for i in range(12)}
+    head = {"metric": "m", "value": 2.36, "unit": "steps/s", "n_gpus": 1, "steps": 20, "warmup": 5, "ms_per_step": 423.0,
+            "higher_is_better": True, "scaling": "weak", "vs_baseline": 9.4, "dtype": "bf16", "data": "synthetic",
+            "config": {"workload": "w" * 200}, "roofline": {"kernel": "k" * 80, "frac": 0.58}}
+    per = {f"config_{i}": {"metric": "m" * 80, "value": 1.5, "unit": "steps/s", "ms_per_step": 2.5, "vs_reference_a100": 9.0,
+                           "workload": "w" * 200, "kernels": table, "cpu_baseline": {"sample": "s" * 300}}
+           for i in range(8)}
+    line = bench._line({**head, "kernels": table, "per_config": per})
+    got = json.loads(line)
+    assert len(line) < 4096 and "\n" not in line
+    assert {k: got[k] for k in head} == head and "kernels" not in got
+    assert got["per_config"]["config_3"] == {"value": 1.5, "unit": "steps/s", "ms_per_step": 2.5, "vs_reference_a100": 9.0}
