@@ -481,11 +481,14 @@ int launch_skinny(const void* A, int64_t lda, const void* W, int64_t ldw, const 
 // (16x16x32, W rows as the A operand), same k order, same bias add and rounding:
 // bitwise equal to gemm_kernel.
 // A wave tile is FI feature and FJ token fragments of 16; the six tiles generated
-// are listed with their times at kL4 below.  What bounds them: a 256 x 256 tile's
-// stage is 2048 MFMA cycles for 64 KiB of operand DMA (MFMA-bound); at 128 x 128 it
-// is 512 cycles for 32 KiB, and the CU's ~60 B/clk from L2 takes about as long
+// are listed with their times at kL4 below.  What bounds them, by counters at K =
+// 8192-8960: a 256 x 256 tile's stage takes 2464 cycles, 2048 of them MFMA (83%); a
+// 128 x 128 one 845 for 512 (60%), a 128 x 96 one 707 for 384 (54%).  Waves wait for 9,
+// 12 and 15% of their time, and the LDS reads of a 128 x 128 stage take 262 cycles
+// without bank conflicts, so what a smaller tile adds is mostly issue: the one wave of a
+// SIMD issues as many reads, DMAs and address instructions for fewer MFMAs.
 // (1560 x 1536 x 8960 on 64 x 128 tiles of gemm_kernel 81 us, 128 x 96 here 54 us;
-// 2048 x 6144 x 1536 on 256 x 192 as before).
+// 2048 x 6144 x 1536 on 256 x 192 as before.)
 template <int FI, int FJ>
 struct L4 {
   static constexpr int WTM = 16 * FJ, WTN = 16 * FI, GBM = 2 * WTM, GBN = 2 * WTN;
@@ -714,8 +717,8 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
   // ends at the last row of the matrix: a store past it is dropped and a load
   // returns 0, so the passes have no branches and the staged-row reads and
   // residual loads of many passes are in flight together.
-  constexpr int CPR = WTN / 8;                    // 16-byte units per row (16 or 12)
-  constexpr int RPP = 64 / CPR;                   // rows per pass (4 or 5; lanes past RPP * CPR idle)
+  constexpr int CPR = WTN / 8;                    // 16-byte units per row (16, 12, 8 or 6)
+  constexpr int RPP = 64 / CPR;                   // rows per pass (4, 5, 8 or 10; lanes past RPP * CPR idle)
   constexpr int NPASS = (WTM + RPP - 1) / RPP;
   constexpr bool HAS_RES = EPI == EPI_GATE_RES || EPI == EPI_RES;
   constexpr uint32_t kOut = 0x80000000u;          // an offset past every descriptor's range
@@ -813,9 +816,10 @@ __device__ __forceinline__ void l4_tile(u32x4_t* lds, int L, const bf16_t* __res
 // The tile configurations of gemm_kernel_l4: workgroup tile (tokens x features)
 // and its measured time in us, start + rounds x (tile + stage x K / 64) with a round
 // one tile per CU (least squares over 14 weight shapes of the Wan and SD3.5 blocks,
-// 8 to 28000 rows, weights from HBM; 8-9% rms).  A 256 x 256 tile's stage does 2.3
-// PFLOP/s over the chip, a 128 x 96 one's 1.4: the small tiles move more operand
-// bytes per MFMA, but let 1000-row products use most of the CUs.
+// 8 to 28000 rows, weights from HBM; 8-9% rms.  Longer products lose clock and take
+// more, 56400 x 1536 x 8960 1199 us for 949 predicted; there it only ranks the
+// tiles).  A 256 x 256 tile's stage does 1.78 PFLOP/s over the chip, a 128 x 96 one's
+// 1.06, but the small tiles let 1000-row products use most of the CUs.
 struct L4Cfg {
   int gbm, gbn;
   float start, tile, stage;

@@ -21,6 +21,7 @@ def _views(b, h, s, d, g):
     yield "column slice", r(b, s, h, 3 * d).transpose(1, 2)[..., d:2 * d]
     yield "row slice", r(b, h, s + 5, d)[:, :, 3:s + 3]
     yield "shared batch", r(1, h, s, d).expand(b, h, s, d)
+    yield "shared row", r(b, h, 1, d).expand(b, h, s, d)     # row stride 0
     yield "odd strides", r(b, h, s, d + 1)[..., :d]          # rows not 16-byte aligned: copied
     yield "dim stride", r(b, h, d, s).transpose(2, 3)        # D not contiguous: copied
 
